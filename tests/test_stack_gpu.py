@@ -57,6 +57,51 @@ def test_split_attention_against_oracle(vx, oracle, cuda, stream, heads, kv_head
     assert diff.max() <= 1, f"max {diff.max()} ulp"
 
 
+@pytest.mark.parametrize("heads,kv_heads,head_dim", [(16, 2, 128), (3, 3, 64), (16, 1, 64)])
+@pytest.mark.parametrize("rows,rps,past,causal,keys", [
+    (32, 32, 0, True, None),      # the least rows of one head; a prompt's first rows
+    (33, 33, 31, True, None),     # a query past a wave's 32; the 33rd key
+    (45, 45, 0, False, 60),       # bidirectional, the cache longer than the keys
+    (110, 55, 0, False, 55),      # two sequences that end inside a step and a wave
+    (129, 129, 0, True, None),    # a query past a workgroup's 128 of one head
+    (150, 150, 512, True, None),  # several chunks, rows that end in different ones
+    (160, 40, 300, True, 345),    # several causal sequences behind a past
+])
+def test_tile_attention_against_oracle(vx, oracle, cuda, stream, heads, kv_heads, head_dim,
+                                       rows, rps, past, causal, keys):
+    """The matrix-core attention of many rows against the oracle, what lies
+    in the cache past the attended keys (NaN here) unread. The bound: one
+    bf16 ulp (2^-7 of the value), and what float32 sums in another order
+    leave of an output near zero: scores up to about 8 round to 2^-21, each
+    weight by as much of itself and so the weighted sum by 2^-20 of the
+    largest value."""
+    rng = synth.Rng(37, rows * 1000 + past + head_dim)
+    sequences = rows // rps
+    keys = keys or past + rps
+    capacity = sequences * keys + 3
+    q = f32(1.5 * rng.normal(rows * heads * head_dim).reshape(rows, heads, head_dim))
+    kc = f32(rng.normal(kv_heads * capacity * head_dim).reshape(kv_heads, capacity, head_dim))
+    vc = f32(rng.normal(kv_heads * capacity * head_dim).reshape(kv_heads, capacity, head_dim))
+    for sequence in range(sequences):
+        unread = slice(sequence * keys + past + rps, (sequence + 1) * keys)
+        kc[:, unread] = np.nan
+        vc[:, unread] = np.nan
+    kc[:, sequences * keys:] = np.nan
+    vc[:, sequences * keys:] = np.nan
+    ref = np.zeros((rows, heads, head_dim), np.uint16)
+    oracle.lib().vo_attention(oracle.ptr(q), oracle.ptr(kc), oracle.ptr(vc), oracle.ptr(ref),
+                              rows, rps, keys, past, int(causal), heads, kv_heads, head_dim,
+                              capacity)
+    got = vx.split_attention(dev(q, cuda), dev(kc, cuda), dev(vc, cuda), rps, keys, past,
+                             causal, heads, kv_heads)
+    torch.cuda.synchronize()
+    got, ref = synth.bf16_values(host_bf16(got)), synth.bf16_values(ref)
+    bound = 2.0**-7 * np.abs(ref) + 2.0**-20 * np.nanmax(np.abs(vc))
+    worst = float(np.max(np.abs(got - ref) / bound))
+    print(f"worst {worst:.2f} of the bound", flush=True)
+    assert worst <= 1
+
+
 def make_stack(vx, oracle, config, seed, bf16_weights=False, positions=2048):
     """`positions`: rows of the rotary table; every position a step uses
     must index it (the kernels read row `position` of the table)."""

@@ -25,6 +25,7 @@
 #include "products.hpp"
 #include "q8.hpp"
 #include "q8_tile.hpp"
+#include "tile_attention.hpp"
 #include "voxcpm_amd.h"
 #include "voxcpm_amd_internal.h"
 
@@ -464,6 +465,13 @@ void Attention(const float* q, const float* k_cache, const float* v_cache, Bf16*
                std::size_t rows_per_sequence, std::size_t keys_per_sequence, std::size_t past,
                bool causal, std::size_t heads, std::size_t kv_heads, std::size_t head_dim,
                std::size_t capacity, int splits, const int* past_device, hipStream_t stream) {
+  const AttentionShape shape{rows, rows_per_sequence, keys_per_sequence, past, causal,
+                             heads, kv_heads, head_dim, capacity};
+  if (!fragment && past_device == nullptr &&
+      UseTileAttention(shape, q, k_cache, v_cache, out, partials)) {
+    TileAttention(shape, q, k_cache, v_cache, out, partials, stream);
+    return;
+  }
   AttentionArgs a{};
   a.q = q;
   a.k = k_cache;

@@ -1,0 +1,448 @@
+// Attention of many rows over a float32 key/value cache (a prompt's prefill,
+// a prompt's patches through the local encoder): the reference's Attention
+// (kernels/generator_kernels.hip:160-241) on gfx950's bf16 matrix cores with
+// float32 operands split into three bf16 terms (bf16x3.hpp).
+//
+// A workgroup of four waves takes 128 queries of one KV head -- a query is a
+// (row, query head of the group) pair, so a group's heads share every key
+// and value the workgroup brings in -- and a run of keys, 32 at a time:
+// the threads load the next 32 keys and values into registers, split the
+// current ones into LDS (keys row-major, values transposed), and each wave
+// multiplies them with its 32 queries, which stay split in registers.
+// Scores are made transposed, S^T = K Q^T, so that a lane holds one query's
+// scores (column L % 32) and the exponentials are the next product's B
+// operand where they are: O^T = V^T P^T over the keys in the order S^T left
+// them, which the transposed values in LDS follow. The softmax runs online
+// per query (running maximum and sum, float32).
+//
+// Short of workgroups, the keys are cut into chunks that separate workgroups
+// take; each leaves its maximum, sum and unnormalised values, and a second
+// launch merges a row's chunks in chunk order.
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <cmath>
+#include <cstdint>
+
+#include "bf16x3.hpp"
+#include "common.hpp"
+#include "q8.hpp"
+#include "q8_tile.hpp"
+#include "tile_attention.hpp"
+
+namespace vx {
+namespace {
+
+using bf16x3::F32x16;
+using bf16x3::Octet;
+
+constexpr int kThreads = 256;
+constexpr int kWaves = kThreads / kWave;
+constexpr int kQueries = 32 * kWaves;  // per workgroup
+constexpr int kKeys = 32;              // per step
+// Fewest keys of a chunk (the caller's partials hold a chunk per 64 keys).
+constexpr int kLeastChunk = 128;
+// Workgroups that chunks are cut for: two per compute unit.
+constexpr int kTargetWorkgroups = 512;
+// A transposed value row in LDS: 32 bf16 keys and 16 bytes of padding, so
+// that the 16-byte reads of eight consecutive rows fall on distinct banks.
+constexpr int kValueRow = 80;
+
+struct TileArgs {
+  const float* q;
+  const float* k;
+  const float* v;
+  Bf16* out;
+  float* values;  // [rows][heads][splits][D], several chunks
+  float* stats;   // [rows][heads][splits][2]: maximum, sum
+  int rows_per_sequence;
+  int keys_per_sequence;
+  int past;
+  int causal;
+  int heads;
+  int kv_heads;
+  int capacity;
+  int blocks;  // query blocks per (sequence, KV head)
+  int chunk;   // keys per chunk
+  int splits;  // chunks
+  float scale;
+};
+
+/// exp(x) for x <= 0 to about one ulp: 2^(x log2 e) with the rounding of
+/// the product carried into the result.
+__device__ inline float ExpNegative(float x) {
+  constexpr float kLog2E = 1.44269504088896341F;
+  constexpr float kLog2ELow = 1.92596299e-8F;  // log2 e - kLog2E
+  constexpr float kLn2 = 0.693147180559945309F;
+  const float a = x * kLog2E;
+  const float low = __builtin_fmaf(x, kLog2E, -a) + x * kLog2ELow;
+  const float e = __builtin_amdgcn_exp2f(a);
+  return __builtin_fmaf(e, low * kLn2, e);
+}
+
+/// max over the wave's halves (both lanes of a pair receive it).
+__device__ inline float MaxXor32(float x) {
+  const auto swapped =
+      __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return fmaxf(__uint_as_float(swapped[0]), __uint_as_float(swapped[1]));
+}
+
+template<int D>
+__global__ __launch_bounds__(kThreads, 2) void TileAttentionKernel(TileArgs a) {
+  constexpr int kChunks = D / 8;    // 16-byte chunks of a key row's plane
+  constexpr int kSteps = D / 16;    // MFMA steps of a score
+  constexpr int kTiles = D / 32;    // 32-dimension tiles of the output
+  constexpr int kKeyLoads = kKeys * kChunks / kThreads;  // 8-value pieces per thread
+  constexpr int kValueThreads = kKeys / 4 * (D / 4);     // 4 x 4 pieces
+  __shared__ uint4 key_planes[3][kKeys * kChunks];
+  __shared__ __align__(16) unsigned char value_planes[3][D * kValueRow];
+
+  const int tid = static_cast<int>(threadIdx.x);
+  const int lane = tid % kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int column = lane % 32;
+  const int half = lane / 32;
+  int block = static_cast<int>(blockIdx.x);
+  const int split = block % a.splits;
+  block /= a.splits;
+  // The last query blocks, with the most keys of a causal call, first.
+  const int query_block = a.blocks - 1 - block % a.blocks;
+  block /= a.blocks;
+  const int g = block % a.kv_heads;
+  const int sequence = block / a.kv_heads;
+  const int group = a.heads / a.kv_heads;
+  const int queries = a.rows_per_sequence * group;
+
+  // Keys of query `index` (queries past the last count none).
+  const auto keys_of = [&](int index) {
+    return index >= queries ? 0
+                            : a.past + (a.causal != 0 ? index / group + 1 : a.rows_per_sequence);
+  };
+  const int first_query = query_block * kQueries;
+  const int block_keys = keys_of(min(first_query + kQueries, queries) - 1);
+  const int key_begin = split * a.chunk;
+  const int key_end = min(key_begin + a.chunk, block_keys);
+  if (key_begin >= key_end)
+    return;
+  const int wave_query = first_query + 32 * wave;
+  const int wave_keys =
+      wave_query < queries ? keys_of(min(wave_query + 32, queries) - 1) : 0;
+  const int query = wave_query + column;
+  const int my_keys = keys_of(query);
+  // Steps whose keys every query of the wave counts need no mask.
+  const int whole_keys = wave_query + 32 <= queries ? keys_of(wave_query) : 0;
+  const int local = min(query, queries - 1);
+  const int row = sequence * a.rows_per_sequence + local / group;
+  const int head = g * group + local % group;
+
+  // The caches up to the run's end as buffers: loads past it read zero (the
+  // cache beyond what was written may hold anything).
+  const std::size_t cache = (static_cast<std::size_t>(g) * a.capacity +
+                             static_cast<std::size_t>(sequence) * a.keys_per_sequence) *
+                            D;
+  const std::uint32_t cache_bytes = 4U * D * static_cast<std::uint32_t>(key_end);
+  const __amdgpu_buffer_rsrc_t keys = q8::BufferOf(a.k + cache, cache_bytes);
+  const __amdgpu_buffer_rsrc_t values = q8::BufferOf(a.v + cache, cache_bytes);
+  const auto load16 = [](__amdgpu_buffer_rsrc_t buffer, std::uint32_t offset) {
+    return __builtin_bit_cast(float4, q8::BufferLoad16(buffer, offset, true));
+  };
+
+  // The next step's keys (pieces of eight values) and values (four keys by
+  // four dimensions) in flight.
+  float4 key_next[kKeyLoads][2];
+  float4 value_next[4];
+  const int value_quad = tid % (kKeys / 4);  // keys 4 value_quad .. + 3
+  const int dim_quad = tid / (kKeys / 4);    // dimensions 4 dim_quad .. + 3
+  const auto load = [&](int key0) {
+    const std::uint32_t from = 4U * D * static_cast<std::uint32_t>(key0);
+#pragma unroll
+    for (int i = 0; i < kKeyLoads; ++i) {
+      const std::uint32_t piece = static_cast<std::uint32_t>(tid + kThreads * i);
+      key_next[i][0] = load16(keys, from + 32U * piece);
+      key_next[i][1] = load16(keys, from + 32U * piece + 16U);
+    }
+    if (kValueThreads == kThreads || tid < kValueThreads) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        value_next[j] =
+            load16(values, from + 4U * static_cast<std::uint32_t>(D * (4 * value_quad + j) +
+                                                                  4 * dim_quad));
+    }
+  };
+  const auto store = [&]() {
+#pragma unroll
+    for (int i = 0; i < kKeyLoads; ++i) {
+      const int piece = tid + kThreads * i;
+      const int key = piece / kChunks;
+      const Octet o = bf16x3::Split(key_next[i][0], key_next[i][1]);
+      // Chunk c of key s at c ^ (s % 8): the 16-byte reads of eight
+      // consecutive keys fall on distinct banks.
+      const int at = key * kChunks + ((piece % kChunks) ^ (key % 8));
+      key_planes[0][at] = o.h;
+      key_planes[1][at] = o.m;
+      key_planes[2][at] = o.l;
+    }
+    if (kValueThreads == kThreads || tid < kValueThreads) {
+      const float4(&v)[4] = value_next;
+      const float rows[4][4] = {{v[0].x, v[1].x, v[2].x, v[3].x},
+                                {v[0].y, v[1].y, v[2].y, v[3].y},
+                                {v[0].z, v[1].z, v[2].z, v[3].z},
+                                {v[0].w, v[1].w, v[2].w, v[3].w}};
+      // S^T leaves keys 16 c + 8 j + 4 half + 0..3 in one lane's registers:
+      // the row holds, per 16 keys, half 0's two quads and then half 1's.
+      const int slot = (value_quad / 4) * 32 + (value_quad % 2) * 16 + ((value_quad / 2) % 2) * 8;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const bf16x3::Pair p0 = bf16x3::Split(rows[e][0], rows[e][1]);
+        const bf16x3::Pair p1 = bf16x3::Split(rows[e][2], rows[e][3]);
+        const int at = (4 * dim_quad + e) * kValueRow + slot;
+        *reinterpret_cast<uint2*>(&value_planes[0][at]) = uint2{p0.h, p1.h};
+        *reinterpret_cast<uint2*>(&value_planes[1][at]) = uint2{p0.m, p1.m};
+        *reinterpret_cast<uint2*>(&value_planes[2][at]) = uint2{p0.l, p1.l};
+      }
+    }
+  };
+
+  load(key_begin);
+  Octet qs[kSteps];
+  {
+    const float* source = a.q + (static_cast<std::size_t>(row) * a.heads + head) * D + 8 * half;
+#pragma unroll
+    for (int s = 0; s < kSteps; ++s) {
+      float4 x = reinterpret_cast<const float4*>(source + 16 * s)[0];
+      float4 y = reinterpret_cast<const float4*>(source + 16 * s)[1];
+      x = make_float4(x.x * a.scale, x.y * a.scale, x.z * a.scale, x.w * a.scale);
+      y = make_float4(y.x * a.scale, y.y * a.scale, y.z * a.scale, y.w * a.scale);
+      qs[s] = bf16x3::Split(x, y);
+    }
+  }
+
+  F32x16 out[kTiles];
+#pragma unroll
+  for (int i = 0; i < kTiles; ++i)
+#pragma unroll
+    for (int v = 0; v < 16; ++v)
+      out[i][v] = 0.0F;
+  float maximum = -INFINITY;
+  float sum = 0.0F;  // of this lane's keys
+
+  for (int key0 = key_begin; key0 < key_end; key0 += kKeys) {
+    __syncthreads();  // the step before has been read
+    store();
+    __syncthreads();
+    if (key0 + kKeys < key_end)
+      load(key0 + kKeys);
+    if (key0 >= wave_keys)
+      continue;
+
+    F32x16 score;
+#pragma unroll
+    for (int v = 0; v < 16; ++v)
+      score[v] = 0.0F;
+#pragma unroll
+    for (int s = 0; s < kSteps; ++s) {
+      const int at = column * kChunks + ((2 * s + half) ^ (column % 8));
+      const Octet o{key_planes[0][at], key_planes[1][at], key_planes[2][at]};
+      score = bf16x3::Multiply(o, qs[s], score);
+    }
+    float p[16];
+#pragma unroll
+    for (int v = 0; v < 16; ++v)
+      p[v] = score[v];
+    const bool masked = key0 + kKeys > whole_keys;
+    if (masked) {
+#pragma unroll
+      for (int v = 0; v < 16; ++v)
+        if (key0 + 8 * (v / 4) + 4 * half + v % 4 >= my_keys)
+          p[v] = -INFINITY;
+    }
+    float top = p[0];
+#pragma unroll
+    for (int v = 1; v < 16; ++v)
+      top = fmaxf(top, p[v]);
+    top = fmaxf(maximum, MaxXor32(top));
+    if (__any(top > maximum)) {
+      // (-inf - top would make 2^(x log2 e)'s correction a NaN.)
+      const float decay = maximum == -INFINITY ? 0.0F : ExpNegative(maximum - top);
+      sum *= decay;
+#pragma unroll
+      for (int i = 0; i < kTiles; ++i)
+#pragma unroll
+        for (int v = 0; v < 16; ++v)
+          out[i][v] *= decay;
+      maximum = top;
+    }
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+      const bool drop = masked && p[v] == -INFINITY;
+      const float e = ExpNegative(drop ? 0.0F : p[v] - maximum);
+      p[v] = drop ? 0.0F : e;
+      sum += p[v];
+    }
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      const Octet weights =
+          bf16x3::Split(make_float4(p[8 * c], p[8 * c + 1], p[8 * c + 2], p[8 * c + 3]),
+                        make_float4(p[8 * c + 4], p[8 * c + 5], p[8 * c + 6], p[8 * c + 7]));
+#pragma unroll
+      for (int i = 0; i < kTiles; ++i) {
+        const int at = (32 * i + column) * kValueRow + 32 * c + 16 * half;
+        const Octet o{*reinterpret_cast<const uint4*>(&value_planes[0][at]),
+                      *reinterpret_cast<const uint4*>(&value_planes[1][at]),
+                      *reinterpret_cast<const uint4*>(&value_planes[2][at])};
+        out[i] = bf16x3::Multiply(o, weights, out[i]);
+      }
+    }
+  }
+
+  sum = AddXor32(sum);
+  if (key_begin >= my_keys)
+    return;  // past the last query, or before this chunk: nothing to leave
+  // Element v of tile i: dimension 32 i + 8 (v / 4) + 4 half + v % 4.
+  const std::size_t at = static_cast<std::size_t>(row) * a.heads + head;
+  if (a.splits == 1) {
+    const float inverse = 1.0F / sum;
+    Bf16* target = a.out + at * D + 4 * half;
+#pragma unroll
+    for (int i = 0; i < kTiles; ++i)
+#pragma unroll
+      for (int b = 0; b < 4; ++b)
+        *reinterpret_cast<uint2*>(target + 32 * i + 8 * b) =
+            uint2{q8::PackBf16x2(out[i][4 * b] * inverse, out[i][4 * b + 1] * inverse),
+                  q8::PackBf16x2(out[i][4 * b + 2] * inverse, out[i][4 * b + 3] * inverse)};
+    return;
+  }
+  float* target = a.values + (at * a.splits + split) * D + 4 * half;
+#pragma unroll
+  for (int i = 0; i < kTiles; ++i)
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+      *reinterpret_cast<float4*>(target + 32 * i + 8 * b) =
+          make_float4(out[i][4 * b], out[i][4 * b + 1], out[i][4 * b + 2], out[i][4 * b + 3]);
+  if (half == 0) {
+    float* stats = a.stats + (at * a.splits + split) * 2;
+    stats[0] = maximum;
+    stats[1] = sum;
+  }
+}
+
+/// The chunks of a (row, head) met in chunk order: M = max m_c, L = sum
+/// l_c exp(m_c - M), out = bf16(sum o_c exp(m_c - M) / L) over the row's
+/// chunks. D / 4 lanes per (row, head), four dimensions each.
+template<int D>
+__global__ __launch_bounds__(kThreads) void MergeChunksKernel(TileArgs a, int items) {
+  constexpr int kLanes = D / 4;
+  constexpr int kBatch = 4;
+  const int item = static_cast<int>(blockIdx.x) * (kThreads / kLanes) +
+                   static_cast<int>(threadIdx.x) / kLanes;
+  if (item >= items)
+    return;
+  const int lane = static_cast<int>(threadIdx.x) % kLanes;
+  const int local = (item / a.heads) % a.rows_per_sequence;
+  const int keys = a.past + (a.causal != 0 ? local + 1 : a.rows_per_sequence);
+  const int chunks = (keys + a.chunk - 1) / a.chunk;
+  const std::size_t first = static_cast<std::size_t>(item) * a.splits;
+  const float2* stats = reinterpret_cast<const float2*>(a.stats) + first;
+  const float4* values = reinterpret_cast<const float4*>(a.values + first * D) + lane;
+  float top = -INFINITY;
+  for (int c = 0; c < chunks; ++c)
+    top = fmaxf(top, stats[c].x);
+  float4 out = make_float4(0.0F, 0.0F, 0.0F, 0.0F);
+  float sum = 0.0F;
+  for (int c0 = 0; c0 < chunks; c0 += kBatch) {
+    float4 v[kBatch];
+    float2 s[kBatch];
+#pragma unroll
+    for (int b = 0; b < kBatch; ++b) {
+      const int c = min(c0 + b, chunks - 1);
+      v[b] = values[static_cast<std::size_t>(c) * kLanes];
+      s[b] = stats[c];
+    }
+#pragma unroll
+    for (int b = 0; b < kBatch; ++b) {
+      if (c0 + b >= chunks)
+        break;
+      const float f = expf(s[b].x - top);
+      sum += s[b].y * f;
+      out.x += v[b].x * f;
+      out.y += v[b].y * f;
+      out.z += v[b].z * f;
+      out.w += v[b].w * f;
+    }
+  }
+  const float inverse = 1.0F / sum;
+  *reinterpret_cast<uint2*>(a.out + static_cast<std::size_t>(item) * D + 4 * lane) =
+      uint2{q8::PackBf16x2(out.x * inverse, out.y * inverse),
+            q8::PackBf16x2(out.z * inverse, out.w * inverse)};
+}
+
+template<int D>
+void Launch(const TileArgs& args, std::size_t workgroups, std::size_t items, hipStream_t stream) {
+  TileAttentionKernel<D><<<static_cast<unsigned>(workgroups), kThreads, 0, stream>>>(args);
+  if (args.splits > 1) {
+    constexpr std::size_t kItems = kThreads / (D / 4);
+    MergeChunksKernel<D><<<static_cast<unsigned>((items + kItems - 1) / kItems), kThreads, 0,
+                           stream>>>(args, static_cast<int>(items));
+  }
+}
+
+bool Aligned16(const void* p) { return reinterpret_cast<std::uintptr_t>(p) % 16 == 0; }
+
+}  // namespace
+
+bool UseTileAttention(const AttentionShape& s, const float* q, const float* k_cache,
+                      const float* v_cache, const Bf16* out, const float* partials) {
+  const std::size_t group = s.heads / s.kv_heads;
+  // The kernel's indices are 32-bit; the caches are read in 16-byte pieces.
+  return s.rows_per_sequence * group >= 32 && s.rows * s.heads < (std::size_t{1} << 24) &&
+         s.past + s.rows_per_sequence < (std::size_t{1} << 21) && Aligned16(q) &&
+         Aligned16(k_cache) && Aligned16(v_cache) && Aligned16(out) && Aligned16(partials);
+}
+
+void TileAttention(const AttentionShape& s, const float* q, const float* k_cache,
+                   const float* v_cache, Bf16* out, float* partials, hipStream_t stream) {
+  const std::size_t group = s.heads / s.kv_heads;
+  const std::size_t sequences = s.rows / s.rows_per_sequence;
+  const std::size_t queries = s.rows_per_sequence * group;
+  const std::size_t blocks = (queries + kQueries - 1) / kQueries;
+  // Steps of all query blocks, and the chunk that cuts them into about
+  // kTargetWorkgroups runs.
+  std::size_t steps = 0;
+  for (std::size_t b = 0; b < blocks; ++b) {
+    const std::size_t last = std::min((b + 1) * kQueries, queries) - 1;
+    const std::size_t keys = s.past + (s.causal ? last / group + 1 : s.rows_per_sequence);
+    steps += (keys + kKeys - 1) / kKeys;
+  }
+  steps *= sequences * s.kv_heads;
+  const std::size_t most = s.past + s.rows_per_sequence;
+  const std::size_t chunk =
+      std::max<std::size_t>(kLeastChunk, (steps + kTargetWorkgroups - 1) / kTargetWorkgroups *
+                                             kKeys);
+  const std::size_t splits = (most + chunk - 1) / chunk;
+  TileArgs args{};
+  args.q = q;
+  args.k = k_cache;
+  args.v = v_cache;
+  args.out = out;
+  args.values = partials;
+  args.stats = partials == nullptr ? nullptr : partials + s.rows * s.heads * splits * s.head_dim;
+  args.rows_per_sequence = static_cast<int>(s.rows_per_sequence);
+  args.keys_per_sequence = static_cast<int>(s.keys_per_sequence);
+  args.past = static_cast<int>(s.past);
+  args.causal = s.causal ? 1 : 0;
+  args.heads = static_cast<int>(s.heads);
+  args.kv_heads = static_cast<int>(s.kv_heads);
+  args.capacity = static_cast<int>(s.capacity);
+  args.blocks = static_cast<int>(blocks);
+  args.chunk = static_cast<int>(chunk);
+  args.splits = static_cast<int>(splits);
+  args.scale = 1.0F / std::sqrt(static_cast<float>(s.head_dim));
+  const std::size_t workgroups = sequences * s.kv_heads * blocks * splits;
+  const std::size_t items = s.rows * s.heads;
+  if (s.head_dim == 64)
+    Launch<64>(args, workgroups, items, stream);
+  else
+    Launch<128>(args, workgroups, items, stream);
+}
+
+}  // namespace vx

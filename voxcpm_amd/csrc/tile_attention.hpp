@@ -1,0 +1,34 @@
+// The many-row attention over a key/value cache (tile_attention.hip).
+#ifndef VOXCPM_AMD_TILE_ATTENTION_HPP_
+#define VOXCPM_AMD_TILE_ATTENTION_HPP_
+
+#include <hip/hip_runtime.h>
+
+#include <cstddef>
+
+#include "common.hpp"
+
+namespace vx {
+
+/// Attention's arguments (kernels/generator_kernels.hip:160-241): q
+/// [rows][heads][head_dim] rotated and unscaled, one layer's caches
+/// [kv_heads][capacity][head_dim], out [rows][heads head_dim] row-major.
+struct AttentionShape {
+  std::size_t rows, rows_per_sequence, keys_per_sequence, past;
+  bool causal;
+  std::size_t heads, kv_heads, head_dim, capacity;
+};
+
+/// Whether the matrix-core attention takes these pointers and this shape,
+/// and is the faster kernel for it.
+bool UseTileAttention(const AttentionShape& s, const float* q, const float* k_cache,
+                      const float* v_cache, const Bf16* out, const float* partials);
+
+/// `partials`: rows x heads x ceil(keys / 64) x (head_dim + 2) floats, or
+/// null where a row attends to at most 64 keys.
+void TileAttention(const AttentionShape& s, const float* q, const float* k_cache,
+                   const float* v_cache, Bf16* out, float* partials, hipStream_t stream);
+
+}  // namespace vx
+
+#endif  // VOXCPM_AMD_TILE_ATTENTION_HPP_
