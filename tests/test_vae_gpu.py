@@ -139,3 +139,66 @@ def test_vae_decode_argument_checks(vx, cuda):
         vae.decode(good, torch.empty(4 * config.hop - 1, dtype=torch.float32, device=cuda))
     vae.decode(good, torch.empty(4 * config.hop, dtype=torch.float32, device=cuda))
     torch.cuda.synchronize()
+
+
+# Chunks of 9 frames and more take the wide path (float32 products as float16
+# pairs, units of 32 and 64 channels in one launch): "wide" has a product
+# per kind of block (128 channels by depthwise launch and product, 64 and 32
+# fused), row counts that fill no tile at every dilation, and shorter
+# chunks between wide ones, whose histories the two paths share.
+WIDE = synth.VaeConfig(latent=16, decoder_dim=256, rates=(8, 3, 2))
+
+
+@pytest.mark.parametrize("chunks", [(20, 4, 31), (9, 9), (3, 50, 1, 10)])
+def test_vae_wide_chunks_against_oracle(vx, oracle, cuda, stream, chunks):
+    weights = synth.vae_weights(WIDE, 101)
+    frames = sum(chunks)
+    latents = synth.Rng(102, frames).normal(frames * WIDE.latent).astype(np.float32)
+    latents = latents.reshape(frames, WIDE.latent)
+    ref = oracle.OracleVae(weights).decode(latents)
+    vae = vx.Vae(weights)
+    device_latents = torch.from_numpy(latents).to(cuda)
+    for attempt in range(3):  # the same buffers again: eager, captured, replayed
+        pieces, at = [], 0
+        for n in chunks:
+            pieces.append(vae.decode(device_latents[at:at + n]).cpu().numpy())
+            at += n
+        error = float(np.max(np.abs(np.concatenate(pieces) - ref)))
+        print(f"wide {chunks} stream {attempt}: max |d| {error:.2e}", flush=True)
+        assert error <= BOUND
+        vae.reset()
+
+
+def test_vae_wide_past_float16(vx, oracle, cuda):
+    """Activations of 1e6 (the input convolution scaled up, the output one
+    scaled down): past float16's range the wide path's workgroups start over
+    from bfloat16 triples."""
+    weights = synth.vae_weights(WIDE, 103)
+    weights.tensors["in_pointwise"] = weights.tensors["in_pointwise"] * np.float32(1e6)
+    weights.tensors["out_conv"] = weights.tensors["out_conv"] * np.float32(1e-6)
+    frames = 25
+    latents = synth.Rng(104, frames).normal(frames * WIDE.latent).astype(np.float32)
+    latents = latents.reshape(frames, WIDE.latent)
+    ref = oracle.OracleVae(weights).decode(latents)
+    got = vx.Vae(weights).decode(torch.from_numpy(latents).to(cuda)).cpu().numpy()
+    error = float(np.max(np.abs(got - ref)))
+    print(f"past float16: max |d| {error:.2e}, signal std {np.std(ref):.3f}", flush=True)
+    assert np.std(ref) > 0.1
+    assert error <= BOUND
+
+
+def test_vae_wide_against_short_chunks(vx, cuda):
+    """61 frames at the VoxCPM2 shape at once (every product tile shape of
+    the wide path) against the same latents in chunks of 8 frames, which
+    take the float32 kernels."""
+    config = CONFIGS["voxcpm2"]
+    weights = synth.vae_weights(config, 105)
+    frames = 61
+    latents = torch.from_numpy(synth.Rng(106, frames).normal(frames * config.latent).astype(
+        np.float32).reshape(frames, config.latent)).to(cuda)
+    at_once = vx.Vae(weights).decode(latents).cpu().numpy()
+    chunked = vx.Vae(weights)
+    pieces = [chunked.decode(latents[at:at + 8]).cpu().numpy() for at in range(0, frames, 8)]
+    error = float(np.max(np.abs(at_once - np.concatenate(pieces))))
+    print(f"wide against 8-frame chunks: max |d| {error:.2e}", flush=True)
+    assert error <= BOUND

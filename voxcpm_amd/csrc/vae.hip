@@ -20,8 +20,9 @@
 // products (the reference calls hipblasSgemm) take float32 MFMA kernels:
 // 16-column, 32-row tiles that read the weights in place, or, where those
 // tiles would re-read over 32 MiB of activations between them, 32 x 32
-// tiles staged through LDS. Up to 16 latent frames per chunk the launches
-// replay as one HIP graph.
+// tiles staged through LDS. From 9 frames a chunk takes the wide path
+// (LaunchBlocksWide, vae_wide.hip). Up to 16 latent frames per chunk the
+// launches replay as one HIP graph.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -31,16 +32,24 @@
 
 #include "common.hpp"
 #include "q8_tile.hpp"
+#include "snake.hpp"
+#include "vae_wide.hpp"
 #include "voxcpm_amd.h"
 
 namespace {
 
 using vx::kWave;
+using vx::Snake;
+using vx::SnakeScale;
 
 constexpr int kThreads = 256;
 constexpr int kTaps = 7;
 constexpr int kDilations[3] = {1, 3, 9};
 constexpr std::size_t kMaxGraphFrames = 16;
+// Fewest frames of the wide path (measured on MI355X at VoxCPM2's shape: a
+// chunk of 8 frames 309 us on the few-row kernels, 335 us on the wide path;
+// 9 frames 354 and 338 us, 16 frames 435 and 357 us).
+constexpr std::size_t kWideFrames = 9;
 // Output samples per decode call: a product's row blocks of 32 rows are
 // grid rows, at most 65535 of them.
 constexpr std::size_t kMaxSamples = std::size_t{65535} * 32;
@@ -56,21 +65,6 @@ constexpr int kWaveThreads = kWave;
 dim3 WaveBlocks(std::size_t count) {
   return dim3(static_cast<unsigned>((count + kWaveThreads - 1) / kWaveThreads));
 }
-
-/// A channel's 1 / (a + 1e-9) in Snake.
-__device__ inline float SnakeScale(float a) { return 1.0F / (a + 1e-9F); }
-/// Snake(y) = y + sin^2(a y) / (a + 1e-9), `inverse` the channel's
-/// SnakeScale(a). The sine is the hardware's (v_sin_f32 takes turns:
-/// sin(2 pi r)) of a y in turns reduced to [-1/2, 1/2]: the decoder
-/// evaluates Snake on every element of every unit and block input, and the
-/// library sine's range reduction and polynomial made the units' products
-/// bound by their vector instructions.
-__device__ inline float Snake(float y, float a, float inverse) {
-  const float turns = a * y * 0.159154943091895336F;  // 1 / (2 pi)
-  const float s = __builtin_amdgcn_sinf(turns - rintf(turns));
-  return y + inverse * (s * s);
-}
-__device__ inline float Snake(float y, float a) { return Snake(y, a, SnakeScale(a)); }
 
 /// Up to N copies (to[e] = from[e], e < count) spread over every thread of
 /// a grid: each thread's first element is loaded by Load() beside the
@@ -162,16 +156,26 @@ __global__ void DepthwiseKernel(const float* work, const float* w, const float* 
 /// be): lane q takes channel quads q, q + lanes, .., each with one 16-byte
 /// load per tap and its four channels' 28 taps as seven 16-byte loads, and
 /// the frame's lanes add their sums by butterfly. Also state = work's last
-/// 6 rows (this kernel never reads the state) and copy_to = copy_from
-/// (copy_count floats: the latents' history, which the first product of
-/// the chunk read). c a multiple of 4.
+/// 6 rows (this kernel never reads the state) and two more refreshes,
+/// copies[i].to = copies[i].from: the latents' history, which the first
+/// product of the chunk read, and the wide path's states. c a multiple of 4.
+struct Refresh {
+  const float* from = nullptr;
+  float* to = nullptr;
+  int count = 0;
+};
+struct Refreshes {
+  Refresh latents;
+  Refresh states;
+};
 __global__ void ToMonoKernel(const float* work, const float* w, float b, float* samples,
                              float* state, std::size_t t, std::size_t c, int lanes,
-                             const float* copy_from, float* copy_to, int copy_count) {
+                             Refreshes refreshes) {
   const std::size_t i = static_cast<std::size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  SideCopies<2> copies;  // the state refreshes, loaded beside the window
+  SideCopies<3> copies;  // the state refreshes, loaded beside the window
   copies.Add(0, state, work + t * c, static_cast<int>((kTaps - 1) * c));
-  copies.Add(1, copy_to, copy_from, copy_count);
+  copies.Add(1, refreshes.latents.to, refreshes.latents.from, refreshes.latents.count);
+  copies.Add(2, refreshes.states.to, refreshes.states.from, refreshes.states.count);
   copies.Load();
   const std::size_t f = i / static_cast<std::size_t>(lanes);
   const int q = static_cast<int>(i % static_cast<std::size_t>(lanes));
@@ -926,6 +930,23 @@ struct Block {
   float* up2 = nullptr;       // [s out][2 in]
   float* state = nullptr;     // [in]: the last frame's Snake output
   float* unit_state[3] = {};  // [6 d][out]
+
+  std::size_t UnitStateFloats(int unit) const {
+    return static_cast<std::size_t>(kTaps - 1) * kDilations[unit] * out;
+  }
+  std::size_t StateFloats() const {
+    return in + UnitStateFloats(0) + UnitStateFloats(1) + UnitStateFloats(2);
+  }
+  /// Places the histories from `at` on; returns their end.
+  float* PlaceStates(float* at) {
+    state = at;
+    at += in;
+    for (int u = 0; u < 3; ++u) {
+      unit_state[u] = at;
+      at += UnitStateFloats(u);
+    }
+    return at;
+  }
 };
 
 struct GraphKey {
@@ -947,6 +968,15 @@ struct vx_vae {
   std::vector<Block> blocks;
   std::size_t out_channels = 0;
   std::size_t hop = 1;
+  // Every history in one allocation (a reset is one launch): the blocks'
+  // states and their units', then the latents' and the output's.
+  float* states = nullptr;
+  std::size_t state_floats = 0;
+  // The wide path leaves the blocks' and units' histories at the same
+  // offsets of states_next; its last launch copies the first
+  // block_state_floats of it back.
+  float* states_next = nullptr;
+  std::size_t block_state_floats = 0;
   float* in_state = nullptr;   // [6][latent]
   float* in_state_next = nullptr;  // [6][latent]: the next chunk's, copied in at the end
   float* out_state = nullptr;  // [6][out_channels]
@@ -964,14 +994,10 @@ struct vx_vae {
   ~vx_vae() {
     if (graph != nullptr)
       (void)hipGraphExecDestroy(graph);
-    for (Block& b : blocks) {
+    for (Block& b : blocks)
       (void)hipFree(b.up2);
-      (void)hipFree(b.state);
-      for (float* s : b.unit_state)
-        (void)hipFree(s);
-    }
-    for (void* p : {static_cast<void*>(in_state), static_cast<void*>(in_state_next),
-                    static_cast<void*>(out_state),
+    for (void* p : {static_cast<void*>(states), static_cast<void*>(states_next),
+                    static_cast<void*>(in_state_next),
                     static_cast<void*>(hidden), static_cast<void*>(next),
                     static_cast<void*>(work), static_cast<void*>(scratch),
                     static_cast<void*>(scratch2), static_cast<void*>(partials)})
@@ -1152,6 +1178,105 @@ struct vx_vae {
     return VX_OK;
   }
 
+  /// Whether a chunk takes the wide path (LaunchBlocksWide): kWideFrames
+  /// frames, channels whole reduction steps of 32, every unit's chunk at
+  /// least its history (54 rows), and operands within the kernels' 31-bit
+  /// offsets.
+  bool Wide(std::size_t frames) const {
+    if (frames < kWideFrames || out_channels % 32 != 0)
+      return false;
+    constexpr std::size_t kMost = std::size_t{1} << 31;
+    std::size_t t = frames;
+    for (const Block& b : blocks) {
+      const std::size_t up = t * b.stride;
+      if (up < (kTaps - 1) * kDilations[2] || (t + 1) * 2 * b.in * sizeof(float) >= kMost ||
+          (up + kTaps) * b.out * sizeof(float) >= kMost ||
+          b.stride * b.out * 2 * b.in * sizeof(float) >= kMost)
+        return false;
+      t = up;
+    }
+    return true;
+  }
+
+  /// The decoder blocks over many rows (vae_wide.hip), from block 0's input
+  /// x2 in `work`: per block the transposed convolution into the stream and
+  /// three units, each one launch where its channels allow (else the
+  /// depthwise convolution and a product); the last unit makes the next
+  /// block's input rows in `work` or the output window in scratch2.
+  /// Histories are left in states_next.
+  void LaunchBlocksWide(std::size_t frames, float* stream_rows, float* next_rows,
+                        hipStream_t stream) {
+    const auto next_of = [&](float* state) { return states_next + (state - states); };
+    std::size_t t = frames;
+    for (std::size_t bi = 0; bi < blocks.size(); ++bi) {
+      const Block& b = blocks[bi];
+      vx::vae::Product up;
+      up.x = work;
+      up.w = b.up2;
+      up.taps = bi > 0;
+      up.tail = bi > 0 ? nullptr : next_of(b.state);
+      up.t = static_cast<int>(t);
+      up.k = static_cast<int>(2 * b.in);
+      up.n = static_cast<int>(b.stride * b.out);
+      up.epilogue.bias = b.w.up_bias;
+      up.epilogue.channels = static_cast<int>(b.out);
+      up.epilogue.out = next_rows;
+      vx::vae::RunProduct(up, stream);
+      std::swap(stream_rows, next_rows);
+      t *= b.stride;
+      for (int u = 0; u < 3; ++u) {
+        const vx_vae_unit& w = b.w.units[u];
+        vx::vae::Unit unit;
+        unit.y = stream_rows;
+        unit.alpha_in = w.alpha_in;
+        unit.taps = w.depthwise;
+        unit.bias = w.depthwise_bias;
+        unit.alpha_out = w.alpha_out;
+        unit.state = b.unit_state[u];
+        unit.state_next = next_of(b.unit_state[u]);
+        unit.t = static_cast<int>(t);
+        unit.c = static_cast<int>(b.out);
+        unit.d = kDilations[u];
+        vx::vae::Epilogue e;
+        e.bias = w.pointwise_bias;
+        e.channels = static_cast<int>(b.out);
+        e.prior = stream_rows;
+        if (u == 2 && bi + 1 < blocks.size()) {
+          const Block& after = blocks[bi + 1];
+          e.target = vx::vae::Target::kBlockInput;
+          e.out = work;
+          e.scale = after.w.scale;
+          e.shift = after.w.bias;
+          e.alpha = after.w.alpha;
+          e.history = after.state;
+          e.history_next = next_of(after.state);
+        } else if (u == 2) {
+          e.target = vx::vae::Target::kOutput;
+          e.out = scratch2;
+          e.alpha = weights.out_alpha;
+          e.history = out_state;
+        }
+        if (vx::vae::UnitSupported(b.out)) {
+          if (u < 2)
+            e.out = next_rows;
+          vx::vae::RunUnit(unit, w.pointwise, e, stream);
+          std::swap(stream_rows, next_rows);
+          continue;
+        }
+        vx::vae::RunDepthwise(unit, scratch, stream);
+        vx::vae::Product product;
+        product.x = scratch;
+        product.w = w.pointwise;
+        product.t = unit.t;
+        product.k = product.n = unit.c;
+        product.epilogue = e;
+        if (u < 2)
+          product.epilogue.out = stream_rows;
+        vx::vae::RunProduct(product, stream);
+      }
+    }
+  }
+
   int Launch(const float* latents, std::size_t frames, float* samples, hipStream_t stream) {
     const std::size_t latent = shape.latent_dim;
     // The residual stream and the transposed convolutions' outputs trade
@@ -1243,7 +1368,12 @@ struct vx_vae {
                                stream_rows, latent, shape.decoder_dim, false,
                                block_input_of(blocks.front(), weights.in_pointwise_bias)));
     }
-    for (std::size_t bi = 0; bi < blocks.size(); ++bi) {
+    const bool wide = Wide(frames);
+    if (wide) {
+      LaunchBlocksWide(frames, stream_rows, next_rows, stream);
+      t = frames * hop;
+    }
+    for (std::size_t bi = 0; bi < blocks.size() && !wide; ++bi) {
       Block& b = blocks[bi];
       const std::size_t t_in = t;
       const std::size_t c = b.out;
@@ -1276,15 +1406,20 @@ struct vx_vae {
       }
     }
     const std::size_t c = out_channels;
-    float* out_window = windows[1];  // the last unit's (u = 2) next window
+    float* out_window = windows[1];  // the last unit's (u = 2) next window (scratch2)
     int lanes = 1;
     while (lanes < kWave && 4 * static_cast<std::size_t>(lanes) < c)
       lanes *= 2;
-    const std::size_t copy_floats = input_fused ? (kTaps - 1) * latent : 0;
-    ToMonoKernel<<<Blocks(std::max({t * lanes, (kTaps - 1) * c, copy_floats})), kThreads, 0,
-                   stream>>>(out_window, weights.out_conv, weights.out_bias, samples, out_state,
-                             t, c, lanes, input_fused ? in_state_next : nullptr,
-                             input_fused ? in_state : nullptr, static_cast<int>(copy_floats));
+    Refreshes refreshes;
+    if (input_fused)
+      refreshes.latents =
+          Refresh{in_state_next, in_state, static_cast<int>((kTaps - 1) * latent)};
+    if (wide)
+      refreshes.states = Refresh{states_next, states, static_cast<int>(block_state_floats)};
+    ToMonoKernel<<<Blocks(std::max({t * lanes, (kTaps - 1) * c,
+                                    static_cast<std::size_t>(refreshes.latents.count)})),
+                   kThreads, 0, stream>>>(out_window, weights.out_conv, weights.out_bias, samples,
+                                          out_state, t, c, lanes, refreshes);
     return vx::LaunchStatus("vx_vae_decode");
   }
 };
@@ -1345,12 +1480,7 @@ int vx_vae_create(vx_vae** vae, const vx_vae_shape* shape, const vx_vae_weights*
     block.w = weights->blocks[b];
     created->hop *= block.stride;
     status = Allocate(&block.up2, block.stride * block.out * 2 * block.in, "vx_vae: hipMalloc");
-    if (status == VX_OK)
-      status = Allocate(&block.state, block.in, "vx_vae: hipMalloc");
-    for (int u = 0; u < 3 && status == VX_OK; ++u)
-      status = Allocate(&block.unit_state[u],
-                        static_cast<std::size_t>(kTaps - 1) * kDilations[u] * block.out,
-                        "vx_vae: hipMalloc");
+    created->block_state_floats += block.StateFloats();
     if (status == VX_OK) {
       const std::size_t count = block.stride * block.out * 2 * block.in;
       RepackUpKernel<<<Blocks(count), kThreads>>>(block.w.up, block.up2, block.in, block.out,
@@ -1361,13 +1491,20 @@ int vx_vae_create(vx_vae** vae, const vx_vae_shape* shape, const vx_vae_weights*
     c /= 2;
   }
   created->out_channels = c;
+  created->state_floats =
+      created->block_state_floats + (kTaps - 1) * (shape->latent_dim + c);
   if (status == VX_OK)
-    status = Allocate(&created->in_state, (kTaps - 1) * shape->latent_dim, "vx_vae: hipMalloc");
+    status = Allocate(&created->states, created->state_floats, "vx_vae: hipMalloc");
+  if (status == VX_OK)
+    status = Allocate(&created->states_next, created->block_state_floats, "vx_vae: hipMalloc");
   if (status == VX_OK)
     status = Allocate(&created->in_state_next, (kTaps - 1) * shape->latent_dim,
                       "vx_vae: hipMalloc");
-  if (status == VX_OK)
-    status = Allocate(&created->out_state, (kTaps - 1) * c, "vx_vae: hipMalloc");
+  float* state = created->states;
+  for (Block& block : created->blocks)
+    state = block.PlaceStates(state);
+  created->in_state = state;
+  created->out_state = state + (kTaps - 1) * shape->latent_dim;
   if (status == VX_OK && hipDeviceSynchronize() != hipSuccess)
     status = vx::Fail(VX_HIP_ERROR, "vx_vae_create: repack");
   if (status != VX_OK) {
@@ -1384,18 +1521,8 @@ int vx_vae_reset(vx_vae* vae, void* stream) {
   if (vae == nullptr)
     return vx::Fail(VX_BAD_ARG, "vx_vae_reset: null handle");
   hipStream_t s = vx::Stream(stream);
-  const auto clear = [&](float* p, std::size_t count) {
-    ZeroKernel<<<Blocks(count), kThreads, 0, s>>>(p, count);
-    return hipGetLastError() == hipSuccess;
-  };
-  bool ok = clear(vae->in_state, (kTaps - 1) * vae->shape.latent_dim) &&
-            clear(vae->out_state, (kTaps - 1) * vae->out_channels);
-  for (Block& b : vae->blocks) {
-    ok = ok && clear(b.state, b.in);
-    for (int u = 0; u < 3; ++u)
-      ok = ok && clear(b.unit_state[u], static_cast<std::size_t>(kTaps - 1) * kDilations[u] * b.out);
-  }
-  if (!ok)
+  ZeroKernel<<<Blocks(vae->state_floats), kThreads, 0, s>>>(vae->states, vae->state_floats);
+  if (hipGetLastError() != hipSuccess)
     return vx::Fail(VX_HIP_ERROR, "vx_vae_reset: launch");
   return vx::Succeed();
 }
