@@ -546,7 +546,8 @@ def gpu_prefill(args, torch, ops, synth, device, stream):
         plan = (ctypes.c_int32 * 4)()
         _lib.check(_lib.lib().vx_q8_prefill_plan(m, k, n, scratch.handle, plan))
         names = {0: "TiledKernel (q8_tiled.hip)", 1: "GemmKernel (q8_gemm.hip)",
-                 2: "EngineKernel in blocks of 64 rows (q8_tile.hpp)"}
+                 2: "EngineKernel in blocks of 64 rows (q8_tile.hpp)",
+                 3: "PrefillKernel (q8_prefill.hip)"}
         split = f", k split {plan[3]} ways" if plan[3] > 1 else ""
         return names[plan[0]] + split
 

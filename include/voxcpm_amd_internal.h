@@ -41,8 +41,10 @@ int vx_q8_linear_engine(const uint16_t* x, const void* packed, float* y,
  * (128 x 256), 2 (128 x 128), 3 (256 x 128), 4 (256 x 256, two steps),
  * 5 (128 x 64), k split over `splits` workgroups (the scratch must hold
  * splits m n floats when splits > 1); shape 6 is the skinny engine in
- * blocks of 64 rows (no split). VX_UNSUPPORTED for other shapes. The plan
- * search behind vx_q8_linear's prefill plans. */
+ * blocks of 64 rows (no split); shapes 7 to 13 are the panel-operand
+ * kernels (128 x 256, 128 x 128 in 2 groups of k, 64 x 128 in 4, 64 x 64 and
+ * 32 x 64 in 8, 160 x 256, 96 x 256; no split). VX_UNSUPPORTED for other
+ * shapes. The plan search behind vx_q8_linear's prefill plans. */
 int vx_q8_linear_gemm(const uint16_t* x, const void* packed, float* y,
                       size_t m, size_t k, size_t n, int shape, int splits,
                       vx_scratch* scratch, void* stream);
@@ -61,8 +63,8 @@ int vx_q8_plan(size_t m, size_t k, size_t n, vx_scratch* scratch,
 
 /* The plan of an m x k x n product of more than 128 rows (the expanded
  * path) with this scratch: out4 = {kernel (0 the tiled kernel, 1 the
- * 32 x 32 MFMA kernel, 2 the skinny engine in blocks of 64 rows), rows per
- * tile, columns per tile, splits along k}.
+ * 32 x 32 MFMA kernel, 2 the skinny engine in blocks of 64 rows, 3 the
+ * panel-operand kernels), rows per tile, columns per tile, splits along k}.
  * Counterpart of the plan gemm.cpp:259-313 picks between hipBLASLt and
  * its chunked products. */
 int vx_q8_prefill_plan(size_t m, size_t k, size_t n, vx_scratch* scratch, int32_t* out4);

@@ -12,7 +12,7 @@ import numpy as np
 import pytest
 import torch
 
-from voxcpm_amd import synth
+from voxcpm_amd import _lib, synth
 
 pytestmark = pytest.mark.gpu
 
@@ -359,6 +359,37 @@ def test_prefill_benched_shapes(vx, oracle, cuda, stream, rows, n):
                            np.ascontiguousarray(blocks[cols]), oracle)
     print(f"prefill {rows}x{k}x{n}: worst {worst:.2e}", flush=True)
     assert worst <= 1e-4
+
+
+# Shapes 7 to 13 of vx_q8_linear_gemm: every tile of the panel-operand
+# kernels (rows x columns, groups of k), on sizes that end inside a tile, a
+# panel pair (k 96, 1120) and a group's run of k, and on fewer k steps than
+# groups.
+@pytest.mark.parametrize("shape", range(7, 14))
+@pytest.mark.parametrize("weights", ["q8", "bf16"])
+@pytest.mark.parametrize("rows,k,n", [(129, 96, 40), (161, 1120, 2055), (333, 64, 272),
+                                      (257, 4160, 130)])
+def test_panel_operand_shapes(vx, oracle, cuda, stream, shape, weights, rows, k, n):
+    rng = synth.Rng(11, rows + n)
+    x = synth.activations(rng, rows, k)
+    x_dev = to_device(x, cuda)
+    y = torch.full((rows, n), float("nan"), dtype=torch.float32, device=cuda)
+    if weights == "q8":
+        blocks = synth.q8_blocks(rng, n, k)
+        packed = vx.q8_pack(to_device(blocks, cuda), n, k)
+        function = _lib.lib().vx_q8_linear_gemm
+    else:
+        w = synth.bf16_bits((0.02 * rng.normal(n * k)).astype(np.float32)).reshape(n, k)
+        packed = vx.bf16_pack(to_device(w, cuda))
+        function = _lib.lib().vx_bf16_linear_gemm
+    _lib.check(function(x_dev.data_ptr(), packed.data_ptr(), y.data_ptr(), rows, k, n, shape, 1,
+                        None, torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    got = y.cpu().numpy()
+    worst = expanded_check(got, x, blocks, oracle) if weights == "q8" else \
+        oracle.bf16_check(got, x, w)
+    # float32 sums of at most 4160 products: 1e-5 of sum |x w|.
+    assert worst <= LIMIT, worst
 
 
 def test_stream_read_reads_every_byte(vx, cuda, stream):

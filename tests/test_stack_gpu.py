@@ -236,6 +236,22 @@ def test_stack_bf16_weights(vx, oracle, cuda, stream):
     run.step(h, [5], [5], 1, 1, 5, True, "bf16 decode")
 
 
+@pytest.mark.parametrize("bf16_weights", [False, True])
+@pytest.mark.parametrize("rows", [129, 170])
+def test_stack_prompt_rows(vx, oracle, cuda, stream, rows, bf16_weights):
+    """A prompt past the exact rows: the panel-operand products, SwiGLU in
+    gate_up's epilogue and the residual adds in o's and down's, then a
+    second prompt behind the first."""
+    config = STACKS["gqa-hd64"]
+    run = Run(vx, oracle, cuda, config, 49, capacity=2 * rows, bf16_weights=bf16_weights)
+    assert run.gpu.path(rows) == _lib.STACK_PATH_UNFUSED
+    rng = synth.Rng(50, rows)
+    for past in (0, rows):
+        h0 = rng.normal(rows * config.hidden).astype(np.float32).reshape(rows, config.hidden)
+        at = past + np.arange(rows)
+        run.step(h0, at, at, rows, rows, past, True, f"prompt of {rows} behind {past}")
+
+
 def test_stack_argument_errors(vx, cuda, stream):
     """Bad layouts fail before anything is launched."""
     config = STACKS["gqa-hd64"]

@@ -6,6 +6,7 @@
 
 #include "common.hpp"
 #include "products.hpp"
+#include "q8_prefill.hpp"
 #include "q8.hpp"
 #include "q8_tile.hpp"
 
@@ -113,6 +114,21 @@ int Product(const uint16_t* x, const void* packed, float* y, uint16_t* y_bf16,
             size_t m, size_t k, size_t n, int accumulate, vx_scratch* scratch,
             int rg, int waves, int splits, void* stream,
             vx::q8::Weights kind = vx::q8::Weights::kQ8) {
+  if (vx::prefill::Use(m, k, n)) {
+    vx::prefill::Product p;
+    p.x = x;
+    p.w = packed;
+    p.bf16 = kind != vx::q8::Weights::kQ8;
+    p.m = m;
+    p.k = k;
+    p.n = n;
+    p.kind = y == nullptr ? vx::prefill::Out::kBf16
+             : accumulate != 0 ? vx::prefill::Out::kAccumulate
+                               : vx::prefill::Out::kStore;
+    p.y = y;
+    p.out = y_bf16;
+    return vx::prefill::Run(p, vx::Stream(stream));
+  }
   if (vx::UseRowBlocks(m, k, n, kind == vx::q8::Weights::kQ8))
     return vx::RunRowBlocks(x, packed, y, y_bf16, m, k, n, accumulate != 0,
                             kind != vx::q8::Weights::kQ8, vx::Stream(stream));
@@ -135,6 +151,22 @@ int Product(const uint16_t* x, const void* packed, float* y, uint16_t* y_bf16,
                        scratch != nullptr ? scratch->partials : nullptr,
                        scratch != nullptr ? scratch->counters : nullptr,
                        vx::Stream(stream), kind);
+}
+
+/// The panel-operand prefill product (q8_prefill.hip) with a forced shape.
+int Prefill(const uint16_t* x, const void* packed, float* y, size_t m, size_t k, size_t n,
+            bool bf16, int shape, void* stream) {
+  if (shape >= vx::prefill::kShapes || !vx::prefill::Supported(m, k, n))
+    return vx::Fail(VX_UNSUPPORTED, "prefill product: no such plan");
+  vx::prefill::Product p;
+  p.x = x;
+  p.w = packed;
+  p.bf16 = bf16;
+  p.m = m;
+  p.k = k;
+  p.n = n;
+  p.y = y;
+  return vx::prefill::Run(p, vx::Stream(stream), shape);
 }
 
 }  // namespace
@@ -261,6 +293,8 @@ int vx_q8_linear_gemm(const uint16_t* x, const void* packed, float* y, size_t m,
     return vx::Fail(VX_BAD_ARG, "vx_q8_linear_gemm: more than 128 rows and a shape");
   if (shape == 6)  // the skinny engine in blocks of 64 rows
     return vx::RunRowBlocks(x, packed, y, nullptr, m, k, n, false, false, vx::Stream(stream));
+  if (shape > 6)
+    return Prefill(x, packed, y, m, k, n, false, shape - 7, stream);
   return vx::RunGemm(x, packed, y, nullptr, m, k, n, false, false,
                      scratch != nullptr ? scratch->partials : nullptr,
                      scratch != nullptr ? scratch->partial_floats : 0, vx::Stream(stream),
@@ -275,6 +309,8 @@ int vx_bf16_linear_gemm(const uint16_t* x, const void* packed, float* y, size_t 
     return vx::Fail(VX_BAD_ARG, "vx_bf16_linear_gemm: more than 128 rows and a shape");
   if (shape == 6)
     return vx::RunRowBlocks(x, packed, y, nullptr, m, k, n, false, true, vx::Stream(stream));
+  if (shape > 6)
+    return Prefill(x, packed, y, m, k, n, true, shape - 7, stream);
   return vx::RunGemm(x, packed, y, nullptr, m, k, n, false, true,
                      scratch != nullptr ? scratch->partials : nullptr,
                      scratch != nullptr ? scratch->partial_floats : 0, vx::Stream(stream),
@@ -332,7 +368,13 @@ int vx_q8_prefill_plan(size_t m, size_t k, size_t n, vx_scratch* scratch, int32_
   if (out4 == nullptr || m <= vx::kExactRows || k % 32 != 0 || k == 0 || n == 0)
     return vx::Fail(VX_BAD_ARG, "vx_q8_prefill_plan: bad arguments");
   const std::size_t floats = scratch != nullptr ? scratch->partial_floats : 0;
-  if (vx::UseRowBlocks(m, k, n, true)) {
+  if (vx::prefill::Use(m, k, n)) {
+    const vx::prefill::Shape shape = vx::prefill::ShapeOf(vx::prefill::PickShape(m, k, n));
+    out4[0] = 3;
+    out4[1] = shape.bm;
+    out4[2] = shape.bn;
+    out4[3] = 1;
+  } else if (vx::UseRowBlocks(m, k, n, true)) {
     out4[0] = 2;
     out4[1] = 64;
     out4[2] = static_cast<int32_t>(16 * (n > 4096 ? 2 : 1));  // columns per workgroup

@@ -1,0 +1,528 @@
+// Q8_0 (or bf16) panels x bfloat16 rows for more than 128 rows, the
+// reference's expansion of Q8_0 weights to bf16(f16 scale * q) with one
+// float32 sum over k (gemm.cpp:305-312, kernels/wmma_products.hip:94-112),
+// on gfx950's 32 x 32 x 16 bf16 matrix cores.
+//
+// The panels hold each lane's operand bytes together, so a wave loads its
+// columns' weights straight into registers, expands them there and multiplies
+// them with every row of the workgroup's tile: only the activations pass
+// through LDS. (With both operands in LDS a 64 x 64 wave tile reads 16 KB per
+// 16 MFMAs, as much as the LDS delivers in their time.) Four to eight waves
+// along n share a tile's rows; where a product has too few tiles for the
+// compute units, KG groups of waves take a run of k each and their sums meet
+// in LDS in group order, which needs no second launch. k advances 64 columns
+// (a panel pair) per step, with two steps' weights and activations in flight
+// and one barrier per step.
+//
+// A wave's 32-column tile is two panel groups of 16 rows: neighbours, or for
+// SwiGLU a gate group and its up group, whose sums then sit 16 lanes apart.
+//
+// What bounds them: up to about 200 tiles of few steps the launch, the first
+// loads and the sums' meeting (4 to 6 us), then about 0.85 us a step, whose
+// products take 0.45 us (128 x 256): the rest is the wait for the step's
+// barrier and first operands, which two more steps in flight shortened
+// (1.0 -> 0.88 us). Measured on MI355X against the tiled, split and
+// 64-row-block kernels these replaced (Q8_0, us): 310 x 1024 x 2560 17.1 ->
+// 7.9, 310 x 2048 x 1024 8.9 -> 7.4, 310 x 1024 x 8192 17.3 -> 12.1,
+// 310 x 4096 x 1024 14.0 -> 10.6, 617 x 2048 x 2560 22.6 -> 13.9, 617 x 6144 x
+// 2048 57 -> 28, 617 x 2048 x 12288 64 -> 36, 777 x 2048 x 12288 56 -> 41; bf16
+// 333 x 4096 x 1024 15.7 -> 10.7.
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <cstdint>
+#include <type_traits>
+
+#include "bf16x3.hpp"
+#include "common.hpp"
+#include "products.hpp"
+#include "q8.hpp"
+#include "q8_prefill.hpp"
+#include "q8_tile.hpp"
+
+namespace vx::prefill {
+namespace {
+
+using bf16x3::F32x16;
+using q8::AsBf16x8;
+
+constexpr int kDies = 8;
+
+struct Args {
+  const Bf16* x;
+  const std::uint8_t* w;
+  float* y;
+  Bf16* out;
+  int m, k, n;
+  int pairs, groups;
+  int m_tiles;
+  int tiles;
+  int pair_stride;  // panel groups from a column tile's first group to its second
+};
+
+/// Workgroup b runs on die b % 8: die d takes a contiguous range of tiles (a
+/// weight tile's row tiles first), so that its L2 serves their weights.
+__device__ inline int DieOrdered(int b, int blocks) {
+  const int per = blocks / kDies;
+  const int extra = blocks % kDies;
+  const int die = b % kDies;
+  return die * per + min(die, extra) + b / kDies;
+}
+
+/// LDS index of 16-byte chunk `chunk` (0..7) of 128-byte row `row`: the rows
+/// alternate between the halves of a 256-byte bank line, so the chunk swaps
+/// with row / 2.
+__device__ inline int Swizzled(int row, int chunk) {
+  return row * 8 + (chunk ^ ((row >> 1) & 7));
+}
+
+/// BM rows, FN 32-column tiles per wave, NW waves along n, KG groups of k,
+/// DW steps' weights in flight per wave.
+template<int BM, int FN, int NW, int KG, int DW>
+struct Tile {
+  static constexpr int kFn = FN;
+  static constexpr int kNw = NW;
+  static constexpr int kKg = KG;
+  static constexpr int kDw = DW;
+  // Operands a quarter step ahead where the registers allow (up to two waves
+  // per SIMD); with four waves per SIMD they cover each other's waits.
+  static constexpr bool kAhead = KG <= 2;
+  static constexpr int kBm = BM;
+  static constexpr int kFm = BM / 32;
+  static constexpr int kColumns = 32 * FN * NW;
+  static constexpr int kGroupThreads = NW * kWave;
+  static constexpr int kThreads = kGroupThreads * KG;
+  static constexpr int kPieces = BM * 8 / kGroupThreads;  // 16-byte x pieces per thread per step
+  static constexpr int kStageBytes = 2 * BM * 128;        // per group
+  // Four groups and more share the sums' meeting: each adds all groups' of
+  // its share of the values; of two the first adds the second's.
+  static constexpr bool kShared = KG >= 4;
+  static constexpr int kMeetBytes = (kShared ? KG : KG - 1) * BM * kColumns * 4;
+  static constexpr int kLds = KG * kStageBytes > kMeetBytes ? KG * kStageBytes : kMeetBytes;
+};
+
+template<class T, bool BF16, int OUT>
+__global__ __launch_bounds__(T::kThreads, T::kThreads / 256) void PrefillKernel(Args a) {
+  constexpr int FN = T::kFn;
+  constexpr int NW = T::kNw;
+  constexpr int KG = T::kKg;
+  constexpr int DW = BF16 ? 2 : T::kDw;  // bf16 panels take twice the registers
+  constexpr int kUnit = BF16 ? q8::kBf16UnitBytes : q8::kUnitBytes;
+  constexpr int kFm = T::kFm;
+  constexpr int kPieces = T::kPieces;
+  constexpr int kLoads = BF16 ? 4 : 2;  // 16-byte weight loads per column tile and step
+  // Vector instructions of a quarter step (expansion of 8 FN weights, about
+  // 25 each, and addresses) per product.
+  constexpr int kShare = ((BF16 ? 0 : 22) * FN + 8) / (kFm * FN) + 1;
+  __shared__ __align__(16) unsigned char lds[T::kLds];
+
+  const int lane = static_cast<int>(threadIdx.x) % kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWave);
+  const int group = wave / NW;  // of k
+  const int wn = wave % NW;
+  const int tid = static_cast<int>(threadIdx.x) % T::kGroupThreads;
+  uint4* const stages = reinterpret_cast<uint4*>(lds) + group * (T::kStageBytes / 16);
+  const int tile = DieOrdered(static_cast<int>(blockIdx.x), a.tiles);
+  const int row0 = __builtin_amdgcn_readfirstlane((tile % a.m_tiles) * T::kBm);
+  const int n_tile = __builtin_amdgcn_readfirstlane(tile / a.m_tiles);
+  const int steps = (a.pairs + KG - 1) / KG;
+  const int first = group * steps;
+  const int last = min(a.pairs, first + steps);
+
+  const __amdgpu_buffer_rsrc_t x_buffer = q8::BufferOf(
+      a.x, 2U * static_cast<std::uint32_t>(a.m) * static_cast<std::uint32_t>(a.k));
+  // Column tile j: panel groups first_group(j) and pair_stride further on.
+  const int column_tile = n_tile * (FN * NW) + wn * FN;
+  const auto first_group = [&](int j) {
+    return OUT == static_cast<int>(Out::kSwiGlu) ? column_tile + j : 2 * (column_tile + j);
+  };
+  const std::uint32_t group_bytes = static_cast<std::uint32_t>(a.pairs) * kUnit;
+  __amdgpu_buffer_rsrc_t w_buffer[FN];
+#pragma unroll
+  for (int j = 0; j < FN; ++j) {
+    const int g = first_group(j);
+    const int left = max(0, min(a.groups - g, a.pair_stride + 1));
+    w_buffer[j] = q8::BufferOf(a.w + static_cast<std::size_t>(g) * group_bytes,
+                               static_cast<std::uint32_t>(left) * group_bytes);
+  }
+  const std::uint32_t w_lane =
+      static_cast<std::uint32_t>(lane % 32 / 16) * static_cast<std::uint32_t>(a.pair_stride) *
+          group_bytes +
+      16U * static_cast<std::uint32_t>(16 * (lane / 32) + lane % 16);
+  const std::uint32_t s_lane =
+      static_cast<std::uint32_t>(lane % 32 / 16) * static_cast<std::uint32_t>(a.pair_stride) *
+          group_bytes +
+      q8::kValueBytes + 4U * static_cast<std::uint32_t>(lane % 16);
+
+  struct Weights {
+    uint4 v[FN][kLoads];
+    std::uint32_t scales[FN];
+  };
+  // Load i of a tile: octets 2 i + lane / 32 of both blocks (Q8_0), or of
+  // block i / 2 octets 2 (i % 2) + lane / 32 (bf16).
+  const auto load_weights = [&](int step, Weights& w) {
+    const bool live = step < last;
+    const std::uint32_t unit = static_cast<std::uint32_t>(step) * kUnit;
+#pragma unroll
+    for (int j = 0; j < FN; ++j) {
+#pragma unroll
+      for (int i = 0; i < kLoads; ++i)
+        w.v[j][i] = q8::BufferLoad16(
+            w_buffer[j],
+            w_lane + unit + (BF16 ? 1024U * (i / 2) + 512U * (i % 2) : 512U * i), live);
+      if constexpr (!BF16)
+        w.scales[j] = q8::BufferLoad4(w_buffer[j], s_lane + unit, live);
+    }
+  };
+  const auto weights_of = [&](const Weights& w, int j, int block, int half) {
+    if constexpr (BF16)
+      return AsBf16x8(w.v[j][2 * block + half]);
+    const uint4& v = w.v[j][half];
+    const float scale = HalfValue(static_cast<std::uint16_t>(
+        block == 0 ? w.scales[j] & 0xFFFFU : w.scales[j] >> 16));
+    return AsBf16x8(block == 0 ? q8::Expand(v.x, v.y, scale) : q8::Expand(v.z, v.w, scale));
+  };
+  std::uint32_t x_at[kPieces];
+#pragma unroll
+  for (int i = 0; i < kPieces; ++i) {
+    const int piece = tid + T::kGroupThreads * i;
+    const int row = row0 + piece / 8;
+    x_at[i] = row < a.m ? 2U * static_cast<std::uint32_t>(row * a.k + 8 * (piece % 8))
+                        : q8::kPastBuffer;
+  }
+  const auto load_x = [&](int step, int i) {
+    const int column = 64 * step + 8 * ((tid + T::kGroupThreads * i) % 8);
+    return q8::BufferLoad16(x_buffer, x_at[i] + 128U * static_cast<std::uint32_t>(step),
+                            step < last && column < a.k && x_at[i] != q8::kPastBuffer);
+  };
+  const auto store_x = [&](int stage, int i, const uint4& v) {
+    const int piece = tid + T::kGroupThreads * i;
+    stages[stage * T::kBm * 8 + Swizzled(piece / 8, piece % 8)] = v;
+  };
+
+  F32x16 acc[kFm][FN];
+#pragma unroll
+  for (int i = 0; i < kFm; ++i)
+#pragma unroll
+    for (int j = 0; j < FN; ++j)
+#pragma unroll
+      for (int v = 0; v < 16; ++v)
+        acc[i][j][v] = 0.0F;
+  uint4 xs[2][kPieces];
+  Weights ws[DW];
+  // In the order they are waited for: a wait covers every older load.
+#pragma unroll
+  for (int i = 0; i < kPieces; ++i)
+    xs[0][i] = load_x(first, i);
+  load_weights(first, ws[0]);
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int i = 0; i < kPieces; ++i)
+    xs[1][i] = load_x(first + 1, i);
+#pragma unroll
+  for (int d = 1; d < DW; ++d) {
+    load_weights(first + d, ws[d]);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+#pragma unroll
+  for (int i = 0; i < kPieces; ++i) {
+    store_x(0, i, xs[0][i]);
+    xs[0][i] = load_x(first + 2, i);
+  }
+  const auto multiply = [&](const uint4(&x)[kFm], const q8::Bf16x8(&w)[FN]) {
+#pragma unroll
+    for (int j = 0; j < FN; ++j)
+#pragma unroll
+      for (int i = 0; i < kFm; ++i)
+        acc[i][j] = bf16x3::Mfma32(AsBf16x8(x[i]), w[j], acc[i][j]);
+  };
+  // The operands of a step's quarters (16 columns of k). Ahead: two at a
+  // time, each quarter read and expanded under the products of the one
+  // before it, the first under the last quarter of the step before (of the
+  // first step: zeros).
+  uint4 x_operand[2][kFm];
+  q8::Bf16x8 w_operand[2][FN];
+  if constexpr (T::kAhead) {
+#pragma unroll
+    for (int i = 0; i < kFm; ++i)
+      x_operand[1][i] = uint4{0U, 0U, 0U, 0U};
+#pragma unroll
+    for (int j = 0; j < FN; ++j)
+      w_operand[1][j] = AsBf16x8(uint4{0U, 0U, 0U, 0U});
+  }
+  __syncthreads();
+  for (int step0 = 0; step0 < steps; step0 += DW) {
+#pragma unroll
+    for (int d = 0; d < DW; ++d) {
+      if (step0 + d >= steps)
+        break;
+      const int step = first + step0 + d;
+      // LDS stage d % 2 and weight set d hold the step, the other register
+      // set of x the next one.
+      const int next = 1 - d % 2;
+      const uint4* const rows = stages + d % 2 * T::kBm * 8;
+#pragma unroll
+      for (int kk = 0; kk < 4; ++kk) {
+        const int now = T::kAhead ? kk % 2 : 0;
+#pragma unroll
+        for (int i = 0; i < kFm; ++i)
+          x_operand[now][i] = rows[Swizzled(32 * i + lane % 32, 2 * kk + lane / 32)];
+        if constexpr (T::kAhead)
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int j = 0; j < FN; ++j)
+          w_operand[now][j] = weights_of(ws[d], j, kk / 2, kk % 2);
+        const int ready = T::kAhead ? 1 - now : 0;
+        multiply(x_operand[ready], w_operand[ready]);
+#pragma unroll
+        for (int i = kk * kPieces / 4; i < (kk + 1) * kPieces / 4; ++i) {
+          store_x(next, i, xs[next][i]);
+          xs[next][i] = load_x(step + 3, i);
+        }
+        if (kk == 3)
+          load_weights(step + DW, ws[d]);
+        if constexpr (T::kAhead) {
+          // A share of the vector instructions behind every product.
+#pragma unroll
+          for (int q = 0; q < kFm * FN; ++q) {
+            __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x2, kShare, 0);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+      __syncthreads();
+    }
+  }
+  if constexpr (T::kAhead)
+    multiply(x_operand[1], w_operand[1]);
+  if constexpr (KG > 1)
+    __syncthreads();  // the stages have been read: the sums take their place
+
+  // The tile's output rows as one buffer: rows past m lie past it, and its
+  // range check drops them. Element e of column tile j: row 32 (e / 16) +
+  // 8 (e % 16 / 4) + 4 (lane / 32) + e % 4 of the tile, column lane % 32.
+  constexpr bool kPaired = OUT == static_cast<int>(Out::kSwiGlu);
+  constexpr std::uint32_t kBytes = OUT >= static_cast<int>(Out::kBf16) ? 2 : 4;
+  const std::uint32_t width = static_cast<std::uint32_t>(kPaired ? a.n / 2 : a.n);
+  const std::uint32_t row_bytes = width * kBytes;
+  const __amdgpu_buffer_rsrc_t out = q8::BufferOf(
+      (kBytes == 2 ? reinterpret_cast<unsigned char*>(a.out)
+                   : reinterpret_cast<unsigned char*>(a.y)) +
+          static_cast<std::size_t>(row0) * row_bytes,
+      static_cast<std::uint32_t>(min(T::kBm, a.m - row0)) * row_bytes);
+  const auto emit = [&](auto count, const float* value, int e0, int j) {
+    constexpr int kCount = decltype(count)::value;
+    const std::uint32_t column = static_cast<std::uint32_t>(
+        kPaired ? 16 * (column_tile + j) + lane % 16 : 32 * (column_tile + j) + lane % 32);
+    const bool writes = column < width && (!kPaired || lane % 32 < 16);
+    int offset[kCount];
+#pragma unroll
+    for (int e = 0; e < kCount; ++e) {
+      const int at = e0 + e;
+      const int row = 32 * (at / 16) + 8 * (at % 16 / 4) + 4 * (lane / 32) + at % 4;
+      offset[e] = static_cast<int>(
+          writes ? static_cast<std::uint32_t>(row) * row_bytes + kBytes * column
+                 : q8::kPastBuffer);
+    }
+    if constexpr (kPaired) {
+#pragma unroll
+      for (int e = 0; e < kCount; ++e) {
+        // Lanes 0-15 of each 32 hold the gate, the lane 16 on the up.
+        const float gate = value[e];
+        const auto swapped = __builtin_amdgcn_permlane16_swap(
+            __float_as_uint(gate), __float_as_uint(gate), false, false);
+        const float up = __uint_as_float(swapped[1]);
+        __builtin_amdgcn_raw_buffer_store_b16(
+            q8::Bf16Fast(gate / (1.0F + expf(-gate)) * up), out, offset[e], 0, 0);
+      }
+    } else if constexpr (OUT == static_cast<int>(Out::kBf16)) {
+#pragma unroll
+      for (int e = 0; e < kCount; ++e)
+        __builtin_amdgcn_raw_buffer_store_b16(q8::Bf16Fast(value[e]), out, offset[e], 0, 0);
+    } else {
+      float prior[kCount];
+#pragma unroll
+      for (int e = 0; e < kCount; ++e)
+        prior[e] = OUT == static_cast<int>(Out::kAccumulate)
+                       ? __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
+                                                       out, offset[e], 0, 0))
+                       : 0.0F;
+#pragma unroll
+      for (int e = 0; e < kCount; ++e) {
+        const float sum =
+            OUT == static_cast<int>(Out::kAccumulate) ? prior[e] + value[e] : value[e];
+        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(std::uint32_t, sum), out,
+                                              offset[e], 0, 0);
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);  // one tile's values at a time
+  };
+  constexpr int kValues = kFm * FN * 16;
+  float* const sums = reinterpret_cast<float*>(lds);  // [groups][values][group threads]
+  const auto put = [&](int slot) {
+#pragma unroll
+    for (int i = 0; i < kFm; ++i)
+#pragma unroll
+      for (int j = 0; j < FN; ++j)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+          const float element = acc[i][j][v];
+          sums[(slot * kValues + (i * FN + j) * 16 + v) * T::kGroupThreads + tid] = element;
+        }
+  };
+  if constexpr (T::kShared) {
+    static_assert(FN == 1, "a share lies within one column tile");
+    constexpr int kShare = kValues / KG;
+    put(group);
+    __syncthreads();
+    float value[kShare];
+#pragma unroll
+    for (int e = 0; e < kShare; ++e)
+      value[e] = sums[(group * kShare + e) * T::kGroupThreads + tid];
+#pragma unroll
+    for (int g = 1; g < KG; ++g)
+#pragma unroll
+      for (int e = 0; e < kShare; ++e)
+        value[e] += sums[(g * kValues + group * kShare + e) * T::kGroupThreads + tid];
+    emit(std::integral_constant<int, kShare>{}, value, group * kShare, 0);
+    return;
+  }
+  if constexpr (KG == 2) {
+    if (group == 1)
+      put(0);
+    __syncthreads();
+    if (group == 1)
+      return;
+  }
+#pragma unroll
+  for (int i = 0; i < kFm; ++i)
+#pragma unroll
+    for (int j = 0; j < FN; ++j) {
+      float value[16];
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        value[v] = acc[i][j][v];
+        if constexpr (KG == 2)
+          value[v] += sums[((i * FN + j) * 16 + v) * T::kGroupThreads + tid];
+      }
+      emit(std::integral_constant<int, 16>{}, value, 16 * i, j);
+    }
+}
+
+template<class T>
+void Launch(const Product& p, Args a, hipStream_t stream) {
+  a.m_tiles = static_cast<int>((p.m + T::kBm - 1) / T::kBm);
+  a.tiles = a.m_tiles * static_cast<int>((p.n + T::kColumns - 1) / T::kColumns);
+  const auto launch = [&](auto kernel) { kernel<<<a.tiles, T::kThreads, 0, stream>>>(a); };
+  if (p.bf16) {
+    switch (p.kind) {
+      case Out::kStore: launch(PrefillKernel<T, true, 0>); break;
+      case Out::kAccumulate: launch(PrefillKernel<T, true, 1>); break;
+      case Out::kBf16: launch(PrefillKernel<T, true, 2>); break;
+      case Out::kSwiGlu: launch(PrefillKernel<T, true, 3>); break;
+    }
+  } else {
+    switch (p.kind) {
+      case Out::kStore: launch(PrefillKernel<T, false, 0>); break;
+      case Out::kAccumulate: launch(PrefillKernel<T, false, 1>); break;
+      case Out::kBf16: launch(PrefillKernel<T, false, 2>); break;
+      case Out::kSwiGlu: launch(PrefillKernel<T, false, 3>); break;
+    }
+  }
+}
+
+}  // namespace
+
+namespace {
+
+/// A shape and its model: a workgroup's time apart from its steps and per
+/// step (64 columns of k) in microseconds, one workgroup per compute unit
+/// (measured on MI355X over m 129..777, k 1024..6144, n 1024..12288; within
+/// a fifth of every time measured there but for grids that fill every
+/// compute unit, which take up to a third longer, all shapes alike).
+struct Model {
+  Shape shape;
+  double fixed, step;
+};
+constexpr Model kModels[kShapes] = {
+    {{128, 256, 1}, 3.0, 0.85}, {{128, 128, 2}, 3.0, 0.87}, {{64, 128, 4}, 6.0, 1.0},
+    {{64, 64, 8}, 5.5, 1.03},   {{32, 64, 8}, 4.0, 0.85},   {{160, 256, 1}, 3.0, 0.97},
+    {{96, 256, 1}, 3.0, 0.75}};
+constexpr std::size_t kComputeUnits = 256;
+
+double Rounds(std::size_t m, std::size_t n, int bm, int bn) {
+  const std::size_t tiles = ((m + bm - 1) / bm) * ((n + bn - 1) / bn);
+  return static_cast<double>((tiles + kComputeUnits - 1) / kComputeUnits);
+}
+
+}  // namespace
+
+Shape ShapeOf(int shape) { return kModels[shape].shape; }
+
+bool Supported(std::size_t m, std::size_t k, std::size_t n) {
+  // The output tile, the activations and a column tile's panels as buffers
+  // of 32-bit offsets.
+  return n <= (std::size_t{1} << 20) && m * k <= (std::size_t{1} << 29) &&
+         q8::Bf16PackedBytes(n, k) < (std::size_t{1} << 31);
+}
+
+int PickShape(std::size_t m, std::size_t k, std::size_t n, double* microseconds) {
+  int best = 0;
+  double least = 0.0;
+  for (int i = 0; i < kShapes; ++i) {
+    const Model& model = kModels[i];
+    const std::size_t groups = static_cast<std::size_t>(model.shape.groups);
+    const double steps = static_cast<double>((q8::Pairs(k) + groups - 1) / groups);
+    const double time = Rounds(m, n, model.shape.bm, model.shape.bn) *
+                        (model.fixed + steps * model.step);
+    if (i == 0 || time < least) {
+      best = i;
+      least = time;
+    }
+  }
+  if (microseconds != nullptr)
+    *microseconds = least;
+  return best;
+}
+
+bool Use(std::size_t m, std::size_t k, std::size_t n) {
+  // Up to 512 rows over 6144 columns of k and more stay on the kernels whose
+  // split over k uses a scratch: that split is part of what the static
+  // scratch entry promises at those sizes (300 x 6144 x 2048 takes 31.6 us
+  // there, 20.7 us here; the stacks, which use no scratch, come here).
+  if (m <= kExactRows || !Supported(m, k, n) || (k >= 6144 && m <= 512))
+    return false;
+  // Against the 256 x 256 tiles of q8_gemm.hip by the same model (3 us, 1.5
+  // a step).
+  double here = 0.0;
+  PickShape(m, k, n, &here);
+  return !UseGemm(m, n) ||
+         here <= Rounds(m, n, 256, 256) * (3.0 + 1.5 * static_cast<double>(q8::Pairs(k)));
+}
+
+int Run(const Product& p, hipStream_t stream, int shape) {
+  Args a{};
+  a.x = p.x;
+  a.w = static_cast<const std::uint8_t*>(p.w);
+  a.y = p.y;
+  a.out = p.out;
+  a.m = static_cast<int>(p.m);
+  a.k = static_cast<int>(p.k);
+  a.n = static_cast<int>(p.n);
+  a.pairs = static_cast<int>(q8::Pairs(p.k));
+  a.groups = static_cast<int>(q8::Groups(p.n));
+  a.pair_stride = p.kind == Out::kSwiGlu ? a.groups / 2 : 1;
+  switch (shape >= 0 ? shape : PickShape(p.m, p.k, p.n)) {
+    case 0: Launch<Tile<128, 2, 4, 1, 4>>(p, a, stream); break;
+    case 1: Launch<Tile<128, 1, 4, 2, 4>>(p, a, stream); break;
+    case 2: Launch<Tile<64, 1, 4, 4, 2>>(p, a, stream); break;
+    case 3: Launch<Tile<64, 1, 2, 8, 2>>(p, a, stream); break;
+    case 4: Launch<Tile<32, 1, 2, 8, 2>>(p, a, stream); break;
+    case 5: Launch<Tile<160, 2, 4, 1, 4>>(p, a, stream); break;
+    default: Launch<Tile<96, 2, 4, 1, 4>>(p, a, stream); break;
+  }
+  return LaunchStatus("prefill product");
+}
+
+}  // namespace vx::prefill

@@ -10,7 +10,9 @@
 // workgroups score, so that a one-row decode step over a long cache still
 // spreads over the compute units; a second launch merges the chunks'
 // softmax statistics in chunk order. More rows take the reference's launch
-// sequence.
+// sequence; past 128 rows its products are q8_prefill.hip's, with SwiGLU in
+// gate_up's epilogue (310 rows through the 12-layer encoder 1087 -> 724 us,
+// 617 through two base-LM layers 452 -> 304 us on MI355X).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -24,6 +26,7 @@
 #include "dit_kernels.hpp"
 #include "products.hpp"
 #include "q8.hpp"
+#include "q8_prefill.hpp"
 #include "q8_tile.hpp"
 #include "tile_attention.hpp"
 #include "voxcpm_amd.h"
@@ -752,6 +755,10 @@ struct vx_stack {
   /// Bf16Gemm::Linear (gemm.cpp:259-313): y[m][n] (+)= x W^T.
   int Linear(const Bf16* x, const void* w, float* y, std::size_t m, std::size_t k,
              std::size_t n, bool accumulate, hipStream_t stream) {
+    if (m > vx::kExactRows && vx::prefill::Supported(m, k, n))
+      return Prefill(x, w, y, nullptr, m, k, n,
+                     accumulate ? vx::prefill::Out::kAccumulate : vx::prefill::Out::kStore,
+                     stream);
     if (m > vx::kExactRows) {
       VX_TRY(Grow(&product_partials, &product_partial_floats, 2 * m * n,
                   "vx_stack_forward: hipMalloc"));
@@ -763,6 +770,38 @@ struct vx_stack {
     const vx::ProductPlan plan = vx::PlanSkinny(m, k, n, 0, 0, 0, 0, 0, Kind());
     return vx::RunSkinny(x, w, y, nullptr, m, k, n, accumulate, plan, nullptr, nullptr,
                          stream, Kind());
+  }
+
+  int Prefill(const Bf16* x, const void* w, float* y, Bf16* out, std::size_t m, std::size_t k,
+              std::size_t n, vx::prefill::Out kind, hipStream_t stream) const {
+    vx::prefill::Product p;
+    p.x = x;
+    p.w = w;
+    p.bf16 = Kind() != vx::q8::Weights::kQ8;
+    p.m = m;
+    p.k = k;
+    p.n = n;
+    p.kind = kind;
+    p.y = y;
+    p.out = out;
+    return vx::prefill::Run(p, stream);
+  }
+
+  /// bf16(silu(gate) up) of the rows in `bf16`, left at *act: in gate_up's
+  /// epilogue beyond the exact rows (the buffer of its sums then holds the
+  /// result), else by a launch of its own, back into `bf16`.
+  int GateUp(const void* w, const Bf16** act, std::size_t m, hipStream_t stream) {
+    const std::size_t n = 2 * shape.ffn;
+    if (m > vx::kExactRows && vx::prefill::Supported(m, shape.hidden, n)) {
+      Bf16* const out = reinterpret_cast<Bf16*>(gate_up);
+      *act = out;
+      return Prefill(bf16, w, nullptr, out, m, shape.hidden, n, vx::prefill::Out::kSwiGlu,
+                     stream);
+    }
+    VX_TRY(Linear(bf16, w, gate_up, m, shape.hidden, n, false, stream));
+    vx::kernels::SwiGlu(gate_up, bf16, m, shape.ffn, stream);
+    *act = bf16;
+    return VX_OK;
   }
 
   int Resolved(std::size_t rows) const {
@@ -861,9 +900,9 @@ struct vx_stack {
       VX_TRY(Linear(bf16, layer.o, f.hidden, rows, q_width, width, true, stream));
       vx::kernels::RmsNorm(f.hidden, layer.post_norm, bf16, nullptr, rows, width, shape.eps,
                            stream);
-      VX_TRY(Linear(bf16, layer.gate_up, gate_up, rows, width, 2 * ffn, false, stream));
-      vx::kernels::SwiGlu(gate_up, bf16, rows, ffn, stream);
-      VX_TRY(Linear(bf16, layer.down, f.hidden, rows, ffn, width, true, stream));
+      const Bf16* act = nullptr;
+      VX_TRY(GateUp(layer.gate_up, &act, rows, stream));
+      VX_TRY(Linear(act, layer.down, f.hidden, rows, ffn, width, true, stream));
     }
     vx::kernels::RmsNorm(f.hidden, weights.norm, bf16, f.output, rows, width, shape.eps,
                          stream);
