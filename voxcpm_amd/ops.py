@@ -28,9 +28,18 @@ def _ptr(tensor: torch.Tensor | None) -> ctypes.c_void_p | None:
     return None if tensor is None else ctypes.c_void_p(tensor.data_ptr())
 
 
+# torch's current stream of a device as its bare handle. Making the Stream
+# object that torch.cuda.current_stream() returns took 2.5 us of an 8.2 us
+# one-row product call; the handle takes 0.07 us.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream(stream: torch.cuda.Stream | None) -> ctypes.c_void_p:
-    stream = stream or torch.cuda.current_stream()
-    return ctypes.c_void_p(stream.cuda_stream)
+    if stream:
+        return ctypes.c_void_p(stream.cuda_stream)
+    if _raw_stream is None:  # a torch without it
+        return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    return ctypes.c_void_p(_raw_stream(torch.cuda.current_device()))
 
 
 def _device(device) -> torch.device:
