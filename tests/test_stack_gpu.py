@@ -357,3 +357,42 @@ def test_stack_decode_replays_past_4096(vx, oracle, cuda, stream):
         ref_h, ref_out = run.cpu.forward(h, at, at, 1, 1, past, True, run.k_cpu, run.v_cpu)
         check_close(output.cpu().numpy(), ref_out, f"replay past {past} output")
         check_close(hidden.cpu().numpy(), ref_h, f"replay past {past} hidden")
+
+
+@pytest.mark.parametrize("heads,kv_heads,head_dim", [(16, 2, 128), (4, 4, 64)])
+@pytest.mark.parametrize("rows,past", [(150, 40), (129, 700)])
+def test_tile_attention_past_float16(vx, cuda, stream, heads, kv_heads, head_dim, rows, past):
+    """What the matrix-core attention's float16 pairs cannot hold: rows before
+    a key are untouched by whatever it holds (a NaN value, an infinite one, a
+    NaN key: the same bits as without it), the rows that count it get float32's result; and
+    operands past 65504 give what their scaled copies give (powers of two:
+    exact, the bound one bf16 ulp of the sum)."""
+    rng = synth.Rng(53, rows + past)
+    keys = past + rows
+    q = f32(1.5 * rng.normal(rows * heads * head_dim).reshape(rows, heads, head_dim))
+    kc = f32(rng.normal(kv_heads * keys * head_dim).reshape(kv_heads, keys, head_dim))
+    vc = f32(rng.normal(kv_heads * keys * head_dim).reshape(kv_heads, keys, head_dim))
+
+    def attend(q, k, v):
+        got = vx.split_attention(dev(f32(q), cuda), dev(f32(k), cuda), dev(f32(v), cuda), rows,
+                                 rows, past, True, heads, kv_heads)
+        torch.cuda.synchronize()
+        return synth.bf16_values(host_bf16(got)).reshape(rows, heads, head_dim)
+
+    plain = attend(q, kc, vc)
+    bound = 2.0**-7 * np.abs(plain) + 2.0**-20 * np.max(np.abs(vc))
+    last = rows - 3  # the row whose key and value are spoilt
+    for value, cache in ((np.nan, "v"), (np.inf, "v"), (np.nan, "k")):
+        spoilt = {"k": kc.copy(), "v": vc.copy()}
+        spoilt[cache][:, past + last, 5] = value
+        got = attend(q, spoilt["k"], spoilt["v"])
+        assert np.all(np.abs(got[:last] - plain[:last]) <= bound[:last]), (value, cache)
+        if cache == "k":
+            assert np.all(np.isnan(got[last:]))
+        else:
+            assert not np.any(np.isfinite(got[last:, :, 5]))
+            rest = np.delete(np.arange(head_dim), 5)
+            assert np.all(np.abs(got[last:][:, :, rest] - plain[last:][:, :, rest]) <=
+                          bound[last:][:, :, rest])
+    assert np.all(np.abs(attend(q, kc, vc * 2.0**20) * 2.0**-20 - plain) <= bound)
+    assert np.all(np.abs(attend(q * 2.0**-20, kc * 2.0**20, vc) - plain) <= bound)

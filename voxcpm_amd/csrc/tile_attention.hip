@@ -1,7 +1,7 @@
 // Attention of many rows over a float32 key/value cache (a prompt's prefill,
 // a prompt's patches through the local encoder): the reference's Attention
-// (kernels/generator_kernels.hip:160-241) on gfx950's bf16 matrix cores with
-// float32 operands split into three bf16 terms (bf16x3.hpp).
+// (kernels/generator_kernels.hip:160-241) on gfx950's f16 matrix cores with
+// float32 operands split into two float16 terms (f16x2.hpp).
 //
 // A workgroup of four waves takes 128 queries of one KV head -- a query is a
 // (row, query head of the group) pair, so a group's heads share every key
@@ -16,8 +16,20 @@
 // per query (running maximum and sum, float32).
 //
 // Short of workgroups, the keys are cut into chunks that separate workgroups
-// take; each leaves its maximum, sum and unnormalised values, and a second
-// launch merges a row's chunks in chunk order.
+// take, as many as run at once; each leaves its maximum, sum and
+// unnormalised values, and a second launch merges a row's chunks in chunk
+// order.
+//
+// A workgroup that met a value past float16's range, or whose sums came out
+// NaN or infinite (a masked key's value weighs 0, which a NaN survives),
+// starts over key by key in float32.
+//
+// Measured on MI355X: 300 rows of 16 heads over 1800 keys 390 us on the
+// float32 split kernel, 55 us from three bfloat16 terms (twice the products,
+// and 570 workgroups in two rounds), 38 us now, of which the merge 6.8 us. A
+// step of one workgroup alone takes 2.1 us, of which the products are 0.65:
+// one wave per SIMD runs scores, softmax and values one after the other, and
+// registers (256 of 256) leave two workgroups per compute unit.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -26,6 +38,7 @@
 
 #include "bf16x3.hpp"
 #include "common.hpp"
+#include "f16x2.hpp"
 #include "q8.hpp"
 #include "q8_tile.hpp"
 #include "tile_attention.hpp"
@@ -34,7 +47,7 @@ namespace vx {
 namespace {
 
 using bf16x3::F32x16;
-using bf16x3::Octet;
+using f16x2::Octet;
 
 constexpr int kThreads = 256;
 constexpr int kWaves = kThreads / kWave;
@@ -42,9 +55,11 @@ constexpr int kQueries = 32 * kWaves;  // per workgroup
 constexpr int kKeys = 32;              // per step
 // Fewest keys of a chunk (the caller's partials hold a chunk per 64 keys).
 constexpr int kLeastChunk = 128;
-// Workgroups that chunks are cut for: two per compute unit.
-constexpr int kTargetWorkgroups = 512;
-// A transposed value row in LDS: 32 bf16 keys and 16 bytes of padding, so
+// Workgroups that run at once, two per compute unit: chunks are cut for as
+// many and no more (570 took two rounds; 300 rows over 1800 keys: 384 and 256
+// workgroups 44 and 43 us against 43, 700 over 2300 80 and 89 against 71 us).
+constexpr std::size_t kTargetWorkgroups = 512;
+// A transposed value row in LDS: 32 f16 keys and 16 bytes of padding, so
 // that the 16-byte reads of eight consecutive rows fall on distinct banks.
 constexpr int kValueRow = 80;
 
@@ -62,6 +77,7 @@ struct TileArgs {
   int heads;
   int kv_heads;
   int capacity;
+  int sequences;
   int blocks;  // query blocks per (sequence, KV head)
   int chunk;   // keys per chunk
   int splits;  // chunks
@@ -87,31 +103,52 @@ __device__ inline float MaxXor32(float x) {
   return fmaxf(__uint_as_float(swapped[0]), __uint_as_float(swapped[1]));
 }
 
+/// Most keys of a query of query block `block`.
+__device__ inline int BlockKeys(const TileArgs& a, int block, int queries, int group) {
+  const int last = min((block + 1) * kQueries, queries) - 1;
+  return a.past + (a.causal != 0 ? last / group + 1 : a.rows_per_sequence);
+}
+
 template<int D>
 __global__ __launch_bounds__(kThreads, 2) void TileAttentionKernel(TileArgs a) {
   constexpr int kChunks = D / 8;    // 16-byte chunks of a key row's plane
+  // A key row in LDS: a chunk of padding puts the 16-byte reads of 16
+  // consecutive keys on distinct banks.
+  constexpr int kKeyRow = kChunks + 1;
   constexpr int kSteps = D / 16;    // MFMA steps of a score
   constexpr int kTiles = D / 32;    // 32-dimension tiles of the output
   constexpr int kKeyLoads = kKeys * kChunks / kThreads;  // 8-value pieces per thread
   constexpr int kValueThreads = kKeys / 4 * (D / 4);     // 4 x 4 pieces
-  __shared__ uint4 key_planes[3][kKeys * kChunks];
-  __shared__ __align__(16) unsigned char value_planes[3][D * kValueRow];
+  __shared__ uint4 key_planes[2][kKeys * kKeyRow];
+  __shared__ __align__(16) unsigned char value_planes[2][D * kValueRow];
+  __shared__ int restart;
 
   const int tid = static_cast<int>(threadIdx.x);
   const int lane = tid % kWave;
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
   const int column = lane % 32;
   const int half = lane / 32;
-  int block = static_cast<int>(blockIdx.x);
-  const int split = block % a.splits;
-  block /= a.splits;
-  // The last query blocks, with the most keys of a causal call, first.
-  const int query_block = a.blocks - 1 - block % a.blocks;
-  block /= a.blocks;
-  const int g = block % a.kv_heads;
-  const int sequence = block / a.kv_heads;
+  // The grid holds the runs that have keys: sequences and KV heads fastest,
+  // then a query block's chunks, the last query blocks, with the most keys
+  // of a causal call, first.
+  const int heads = a.kv_heads * a.sequences;
+  const int g = static_cast<int>(blockIdx.x) % heads % a.kv_heads;
+  const int sequence = static_cast<int>(blockIdx.x) % heads / a.kv_heads;
   const int group = a.heads / a.kv_heads;
   const int queries = a.rows_per_sequence * group;
+  int split = static_cast<int>(blockIdx.x) / heads;
+  int query_block = a.blocks - 1;
+  if (a.splits == 1) {
+    query_block -= split;
+    split = 0;
+  } else {
+    for (;; --query_block) {
+      const int runs = (BlockKeys(a, query_block, queries, group) + a.chunk - 1) / a.chunk;
+      if (split < runs)
+        break;
+      split -= runs;
+    }
+  }
 
   // Keys of query `index` (queries past the last count none).
   const auto keys_of = [&](int index) {
@@ -119,11 +156,9 @@ __global__ __launch_bounds__(kThreads, 2) void TileAttentionKernel(TileArgs a) {
                             : a.past + (a.causal != 0 ? index / group + 1 : a.rows_per_sequence);
   };
   const int first_query = query_block * kQueries;
-  const int block_keys = keys_of(min(first_query + kQueries, queries) - 1);
   const int key_begin = split * a.chunk;
-  const int key_end = min(key_begin + a.chunk, block_keys);
-  if (key_begin >= key_end)
-    return;
+  const int key_end =
+      min(key_begin + a.chunk, BlockKeys(a, query_block, queries, group));
   const int wave_query = first_query + 32 * wave;
   const int wave_keys =
       wave_query < queries ? keys_of(min(wave_query + 32, queries) - 1) : 0;
@@ -131,9 +166,12 @@ __global__ __launch_bounds__(kThreads, 2) void TileAttentionKernel(TileArgs a) {
   const int my_keys = keys_of(query);
   // Steps whose keys every query of the wave counts need no mask.
   const int whole_keys = wave_query + 32 <= queries ? keys_of(wave_query) : 0;
-  const int local = min(query, queries - 1);
-  const int row = sequence * a.rows_per_sequence + local / group;
-  const int head = g * group + local % group;
+  // (row, head) of query `index`, row-major over [rows][heads] (queries past
+  // the last take its).
+  const auto place = [&](int index) {
+    const int local = min(index, queries - 1);
+    return (sequence * a.rows_per_sequence + local / group) * a.heads + g * group + local % group;
+  };
 
   // The caches up to the run's end as buffers: loads past it read zero (the
   // cache beyond what was written may hold anything).
@@ -169,18 +207,17 @@ __global__ __launch_bounds__(kThreads, 2) void TileAttentionKernel(TileArgs a) {
                                                                   4 * dim_quad));
     }
   };
+  float most = 0.0F;  // the largest magnitude this thread has split
   const auto store = [&]() {
 #pragma unroll
     for (int i = 0; i < kKeyLoads; ++i) {
       const int piece = tid + kThreads * i;
       const int key = piece / kChunks;
-      const Octet o = bf16x3::Split(key_next[i][0], key_next[i][1]);
-      // Chunk c of key s at c ^ (s % 8): the 16-byte reads of eight
-      // consecutive keys fall on distinct banks.
-      const int at = key * kChunks + ((piece % kChunks) ^ (key % 8));
+      const Octet o = f16x2::Split(key_next[i][0], key_next[i][1]);
+      most = f16x2::Largest(f16x2::Largest(most, key_next[i][0]), key_next[i][1]);
+      const int at = key * kKeyRow + piece % kChunks;
       key_planes[0][at] = o.h;
-      key_planes[1][at] = o.m;
-      key_planes[2][at] = o.l;
+      key_planes[1][at] = o.l;
     }
     if (kValueThreads == kThreads || tid < kValueThreads) {
       const float4(&v)[4] = value_next;
@@ -193,27 +230,30 @@ __global__ __launch_bounds__(kThreads, 2) void TileAttentionKernel(TileArgs a) {
       const int slot = (value_quad / 4) * 32 + (value_quad % 2) * 16 + ((value_quad / 2) % 2) * 8;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const bf16x3::Pair p0 = bf16x3::Split(rows[e][0], rows[e][1]);
-        const bf16x3::Pair p1 = bf16x3::Split(rows[e][2], rows[e][3]);
+        const f16x2::Pair p0 = f16x2::Split(rows[e][0], rows[e][1]);
+        const f16x2::Pair p1 = f16x2::Split(rows[e][2], rows[e][3]);
+        most = f16x2::Largest(most, v[e]);
         const int at = (4 * dim_quad + e) * kValueRow + slot;
         *reinterpret_cast<uint2*>(&value_planes[0][at]) = uint2{p0.h, p1.h};
-        *reinterpret_cast<uint2*>(&value_planes[1][at]) = uint2{p0.m, p1.m};
-        *reinterpret_cast<uint2*>(&value_planes[2][at]) = uint2{p0.l, p1.l};
+        *reinterpret_cast<uint2*>(&value_planes[1][at]) = uint2{p0.l, p1.l};
       }
     }
   };
 
+  if (tid == 0)
+    restart = 0;
   load(key_begin);
   Octet qs[kSteps];
   {
-    const float* source = a.q + (static_cast<std::size_t>(row) * a.heads + head) * D + 8 * half;
+    const float* source = a.q + static_cast<std::size_t>(place(query)) * D + 8 * half;
 #pragma unroll
     for (int s = 0; s < kSteps; ++s) {
       float4 x = reinterpret_cast<const float4*>(source + 16 * s)[0];
       float4 y = reinterpret_cast<const float4*>(source + 16 * s)[1];
       x = make_float4(x.x * a.scale, x.y * a.scale, x.z * a.scale, x.w * a.scale);
       y = make_float4(y.x * a.scale, y.y * a.scale, y.z * a.scale, y.w * a.scale);
-      qs[s] = bf16x3::Split(x, y);
+      qs[s] = f16x2::Split(x, y);
+      most = f16x2::Largest(f16x2::Largest(most, x), y);
     }
   }
 
@@ -230,25 +270,35 @@ __global__ __launch_bounds__(kThreads, 2) void TileAttentionKernel(TileArgs a) {
     __syncthreads();  // the step before has been read
     store();
     __syncthreads();
-    if (key0 + kKeys < key_end)
-      load(key0 + kKeys);
+    // Steps past the run's end load zeros.
+    load(key0 + kKeys);
     if (key0 >= wave_keys)
       continue;
 
-    F32x16 score;
+    F32x16 score;  // hh
+    F32x16 cross;  // hl + lh, 2048 times their value
 #pragma unroll
     for (int v = 0; v < 16; ++v)
-      score[v] = 0.0F;
+      score[v] = cross[v] = 0.0F;
+    const auto key_octet = [&](int s) {
+      const int at = column * kKeyRow + 2 * s + half;
+      return Octet{key_planes[0][at], key_planes[1][at]};
+    };
+    Octet ahead = key_octet(0);
 #pragma unroll
     for (int s = 0; s < kSteps; ++s) {
-      const int at = column * kChunks + ((2 * s + half) ^ (column % 8));
-      const Octet o{key_planes[0][at], key_planes[1][at], key_planes[2][at]};
-      score = bf16x3::Multiply(o, qs[s], score);
+      const Octet o = ahead;
+      if (s + 1 < kSteps)
+        ahead = key_octet(s + 1);
+      __builtin_amdgcn_sched_barrier(0);  // read before the products it waits for
+      cross = f16x2::Mfma32(o.l, qs[s].h, cross);
+      score = f16x2::Mfma32(o.h, qs[s].h, score);
+      cross = f16x2::Mfma32(o.h, qs[s].l, cross);
     }
     float p[16];
 #pragma unroll
     for (int v = 0; v < 16; ++v)
-      p[v] = score[v];
+      p[v] = __builtin_fmaf(cross[v], f16x2::kCross, score[v]);
     const bool masked = key0 + kKeys > whole_keys;
     if (masked) {
 #pragma unroll
@@ -279,18 +329,92 @@ __global__ __launch_bounds__(kThreads, 2) void TileAttentionKernel(TileArgs a) {
       p[v] = drop ? 0.0F : e;
       sum += p[v];
     }
+    Octet weights[2];
 #pragma unroll
-    for (int c = 0; c < 2; ++c) {
-      const Octet weights =
-          bf16x3::Split(make_float4(p[8 * c], p[8 * c + 1], p[8 * c + 2], p[8 * c + 3]),
-                        make_float4(p[8 * c + 4], p[8 * c + 5], p[8 * c + 6], p[8 * c + 7]));
+    for (int c = 0; c < 2; ++c)
+      weights[c] = f16x2::Split(make_float4(p[8 * c], p[8 * c + 1], p[8 * c + 2], p[8 * c + 3]),
+                                make_float4(p[8 * c + 4], p[8 * c + 5], p[8 * c + 6],
+                                            p[8 * c + 7]));
 #pragma unroll
-      for (int i = 0; i < kTiles; ++i) {
+    for (int i = 0; i < kTiles; ++i) {
+      F32x16 apart;  // the cross terms
+#pragma unroll
+      for (int v = 0; v < 16; ++v)
+        apart[v] = 0.0F;
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
         const int at = (32 * i + column) * kValueRow + 32 * c + 16 * half;
         const Octet o{*reinterpret_cast<const uint4*>(&value_planes[0][at]),
-                      *reinterpret_cast<const uint4*>(&value_planes[1][at]),
-                      *reinterpret_cast<const uint4*>(&value_planes[2][at])};
-        out[i] = bf16x3::Multiply(o, weights, out[i]);
+                      *reinterpret_cast<const uint4*>(&value_planes[1][at])};
+        apart = f16x2::Mfma32(o.l, weights[c].h, apart);
+        out[i] = f16x2::Mfma32(o.h, weights[c].h, out[i]);
+        apart = f16x2::Mfma32(o.h, weights[c].l, apart);
+      }
+#pragma unroll
+      for (int v = 0; v < 16; ++v)
+        out[i][v] = __builtin_fmaf(apart[v], f16x2::kCross, out[i][v]);
+    }
+  }
+
+  // 0, or NaN where a sum is NaN or infinite.
+  float check[4] = {0.0F * sum, 0.0F, 0.0F, 0.0F};
+#pragma unroll
+  for (int i = 0; i < kTiles; ++i)
+#pragma unroll
+    for (int v = 0; v < 16; ++v)
+      check[v % 4] = __builtin_fmaf(out[i][v], 0.0F, check[v % 4]);
+  if (f16x2::TooLarge(most) || check[0] + check[1] + (check[2] + check[3]) != 0.0F)
+    restart = 1;
+  __syncthreads();
+  // Located again rather than held in registers through the steps (a spilled
+  // one's reload waits for the loads in flight).
+  int last_query = query;
+  asm volatile("" : "+v"(last_query));
+  const std::size_t at = static_cast<std::size_t>(place(last_query));
+  if (restart != 0) {
+    // Key by key in float32: each half of the wave takes half the dimensions
+    // of a score, and its own of the values. Keys a query does not count are
+    // left out, whatever they hold.
+    maximum = -INFINITY;
+    sum = 0.0F;
+#pragma unroll
+    for (int i = 0; i < kTiles; ++i)
+#pragma unroll
+      for (int v = 0; v < 16; ++v)
+        out[i][v] = 0.0F;
+#pragma unroll 1
+    for (int key = key_begin; key < key_end; ++key) {
+      const float4* const k4 = reinterpret_cast<const float4*>(
+          a.k + cache + static_cast<std::size_t>(key) * D + half * (D / 2));
+      const float4* const q4 = reinterpret_cast<const float4*>(a.q + at * D + half * (D / 2));
+      float dot = 0.0F;
+#pragma unroll 1
+      for (int i = 0; i < D / 8; ++i) {
+        const float4 x = q4[i];
+        const float4 y = k4[i];
+        dot += x.x * a.scale * y.x + x.y * a.scale * y.y + x.z * a.scale * y.z +
+               x.w * a.scale * y.w;
+      }
+      dot = AddXor32(dot);
+      if (key >= my_keys)
+        continue;
+      const float top = fmaxf(maximum, dot);
+      const float decay = maximum == -INFINITY ? 0.0F : expf(maximum - top);
+      const float e = dot == -INFINITY ? 0.0F : expf(dot - top);
+      maximum = top;
+      sum = sum * decay + (half == 0 ? e : 0.0F);
+      const float* const value = a.v + cache + static_cast<std::size_t>(key) * D + 4 * half;
+#pragma unroll
+      for (int i = 0; i < kTiles; ++i) {
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+          const float4 x = *reinterpret_cast<const float4*>(value + 32 * i + 8 * b);
+          out[i][4 * b] = out[i][4 * b] * decay + e * x.x;
+          out[i][4 * b + 1] = out[i][4 * b + 1] * decay + e * x.y;
+          out[i][4 * b + 2] = out[i][4 * b + 2] * decay + e * x.z;
+          out[i][4 * b + 3] = out[i][4 * b + 3] * decay + e * x.w;
+        }
+        __builtin_amdgcn_sched_barrier(0);  // one tile's values in registers
       }
     }
   }
@@ -299,7 +423,6 @@ __global__ __launch_bounds__(kThreads, 2) void TileAttentionKernel(TileArgs a) {
   if (key_begin >= my_keys)
     return;  // past the last query, or before this chunk: nothing to leave
   // Element v of tile i: dimension 32 i + 8 (v / 4) + 4 half + v % 4.
-  const std::size_t at = static_cast<std::size_t>(row) * a.heads + head;
   if (a.splits == 1) {
     const float inverse = 1.0F / sum;
     Bf16* target = a.out + at * D + 4 * half;
@@ -328,14 +451,17 @@ __global__ __launch_bounds__(kThreads, 2) void TileAttentionKernel(TileArgs a) {
 
 /// The chunks of a (row, head) met in chunk order: M = max m_c, L = sum
 /// l_c exp(m_c - M), out = bf16(sum o_c exp(m_c - M) / L) over the row's
-/// chunks. D / 4 lanes per (row, head), four dimensions each.
+/// chunks. D / 4 lanes per (row, head), four dimensions each; lane c holds
+/// chunk c's statistics (chunks D / 4 apart in turn), and the first chunks'
+/// values are loaded beside them, so that they share a memory round trip (a
+/XX
 template<int D>
 __global__ __launch_bounds__(kThreads) void MergeChunksKernel(TileArgs a, int items) {
   constexpr int kLanes = D / 4;
-  constexpr int kBatch = 4;
+  constexpr int kBatch = 8;
   const int item = static_cast<int>(blockIdx.x) * (kThreads / kLanes) +
                    static_cast<int>(threadIdx.x) / kLanes;
-  if (item >= items)
+  if (item >= items)  // whole groups of lanes
     return;
   const int lane = static_cast<int>(threadIdx.x) % kLanes;
   const int local = (item / a.heads) % a.rows_per_sequence;
@@ -344,32 +470,46 @@ __global__ __launch_bounds__(kThreads) void MergeChunksKernel(TileArgs a, int it
   const std::size_t first = static_cast<std::size_t>(item) * a.splits;
   const float2* stats = reinterpret_cast<const float2*>(a.stats) + first;
   const float4* values = reinterpret_cast<const float4*>(a.values + first * D) + lane;
-  float top = -INFINITY;
-  for (int c = 0; c < chunks; ++c)
+  float4 v[kBatch];
+  const auto load = [&](int c0) {
+#pragma unroll
+    for (int b = 0; b < kBatch; ++b)
+      v[b] = values[static_cast<std::size_t>(min(c0 + b, chunks - 1)) * kLanes];
+  };
+  load(0);
+  const float2 mine = stats[min(lane, chunks - 1)];
+  float top = mine.x;
+  for (int c = lane + kLanes; c < chunks; c += kLanes)
     top = fmaxf(top, stats[c].x);
+#pragma unroll
+  for (int offset = kLanes / 2; offset > 0; offset /= 2)
+    top = fmaxf(top, __shfl_xor(top, offset, kLanes));
   float4 out = make_float4(0.0F, 0.0F, 0.0F, 0.0F);
   float sum = 0.0F;
-  for (int c0 = 0; c0 < chunks; c0 += kBatch) {
-    float4 v[kBatch];
-    float2 s[kBatch];
+  for (int base = 0; base < chunks; base += kLanes) {
+    const float2 s = base == 0 ? mine : stats[min(base + lane, chunks - 1)];
+    const float factor = base + lane < chunks ? expf(s.x - top) : 0.0F;
+    if (base + lane < chunks)
+      sum += s.y * factor;
+    const int count = min(kLanes, chunks - base);
+    for (int c0 = 0; c0 < count; c0 += kBatch) {
+      if (base + c0 > 0)
+        load(base + c0);
 #pragma unroll
-    for (int b = 0; b < kBatch; ++b) {
-      const int c = min(c0 + b, chunks - 1);
-      v[b] = values[static_cast<std::size_t>(c) * kLanes];
-      s[b] = stats[c];
-    }
-#pragma unroll
-    for (int b = 0; b < kBatch; ++b) {
-      if (c0 + b >= chunks)
-        break;
-      const float f = expf(s[b].x - top);
-      sum += s[b].y * f;
-      out.x += v[b].x * f;
-      out.y += v[b].y * f;
-      out.z += v[b].z * f;
-      out.w += v[b].w * f;
+      for (int b = 0; b < kBatch; ++b) {
+        const float f = __shfl(factor, c0 + b, kLanes);
+        if (c0 + b < count) {
+          out.x += v[b].x * f;
+          out.y += v[b].y * f;
+          out.z += v[b].z * f;
+          out.w += v[b].w * f;
+        }
+      }
     }
   }
+#pragma unroll
+  for (int offset = kLanes / 2; offset > 0; offset /= 2)
+    sum += __shfl_xor(sum, offset, kLanes);
   const float inverse = 1.0F / sum;
   *reinterpret_cast<uint2*>(a.out + static_cast<std::size_t>(item) * D + 4 * lane) =
       uint2{q8::PackBf16x2(out.x * inverse, out.y * inverse),
@@ -405,19 +545,26 @@ void TileAttention(const AttentionShape& s, const float* q, const float* k_cache
   const std::size_t sequences = s.rows / s.rows_per_sequence;
   const std::size_t queries = s.rows_per_sequence * group;
   const std::size_t blocks = (queries + kQueries - 1) / kQueries;
-  // Steps of all query blocks, and the chunk that cuts them into about
-  // kTargetWorkgroups runs.
+  const auto keys_of = [&](std::size_t block) {
+    const std::size_t last = std::min((block + 1) * kQueries, queries) - 1;
+    return s.past + (s.causal ? last / group + 1 : s.rows_per_sequence);
+  };
+  // The least chunk that cuts all query blocks' keys into at most
+  // kTargetWorkgroups runs (or leaves them whole).
+  const std::size_t heads = sequences * s.kv_heads;
   std::size_t steps = 0;
-  for (std::size_t b = 0; b < blocks; ++b) {
-    const std::size_t last = std::min((b + 1) * kQueries, queries) - 1;
-    const std::size_t keys = s.past + (s.causal ? last / group + 1 : s.rows_per_sequence);
-    steps += (keys + kKeys - 1) / kKeys;
-  }
-  steps *= sequences * s.kv_heads;
+  for (std::size_t b = 0; b < blocks; ++b)
+    steps += (keys_of(b) + kKeys - 1) / kKeys;
   const std::size_t most = s.past + s.rows_per_sequence;
-  const std::size_t chunk =
-      std::max<std::size_t>(kLeastChunk, (steps + kTargetWorkgroups - 1) / kTargetWorkgroups *
-                                             kKeys);
+  std::size_t chunk = std::max<std::size_t>(
+      kLeastChunk, (steps * heads + kTargetWorkgroups - 1) / kTargetWorkgroups * kKeys);
+  for (; chunk < most; chunk += kKeys) {
+    std::size_t runs = 0;
+    for (std::size_t b = 0; b < blocks; ++b)
+      runs += (keys_of(b) + chunk - 1) / chunk;
+    if (runs * heads <= kTargetWorkgroups)
+      break;
+  }
   const std::size_t splits = (most + chunk - 1) / chunk;
   TileArgs args{};
   args.q = q;
@@ -433,11 +580,14 @@ void TileAttention(const AttentionShape& s, const float* q, const float* k_cache
   args.heads = static_cast<int>(s.heads);
   args.kv_heads = static_cast<int>(s.kv_heads);
   args.capacity = static_cast<int>(s.capacity);
+  args.sequences = static_cast<int>(sequences);
   args.blocks = static_cast<int>(blocks);
   args.chunk = static_cast<int>(chunk);
   args.splits = static_cast<int>(splits);
   args.scale = 1.0F / std::sqrt(static_cast<float>(s.head_dim));
-  const std::size_t workgroups = sequences * s.kv_heads * blocks * splits;
+  std::size_t workgroups = 0;
+  for (std::size_t b = 0; b < blocks; ++b)
+    workgroups += splits == 1 ? heads : (keys_of(b) + chunk - 1) / chunk * heads;
   const std::size_t items = s.rows * s.heads;
   if (s.head_dim == 64)
     Launch<64>(args, workgroups, items, stream);
