@@ -236,20 +236,32 @@ def test_stack_bf16_weights(vx, oracle, cuda, stream):
     run.step(h, [5], [5], 1, 1, 5, True, "bf16 decode")
 
 
+# The VoxCPM2 layers give gate_up the wide tiles (128 x 256 at 400 rows, 128 x
+# 128 in two groups at 310), the small ones the tiles of four and eight groups.
+PROMPTS = {"gqa-hd64": STACKS["gqa-hd64"], "no-rope-hd128": STACKS["no-rope-hd128"],
+           "voxcpm2-encoder": synth.StackConfig(hidden=1024, ffn=4096, layers=1,
+                                                rope_factors=synth.VOXCPM2_SHORT_FACTORS),
+           "voxcpm2-lm": synth.StackConfig(layers=1, rope_factors=synth.VOXCPM2_SHORT_FACTORS)}
+
+
 @pytest.mark.parametrize("bf16_weights", [False, True])
-@pytest.mark.parametrize("rows", [129, 170])
-def test_stack_prompt_rows(vx, oracle, cuda, stream, rows, bf16_weights):
-    """A prompt past the exact rows: the panel-operand products, SwiGLU in
-    gate_up's epilogue and the residual adds in o's and down's, then a
+@pytest.mark.parametrize("name,rows", [("gqa-hd64", 129), ("gqa-hd64", 170),
+                                       ("no-rope-hd128", 150), ("voxcpm2-encoder", 310),
+                                       ("voxcpm2-lm", 400)])
+def test_stack_prompt_rows(vx, oracle, cuda, stream, name, rows, bf16_weights):
+    """A prompt past the exact rows: the norms, the rotary embedding and the
+    caches, SwiGLU and the residual adds in the products' epilogues, then a
     second prompt behind the first."""
-    config = STACKS["gqa-hd64"]
+    config = PROMPTS[name]
     run = Run(vx, oracle, cuda, config, 49, capacity=2 * rows, bf16_weights=bf16_weights)
     assert run.gpu.path(rows) == _lib.STACK_PATH_UNFUSED
     rng = synth.Rng(50, rows)
-    for past in (0, rows):
+    for past in (0, rows) if rows < 200 else (0,):
         h0 = rng.normal(rows * config.hidden).astype(np.float32).reshape(rows, config.hidden)
         at = past + np.arange(rows)
-        run.step(h0, at, at, rows, rows, past, True, f"prompt of {rows} behind {past}")
+        run.step(h0, at, at, rows, rows, past, True, f"{name} prompt of {rows} behind {past}")
+    check_close(run.k_gpu.cpu().numpy(), run.k_cpu, f"{name} key cache")
+    check_close(run.v_gpu.cpu().numpy(), run.v_cpu, f"{name} value cache")
 
 
 def test_stack_argument_errors(vx, cuda, stream):

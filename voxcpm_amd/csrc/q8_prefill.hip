@@ -15,7 +15,11 @@
 // and one barrier per step.
 //
 // A wave's 32-column tile is two panel groups of 16 rows: neighbours, or for
-// SwiGLU a gate group and its up group, whose sums then sit 16 lanes apart.
+// SwiGLU a gate group and its up group, for the rotary embedding a head's two
+// halves, whose sums then sit 16 lanes apart. A residual add's epilogue leaves
+// the next RMSNorm's operand and each row's sums of squares over 32 columns
+// each, which the next product's workgroups add up for their rows' factors: a
+// launch less per norm (3 to 5 us, 2 us of them back in the epilogues).
 //
 // What bounds them: up to about 200 tiles of few steps the launch, the first
 // loads and the sums' meeting (4 to 6 us), then about 0.85 us a step, whose
@@ -58,6 +62,8 @@ struct Args {
   int m_tiles;
   int tiles;
   int pair_stride;  // panel groups from a column tile's first group to its second
+  Norm norm;
+  Qkv qkv;
 };
 
 /// Workgroup b runs on die b % 8: die d takes a contiguous range of tiles (a
@@ -98,6 +104,12 @@ struct Tile {
   // its share of the values; of two the first adds the second's.
   static constexpr bool kShared = KG >= 4;
   static constexpr int kMeetBytes = (kShared ? KG : KG - 1) * BM * kColumns * 4;
+  // Threads that add a row's sums of squares.
+  static constexpr int kRowThreads = kThreads / BM >= 32   ? 32
+                                     : kThreads / BM >= 16 ? 16
+                                     : kThreads / BM >= 4  ? 4
+                                     : kThreads / BM >= 2  ? 2
+                                                           : 1;
   static constexpr int kLds = KG * kStageBytes > kMeetBytes ? KG * kStageBytes : kMeetBytes;
 };
 
@@ -114,7 +126,14 @@ __global__ __launch_bounds__(T::kThreads, T::kThreads / 256) void PrefillKernel(
   // Vector instructions of a quarter step (expansion of 8 FN weights, about
   // 25 each, and addresses) per product.
   constexpr int kShare = ((BF16 ? 0 : 22) * FN + 8) / (kFm * FN) + 1;
+  constexpr bool kNormed = OUT == static_cast<int>(Out::kSwiGlu) ||
+                           OUT == static_cast<int>(Out::kQkvCache);
+  constexpr bool kPaired = kNormed;  // a column tile's groups lie pair_stride apart
   __shared__ __align__(16) unsigned char lds[T::kLds];
+  __shared__ float row_scale[kNormed ? T::kBm : 1];
+  constexpr bool kQkv = OUT == static_cast<int>(Out::kQkvCache);
+  __shared__ std::int32_t row_position[kQkv ? T::kBm : 1];
+  __shared__ std::int32_t row_cache[kQkv ? T::kBm : 1];
 
   const int lane = static_cast<int>(threadIdx.x) % kWave;
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWave);
@@ -134,7 +153,12 @@ __global__ __launch_bounds__(T::kThreads, T::kThreads / 256) void PrefillKernel(
   // Column tile j: panel groups first_group(j) and pair_stride further on.
   const int column_tile = n_tile * (FN * NW) + wn * FN;
   const auto first_group = [&](int j) {
-    return OUT == static_cast<int>(Out::kSwiGlu) ? column_tile + j : 2 * (column_tile + j);
+    const int at = column_tile + j;
+    // A rotary tile: 16 dimensions of a head's first half and of its second.
+    return OUT == static_cast<int>(Out::kQkvCache)
+               ? at / a.pair_stride * 2 * a.pair_stride + at % a.pair_stride
+           : OUT == static_cast<int>(Out::kSwiGlu) ? at
+                                                   : 2 * at;
   };
   const std::uint32_t group_bytes = static_cast<std::uint32_t>(a.pairs) * kUnit;
   __amdgpu_buffer_rsrc_t w_buffer[FN];
@@ -229,6 +253,36 @@ __global__ __launch_bounds__(T::kThreads, T::kThreads / 256) void PrefillKernel(
     store_x(0, i, xs[0][i]);
     xs[0][i] = load_x(first + 2, i);
   }
+  if constexpr (kNormed) {
+    const int row = static_cast<int>(threadIdx.x) / T::kRowThreads;
+    const int part = static_cast<int>(threadIdx.x) % T::kRowThreads;
+    const int count = a.k / 32;
+    if (row < T::kBm) {  // whole groups of kRowThreads lanes
+      const int from = min(row0 + row, a.m - 1);
+      const float* const squares = a.norm.squares + static_cast<std::size_t>(from) * count;
+      float sum = 0.0F;
+      if (count % 4 == 0) {
+        const float4* const quads = reinterpret_cast<const float4*>(squares);
+#pragma unroll 8
+        for (int i = part; i < count / 4; i += T::kRowThreads)
+          sum += quads[i].x + quads[i].y + (quads[i].z + quads[i].w);
+      } else {
+        for (int i = part; i < count; i += T::kRowThreads)
+          sum += squares[i];
+      }
+      if constexpr (OUT == static_cast<int>(Out::kQkvCache)) {
+        if (part == 0) {
+          row_position[row] = a.qkv.positions[from];
+          row_cache[row] = a.qkv.cache_rows[from];
+        }
+      }
+#pragma unroll
+      for (int offset = T::kRowThreads / 2; offset > 0; offset /= 2)
+        sum += __shfl_xor(sum, offset, kWave);
+      if (part == 0)
+        row_scale[row] = rsqrtf(sum / static_cast<float>(a.k) + a.norm.eps);
+    }
+  }
   const auto multiply = [&](const uint4(&x)[kFm], const q8::Bf16x8(&w)[FN]) {
 #pragma unroll
     for (int j = 0; j < FN; ++j)
@@ -302,37 +356,103 @@ __global__ __launch_bounds__(T::kThreads, T::kThreads / 256) void PrefillKernel(
   // The tile's output rows as one buffer: rows past m lie past it, and its
   // range check drops them. Element e of column tile j: row 32 (e / 16) +
   // 8 (e % 16 / 4) + 4 (lane / 32) + e % 4 of the tile, column lane % 32.
-  constexpr bool kPaired = OUT == static_cast<int>(Out::kSwiGlu);
-  constexpr std::uint32_t kBytes = OUT >= static_cast<int>(Out::kBf16) ? 2 : 4;
-  const std::uint32_t width = static_cast<std::uint32_t>(kPaired ? a.n / 2 : a.n);
+  constexpr bool kSwiGlu = OUT == static_cast<int>(Out::kSwiGlu);
+  constexpr std::uint32_t kBytes = kSwiGlu || OUT == static_cast<int>(Out::kBf16) ? 2 : 4;
+  const std::uint32_t width = static_cast<std::uint32_t>(kSwiGlu ? a.n / 2 : a.n);
   const std::uint32_t row_bytes = width * kBytes;
   const __amdgpu_buffer_rsrc_t out = q8::BufferOf(
       (kBytes == 2 ? reinterpret_cast<unsigned char*>(a.out)
                    : reinterpret_cast<unsigned char*>(a.y)) +
           static_cast<std::size_t>(row0) * row_bytes,
       static_cast<std::uint32_t>(min(T::kBm, a.m - row0)) * row_bytes);
+  const auto row_of = [&](int at) {
+    return 32 * (at / 16) + 8 * (at % 16 / 4) + 4 * (lane / 32) + at % 4;
+  };
+  // This lane's and its pair's value of a paired tile: lanes 0-15 of each 32
+  // hold the first group, the lane 16 on the second.
+  const auto pair_of = [&](float value) {
+    const auto swapped = __builtin_amdgcn_permlane16_swap(
+        __float_as_uint(value), __float_as_uint(value), false, false);
+    return __uint_as_float(lane % 32 < 16 ? swapped[1] : swapped[0]);
+  };
+  // The rotary factors of elements e0 .. of column tile j: 1 and 0 where
+  // nothing rotates.
+  const auto load_rotary = [&](auto count, float* c, float* s, int e0, int j) {
+    constexpr int kCount = decltype(count)::value;
+    const int at = column_tile + j;
+    const bool rotates = a.qkv.rope != nullptr &&
+                         at / a.pair_stride < a.qkv.heads + a.qkv.kv_heads;
+#pragma unroll
+    for (int e = 0; e < kCount; ++e) {
+      c[e] = 1.0F;
+      s[e] = 0.0F;
+      if (rotates) {
+        const float* const table =
+            a.qkv.rope +
+            static_cast<std::size_t>(row_position[row_of(e0 + e)]) * a.qkv.head_dim +
+            16 * (at % a.pair_stride) + lane % 16;
+        c[e] = table[0];
+        s[e] = table[a.qkv.head_dim / 2];
+      }
+    }
+  };
+  const auto emit_qkv = [&](auto count, const float* value, const float* c, const float* s,
+                            int e0, int j) {
+    constexpr int kCount = decltype(count)::value;
+    const Qkv& o = a.qkv;
+    const int at = column_tile + j;
+    const int head = at / a.pair_stride;
+    if (32 * at >= a.n)
+      return;
+    const bool second = lane % 32 >= 16;
+    const int dim = 16 * (at % a.pair_stride) + lane % 16 + (second ? o.head_dim / 2 : 0);
+    const bool rotates = o.rope != nullptr && head < o.heads + o.kv_heads;
+    // Query heads lie [row][head], a cache's [row] of its head.
+    const bool query = head < o.heads;
+    float* const base =
+        query ? o.q + static_cast<std::size_t>(head) * o.head_dim + dim
+              : (head < o.heads + o.kv_heads ? o.k_cache : o.v_cache) +
+                    static_cast<std::size_t>((head - o.heads) % o.kv_heads) * o.capacity *
+                        o.head_dim +
+                    dim;
+    const std::size_t stride = static_cast<std::size_t>(query ? o.heads : 1) * o.head_dim;
+#pragma unroll
+    for (int e = 0; e < kCount; ++e) {
+      const int local = row_of(e0 + e);
+      const float own = value[e] * row_scale[local];
+      const float other = pair_of(own);
+      const float rotated = !rotates ? own
+                            : second ? own * c[e] + other * s[e]
+                                     : own * c[e] - other * s[e];
+      if (row0 + local < a.m)
+        base[static_cast<std::size_t>(query ? row0 + local : row_cache[local]) * stride] = rotated;
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
   const auto emit = [&](auto count, const float* value, int e0, int j) {
     constexpr int kCount = decltype(count)::value;
+    if constexpr (kQkv) {
+      float c[kCount], s[kCount];
+      load_rotary(count, c, s, e0, j);
+      emit_qkv(count, value, c, s, e0, j);
+      return;
+    }
     const std::uint32_t column = static_cast<std::uint32_t>(
-        kPaired ? 16 * (column_tile + j) + lane % 16 : 32 * (column_tile + j) + lane % 32);
-    const bool writes = column < width && (!kPaired || lane % 32 < 16);
+        kSwiGlu ? 16 * (column_tile + j) + lane % 16 : 32 * (column_tile + j) + lane % 32);
+    const bool writes = column < width && (!kSwiGlu || lane % 32 < 16);
     int offset[kCount];
 #pragma unroll
     for (int e = 0; e < kCount; ++e) {
-      const int at = e0 + e;
-      const int row = 32 * (at / 16) + 8 * (at % 16 / 4) + 4 * (lane / 32) + at % 4;
+      const int row = row_of(e0 + e);
       offset[e] = static_cast<int>(
           writes ? static_cast<std::uint32_t>(row) * row_bytes + kBytes * column
                  : q8::kPastBuffer);
     }
-    if constexpr (kPaired) {
+    if constexpr (kSwiGlu) {
 #pragma unroll
       for (int e = 0; e < kCount; ++e) {
-        // Lanes 0-15 of each 32 hold the gate, the lane 16 on the up.
-        const float gate = value[e];
-        const auto swapped = __builtin_amdgcn_permlane16_swap(
-            __float_as_uint(gate), __float_as_uint(gate), false, false);
-        const float up = __uint_as_float(swapped[1]);
+        const float gate = value[e] * row_scale[row_of(e0 + e)];
+        const float up = pair_of(gate);
         __builtin_amdgcn_raw_buffer_store_b16(
             q8::Bf16Fast(gate / (1.0F + expf(-gate)) * up), out, offset[e], 0, 0);
       }
@@ -354,6 +474,23 @@ __global__ __launch_bounds__(T::kThreads, T::kThreads / 256) void PrefillKernel(
             OUT == static_cast<int>(Out::kAccumulate) ? prior[e] + value[e] : value[e];
         __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(std::uint32_t, sum), out,
                                               offset[e], 0, 0);
+        prior[e] = sum;
+      }
+      if (OUT == static_cast<int>(Out::kAccumulate) && a.norm.scaled != nullptr) {
+        // The next norm's operand and this column tile's sums of squares.
+        const float gamma = writes ? Bf16Value(a.norm.gamma[column]) : 0.0F;
+#pragma unroll
+        for (int e = 0; e < kCount; ++e) {
+          const int row = row0 + row_of(e0 + e);
+          const float square = AddXor16(RowSum16(writes ? prior[e] * prior[e] : 0.0F));
+          if (row >= a.m || !writes)
+            continue;
+          a.norm.scaled[static_cast<std::size_t>(row) * width + column] =
+              q8::Bf16Fast(prior[e] * gamma);
+          if (lane % 32 == 0)
+            a.norm.squares[static_cast<std::size_t>(row) * (width / 32) + column_tile + j] =
+                square;
+        }
       }
     }
     __builtin_amdgcn_sched_barrier(0);  // one tile's values at a time
@@ -374,6 +511,10 @@ __global__ __launch_bounds__(T::kThreads, T::kThreads / 256) void PrefillKernel(
   if constexpr (T::kShared) {
     static_assert(FN == 1, "a share lies within one column tile");
     constexpr int kShare = kValues / KG;
+    const std::integral_constant<int, kShare> share;
+    float c[kShare], s[kShare];  // loaded while the sums meet
+    if constexpr (kQkv)
+      load_rotary(share, c, s, group * kShare, 0);
     put(group);
     __syncthreads();
     float value[kShare];
@@ -385,7 +526,10 @@ __global__ __launch_bounds__(T::kThreads, T::kThreads / 256) void PrefillKernel(
 #pragma unroll
       for (int e = 0; e < kShare; ++e)
         value[e] += sums[(g * kValues + group * kShare + e) * T::kGroupThreads + tid];
-    emit(std::integral_constant<int, kShare>{}, value, group * kShare, 0);
+    if constexpr (kQkv)
+      emit_qkv(share, value, c, s, group * kShare, 0);
+    else
+      emit(share, value, group * kShare, 0);
     return;
   }
   if constexpr (KG == 2) {
@@ -410,6 +554,32 @@ __global__ __launch_bounds__(T::kThreads, T::kThreads / 256) void PrefillKernel(
     }
 }
 
+/// One thread per four columns: bf16(h gamma), and the sums of squares of
+/// eight threads' 32 columns.
+__global__ void ScaleKernel(const float* h, Norm norm, int m, int width) {
+  const std::size_t at =
+      (static_cast<std::size_t>(blockIdx.x) * blockDim.x + threadIdx.x) * 4;
+  if (at >= static_cast<std::size_t>(m) * width)  // whole groups of eight lanes
+    return;
+  const int column = static_cast<int>(at % static_cast<std::size_t>(width));
+  const float4 x = *reinterpret_cast<const float4*>(h + at);
+  const ushort4 gamma = *reinterpret_cast<const ushort4*>(norm.gamma + column);
+  *reinterpret_cast<uint2*>(norm.scaled + at) =
+      uint2{q8::PackBf16x2(x.x * Bf16Value(gamma.x), x.y * Bf16Value(gamma.y)),
+            q8::PackBf16x2(x.z * Bf16Value(gamma.z), x.w * Bf16Value(gamma.w))};
+  float square = x.x * x.x + x.y * x.y + x.z * x.z + x.w * x.w;
+#pragma unroll
+  for (int offset = 4; offset > 0; offset /= 2)
+    square += __shfl_xor(square, offset, kWave);
+  if (threadIdx.x % 8 == 0)
+    norm.squares[at / 32] = square;
+}
+
+/// The caches' epilogue over 160-row tiles does not unroll (its sums would
+/// lie in memory): Run picks another shape.
+template<class T>
+constexpr bool kTakesQkv = T::kBm != 160;
+
 template<class T>
 void Launch(const Product& p, Args a, hipStream_t stream) {
   a.m_tiles = static_cast<int>((p.m + T::kBm - 1) / T::kBm);
@@ -421,6 +591,10 @@ void Launch(const Product& p, Args a, hipStream_t stream) {
       case Out::kAccumulate: launch(PrefillKernel<T, true, 1>); break;
       case Out::kBf16: launch(PrefillKernel<T, true, 2>); break;
       case Out::kSwiGlu: launch(PrefillKernel<T, true, 3>); break;
+      case Out::kQkvCache:
+        if constexpr (kTakesQkv<T>)
+          launch(PrefillKernel<T, true, 4>);
+        break;
     }
   } else {
     switch (p.kind) {
@@ -428,6 +602,10 @@ void Launch(const Product& p, Args a, hipStream_t stream) {
       case Out::kAccumulate: launch(PrefillKernel<T, false, 1>); break;
       case Out::kBf16: launch(PrefillKernel<T, false, 2>); break;
       case Out::kSwiGlu: launch(PrefillKernel<T, false, 3>); break;
+      case Out::kQkvCache:
+        if constexpr (kTakesQkv<T>)
+          launch(PrefillKernel<T, false, 4>);
+        break;
     }
   }
 }
@@ -501,6 +679,13 @@ bool Use(std::size_t m, std::size_t k, std::size_t n) {
          here <= Rounds(m, n, 256, 256) * (3.0 + 1.5 * static_cast<double>(q8::Pairs(k)));
 }
 
+void Scale(const float* h, const Norm& norm, std::size_t m, std::size_t width,
+           hipStream_t stream) {
+  const std::size_t quads = m * width / 4;
+  ScaleKernel<<<static_cast<unsigned>((quads + 255) / 256), 256, 0, stream>>>(
+      h, norm, static_cast<int>(m), static_cast<int>(width));
+}
+
 int Run(const Product& p, hipStream_t stream, int shape) {
   Args a{};
   a.x = p.x;
@@ -512,8 +697,16 @@ int Run(const Product& p, hipStream_t stream, int shape) {
   a.n = static_cast<int>(p.n);
   a.pairs = static_cast<int>(q8::Pairs(p.k));
   a.groups = static_cast<int>(q8::Groups(p.n));
-  a.pair_stride = p.kind == Out::kSwiGlu ? a.groups / 2 : 1;
-  switch (shape >= 0 ? shape : PickShape(p.m, p.k, p.n)) {
+  a.pair_stride = p.kind == Out::kSwiGlu      ? a.groups / 2
+                  : p.kind == Out::kQkvCache ? p.qkv.head_dim / 32
+                                             : 1;
+  a.norm = p.norm;
+  a.qkv = p.qkv;
+  if (shape < 0)
+    shape = PickShape(p.m, p.k, p.n);
+  if (p.kind == Out::kQkvCache && ShapeOf(shape).bm == 160)
+    shape = 0;
+  switch (shape) {
     case 0: Launch<Tile<128, 2, 4, 1, 4>>(p, a, stream); break;
     case 1: Launch<Tile<128, 1, 4, 2, 4>>(p, a, stream); break;
     case 2: Launch<Tile<64, 1, 4, 4, 2>>(p, a, stream); break;

@@ -8,6 +8,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstddef>
+#include <cstdint>
 
 #include "common.hpp"
 
@@ -17,7 +18,32 @@ enum class Out : int {
   kStore = 0,       // y = product
   kAccumulate = 1,  // y += product
   kBf16 = 2,        // out = bf16(product)
-  kSwiGlu = 3       // out [m][n / 2] = bf16(silu(gate) up), n / 2 columns each
+  kSwiGlu = 3,      // out [m][n / 2] = bf16(silu(gate) up), n / 2 columns each
+  kQkvCache = 4     // rotary embedding, then q and the key and value caches
+};
+
+/// RMSNorm carried through the products: an operand bf16(h gamma) and, per
+/// row of h, its sums of squares over 32 columns each, [m][width / 32]. The
+/// rows' factors rsqrt(sum / width + eps) scale the product's outputs.
+struct Norm {
+  const Bf16* gamma = nullptr;  // [width]
+  Bf16* scaled = nullptr;       // [m][width]
+  float* squares = nullptr;     // [m][width / 32]
+  float eps = 0.0F;
+};
+
+/// What QkvRope's launch takes (dit_kernels.hpp); head_dim a multiple of 32.
+struct Qkv {
+  const float* rope = nullptr;  // [positions][head_dim] cos | sin, or null
+  const std::int32_t* positions = nullptr;
+  const std::int32_t* cache_rows = nullptr;
+  float* q = nullptr;
+  float* k_cache = nullptr;
+  float* v_cache = nullptr;
+  int heads = 0;
+  int kv_heads = 0;
+  int head_dim = 0;
+  int capacity = 0;
 };
 
 struct Product {
@@ -30,6 +56,8 @@ struct Product {
   Out kind = Out::kStore;
   float* y = nullptr;
   Bf16* out = nullptr;
+  Norm norm;  // kSwiGlu, kQkvCache: of x; kAccumulate: of y, made when norm.scaled is set
+  Qkv qkv;
 };
 
 /// Whether the kernels take the product's sizes (their 32-bit offsets).
@@ -45,8 +73,11 @@ Shape ShapeOf(int shape);
 int PickShape(std::size_t m, std::size_t k, std::size_t n, double* microseconds = nullptr);
 /// Whether the standalone products of more than 128 rows take these kernels.
 bool Use(std::size_t m, std::size_t k, std::size_t n);
-/// Launches the product (arguments checked by the caller: CheckProduct; for
-/// kSwiGlu n a multiple of 32). A non-negative `shape` forces that one.
+/// The norm's operand of rows h [m][width], width a multiple of 32.
+void Scale(const float* h, const Norm& norm, std::size_t m, std::size_t width,
+           hipStream_t stream);
+/// Launches the product (arguments checked by the caller: CheckProduct; k a
+/// multiple of 32, and n where the norm or SwiGLU take part). A non-negative `shape` forces that one.
 int Run(const Product& p, hipStream_t stream, int shape = -1);
 
 }  // namespace vx::prefill

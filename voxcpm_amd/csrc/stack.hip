@@ -10,9 +10,11 @@
 // workgroups score, so that a one-row decode step over a long cache still
 // spreads over the compute units; a second launch merges the chunks'
 // softmax statistics in chunk order. More rows take the reference's launch
-// sequence; past 128 rows its products are q8_prefill.hip's, with SwiGLU in
-// gate_up's epilogue (310 rows through the 12-layer encoder 1087 -> 724 us,
-// 617 through two base-LM layers 452 -> 304 us on MI355X).
+// sequence; past 128 rows the norms, the rotary embedding and the caches,
+// SwiGLU and the residual adds go into the epilogues of q8_prefill.hip's
+// products (LaunchPrompt: 310 rows through the 12-layer encoder 727 -> 655 us
+// on MI355X, 617 through two base-LM layers 291 -> 281 us, against a launch for
+// each norm and the rotary embedding).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -712,6 +714,11 @@ struct vx_stack {
   std::size_t gate_up_floats = 0;
   float* attention_partials = nullptr;
   std::size_t attention_partial_floats = 0;
+  // A prompt's norm operand and its rows' sums of squares (LaunchPrompt).
+  Bf16* normed = nullptr;
+  std::size_t normed_count = 0;
+  float* squares = nullptr;
+  std::size_t square_floats = 0;
   float* product_partials = nullptr;  // products beyond 128 rows
   std::size_t product_partial_floats = 0;
 
@@ -742,6 +749,7 @@ struct vx_stack {
     for (void* pointer :
          {static_cast<void*>(qkv), static_cast<void*>(q), static_cast<void*>(bf16),
           static_cast<void*>(gate_up), static_cast<void*>(attention_partials),
+          static_cast<void*>(normed), static_cast<void*>(squares),
           static_cast<void*>(product_partials), static_cast<void*>(h_frag),
           static_cast<void*>(attention_frag), static_cast<void*>(swiglu_frag)})
       if (pointer != nullptr)
@@ -755,10 +763,13 @@ struct vx_stack {
   /// Bf16Gemm::Linear (gemm.cpp:259-313): y[m][n] (+)= x W^T.
   int Linear(const Bf16* x, const void* w, float* y, std::size_t m, std::size_t k,
              std::size_t n, bool accumulate, hipStream_t stream) {
-    if (m > vx::kExactRows && vx::prefill::Supported(m, k, n))
-      return Prefill(x, w, y, nullptr, m, k, n,
-                     accumulate ? vx::prefill::Out::kAccumulate : vx::prefill::Out::kStore,
-                     stream);
+    if (m > vx::kExactRows && vx::prefill::Supported(m, k, n)) {
+      auto product = PromptProduct(
+          x, w, m, k, n,
+          accumulate ? vx::prefill::Out::kAccumulate : vx::prefill::Out::kStore);
+      product.y = y;
+      return vx::prefill::Run(product, stream);
+    }
     if (m > vx::kExactRows) {
       VX_TRY(Grow(&product_partials, &product_partial_floats, 2 * m * n,
                   "vx_stack_forward: hipMalloc"));
@@ -772,8 +783,8 @@ struct vx_stack {
                          stream, Kind());
   }
 
-  int Prefill(const Bf16* x, const void* w, float* y, Bf16* out, std::size_t m, std::size_t k,
-              std::size_t n, vx::prefill::Out kind, hipStream_t stream) const {
+  vx::prefill::Product PromptProduct(const Bf16* x, const void* w, std::size_t m, std::size_t k,
+                                     std::size_t n, vx::prefill::Out kind) const {
     vx::prefill::Product p;
     p.x = x;
     p.w = w;
@@ -782,26 +793,76 @@ struct vx_stack {
     p.k = k;
     p.n = n;
     p.kind = kind;
-    p.y = y;
-    p.out = out;
-    return vx::prefill::Run(p, stream);
+    return p;
   }
 
-  /// bf16(silu(gate) up) of the rows in `bf16`, left at *act: in gate_up's
-  /// epilogue beyond the exact rows (the buffer of its sums then holds the
-  /// result), else by a launch of its own, back into `bf16`.
-  int GateUp(const void* w, const Bf16** act, std::size_t m, hipStream_t stream) {
-    const std::size_t n = 2 * shape.ffn;
-    if (m > vx::kExactRows && vx::prefill::Supported(m, shape.hidden, n)) {
-      Bf16* const out = reinterpret_cast<Bf16*>(gate_up);
-      *act = out;
-      return Prefill(bf16, w, nullptr, out, m, shape.hidden, n, vx::prefill::Out::kSwiGlu,
-                     stream);
+  /// Whether a prompt of `rows` rows takes LaunchPrompt: past the exact
+  /// rows, with whole rotary tiles, within the products' offsets.
+  bool Prompt(std::size_t rows) const {
+    return rows > vx::kExactRows && shape.head_dim % 32 == 0 &&
+           vx::prefill::Supported(rows, shape.hidden, qkv_width) &&
+           vx::prefill::Supported(rows, q_width, shape.hidden) &&
+           vx::prefill::Supported(rows, shape.hidden, 2 * shape.ffn) &&
+           vx::prefill::Supported(rows, shape.ffn, shape.hidden);
+  }
+
+  /// A prompt's layers, five launches each: qkv's product with the norm's
+  /// row factors, the rotary embedding and the caches in its epilogue,
+  /// attention (and the merge of its chunks), o's with the residual add and
+  /// the next norm's operand, gate_up's with the row factors and SwiGLU,
+  /// down's as o's. RMSNorm's factor per row is applied after a product
+  /// instead of before its operand is rounded to bf16 (as the few-row kernels
+  /// of the DiT do).
+  int LaunchPrompt(const ForwardKey& f, std::size_t past, int splits, hipStream_t stream) {
+    using vx::prefill::Out;
+    const std::size_t rows = f.rows;
+    const std::size_t width = shape.hidden;
+    const std::size_t layer_stride = shape.kv_heads * f.capacity * shape.head_dim;
+    Bf16* const act = reinterpret_cast<Bf16*>(gate_up);
+    vx::prefill::Norm norm;
+    norm.scaled = normed;
+    norm.squares = squares;
+    norm.eps = shape.eps;
+    norm.gamma = layers.front().input_norm;
+    vx::prefill::Scale(f.hidden, norm, rows, width, stream);
+    for (std::size_t l = 0; l < layers.size(); ++l) {
+      const vx_dit_layer& layer = layers[l];
+      auto product = PromptProduct(normed, layer.qkv, rows, width, qkv_width, Out::kQkvCache);
+      product.norm = norm;
+      product.qkv.rope = shape.rope != 0 ? weights.rope : nullptr;
+      product.qkv.positions = f.positions;
+      product.qkv.cache_rows = f.cache_rows;
+      product.qkv.q = q;
+      product.qkv.k_cache = f.k_cache + l * layer_stride;
+      product.qkv.v_cache = f.v_cache + l * layer_stride;
+      product.qkv.heads = static_cast<int>(shape.heads);
+      product.qkv.kv_heads = static_cast<int>(shape.kv_heads);
+      product.qkv.head_dim = static_cast<int>(shape.head_dim);
+      product.qkv.capacity = static_cast<int>(f.capacity);
+      VX_TRY(vx::prefill::Run(product, stream));
+      vx::stack::Attention(q, product.qkv.k_cache, product.qkv.v_cache, bf16, false,
+                           attention_partials, rows, f.rows_per_sequence, f.keys_per_sequence,
+                           past, f.causal, shape.heads, shape.kv_heads, shape.head_dim,
+                           f.capacity, splits, nullptr, stream);
+      product = PromptProduct(bf16, layer.o, rows, q_width, width, Out::kAccumulate);
+      product.y = f.hidden;
+      product.norm = norm;
+      product.norm.gamma = layer.post_norm;
+      VX_TRY(vx::prefill::Run(product, stream));
+      product = PromptProduct(normed, layer.gate_up, rows, width, 2 * shape.ffn, Out::kSwiGlu);
+      product.out = act;
+      product.norm = norm;
+      VX_TRY(vx::prefill::Run(product, stream));
+      product = PromptProduct(act, layer.down, rows, shape.ffn, width, Out::kAccumulate);
+      product.y = f.hidden;
+      if (l + 1 < layers.size()) {
+        product.norm = norm;
+        product.norm.gamma = layers[l + 1].input_norm;
+      }
+      VX_TRY(vx::prefill::Run(product, stream));
     }
-    VX_TRY(Linear(bf16, w, gate_up, m, shape.hidden, n, false, stream));
-    vx::kernels::SwiGlu(gate_up, bf16, m, shape.ffn, stream);
-    *act = bf16;
-    return VX_OK;
+    vx::kernels::RmsNorm(f.hidden, weights.norm, bf16, f.output, rows, width, shape.eps, stream);
+    return vx::LaunchStatus("vx_stack_forward");
   }
 
   int Resolved(std::size_t rows) const {
@@ -884,6 +945,8 @@ struct vx_stack {
                            stream);
       return vx::LaunchStatus("vx_stack_forward");
     }
+    if (Prompt(rows))
+      return LaunchPrompt(f, past, splits, stream);
     for (std::size_t l = 0; l < layers.size(); ++l) {
       const vx_dit_layer& layer = layers[l];
       float* keys = f.k_cache + l * layer_stride;
@@ -900,9 +963,9 @@ struct vx_stack {
       VX_TRY(Linear(bf16, layer.o, f.hidden, rows, q_width, width, true, stream));
       vx::kernels::RmsNorm(f.hidden, layer.post_norm, bf16, nullptr, rows, width, shape.eps,
                            stream);
-      const Bf16* act = nullptr;
-      VX_TRY(GateUp(layer.gate_up, &act, rows, stream));
-      VX_TRY(Linear(act, layer.down, f.hidden, rows, ffn, width, true, stream));
+      VX_TRY(Linear(bf16, layer.gate_up, gate_up, rows, width, 2 * ffn, false, stream));
+      vx::kernels::SwiGlu(gate_up, bf16, rows, ffn, stream);
+      VX_TRY(Linear(bf16, layer.down, f.hidden, rows, ffn, width, true, stream));
     }
     vx::kernels::RmsNorm(f.hidden, weights.norm, bf16, f.output, rows, width, shape.eps,
                          stream);
@@ -944,6 +1007,10 @@ struct vx_stack {
     VX_TRY(Grow(&qkv, &qkv_floats, rows * qkv_width, what));
     VX_TRY(Grow(&bf16, &bf16_count, rows * wide, what));
     VX_TRY(Grow(&gate_up, &gate_up_floats, rows * 2 * shape.ffn, what));
+    if (Prompt(rows)) {
+      VX_TRY(Grow(&normed, &normed_count, rows * shape.hidden, what));
+      VX_TRY(Grow(&squares, &square_floats, rows * (shape.hidden / 32), what));
+    }
     const void* after[] = {attention_partials, q, qkv, bf16, gate_up};
     const bool moved = !std::equal(std::begin(before), std::end(before), std::begin(after));
     if (!graphed)
