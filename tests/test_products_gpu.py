@@ -392,6 +392,26 @@ def test_panel_operand_shapes(vx, oracle, cuda, stream, shape, weights, rows, k,
     assert worst <= LIMIT, worst
 
 
+@pytest.mark.parametrize("rows", [65, 77, 128])
+@pytest.mark.parametrize("k,n", [(6144, 2055), (4192, 70)])
+def test_exact_long_reductions(vx, oracle, cuda, stream, rows, k, n):
+    """65 to 128 rows over more than 4096 columns of k take the panel-operand
+    kernels with the exact per-block arithmetic: rows, columns and an odd
+    block count that end inside a tile, accumulation and bf16 results."""
+    rng = synth.Rng(12, rows + n)
+    blocks = synth.q8_blocks(rng, n, k)
+    packed = vx.q8_pack(to_device(blocks, cuda), n, k)
+    x = synth.activations(rng, rows, k)
+    before = rng.normal(rows * n).astype(np.float32).reshape(rows, n)
+    y = run_product(vx, to_device(x, cuda), packed, n, None, None, None, cuda)
+    assert oracle.q8_check(y, x, blocks) <= LIMIT
+    added = run_product(vx, to_device(x, cuda), packed, n, before, None, None, cuda)
+    assert oracle.q8_check(added, x, blocks, before) <= LIMIT
+    y16 = vx.q8_linear_bf16(to_device(x, cuda), packed, n)
+    torch.cuda.synchronize()
+    assert np.array_equal(bf16_host(y16), synth.bf16_bits(y))
+
+
 def test_stream_read_reads_every_byte(vx, cuda, stream):
     """The read-ceiling kernel loads every 16-byte chunk: the XOR of the
     buffer's words reaches the sink only when it equals `never`."""

@@ -114,7 +114,9 @@ int Product(const uint16_t* x, const void* packed, float* y, uint16_t* y_bf16,
             size_t m, size_t k, size_t n, int accumulate, vx_scratch* scratch,
             int rg, int waves, int splits, void* stream,
             vx::q8::Weights kind = vx::q8::Weights::kQ8) {
-  if (vx::prefill::Use(m, k, n)) {
+  const bool exact = kind == vx::q8::Weights::kQ8 && rg == 0 && waves == 0 && splits == 0 &&
+                     vx::prefill::UseExact(m, k, n);
+  if (exact || vx::prefill::Use(m, k, n)) {
     vx::prefill::Product p;
     p.x = x;
     p.w = packed;
@@ -127,7 +129,8 @@ int Product(const uint16_t* x, const void* packed, float* y, uint16_t* y_bf16,
                                : vx::prefill::Out::kStore;
     p.y = y;
     p.out = y_bf16;
-    return vx::prefill::Run(p, vx::Stream(stream));
+    return exact ? vx::prefill::RunExact(p, vx::Stream(stream))
+                 : vx::prefill::Run(p, vx::Stream(stream));
   }
   if (vx::UseRowBlocks(m, k, n, kind == vx::q8::Weights::kQ8))
     return vx::RunRowBlocks(x, packed, y, y_bf16, m, k, n, accumulate != 0,

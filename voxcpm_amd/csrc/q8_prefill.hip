@@ -113,8 +113,13 @@ struct Tile {
   static constexpr int kLds = KG * kStageBytes > kMeetBytes ? KG * kStageBytes : kMeetBytes;
 };
 
-template<class T, bool BF16, int OUT>
+/// MODE: the weights' arithmetic.
+enum Mode : int { kExpanded = 0, kPanels16 = 1, kExact = 2 };
+
+template<class T, int MODE, int OUT>
 __global__ __launch_bounds__(T::kThreads, T::kThreads / 256) void PrefillKernel(Args a) {
+  constexpr bool BF16 = MODE == kPanels16;
+  constexpr bool EXACT = MODE == kExact;
   constexpr int FN = T::kFn;
   constexpr int NW = T::kNw;
   constexpr int KG = T::kKg;
@@ -202,6 +207,8 @@ __global__ __launch_bounds__(T::kThreads, T::kThreads / 256) void PrefillKernel(
     if constexpr (BF16)
       return AsBf16x8(w.v[j][2 * block + half]);
     const uint4& v = w.v[j][half];
+    if constexpr (EXACT)
+      return block == 0 ? q8::Int8x8ToBf16(v.x, v.y) : q8::Int8x8ToBf16(v.z, v.w);
     const float scale = HalfValue(static_cast<std::uint16_t>(
         block == 0 ? w.scales[j] & 0xFFFFU : w.scales[j] >> 16));
     return AsBf16x8(block == 0 ? q8::Expand(v.x, v.y, scale) : q8::Expand(v.z, v.w, scale));
@@ -296,6 +303,7 @@ __global__ __launch_bounds__(T::kThreads, T::kThreads / 256) void PrefillKernel(
   // first step: zeros).
   uint4 x_operand[2][kFm];
   q8::Bf16x8 w_operand[2][FN];
+  F32x16 block_sum[EXACT ? kFm : 1];
   if constexpr (T::kAhead) {
 #pragma unroll
     for (int i = 0; i < kFm; ++i)
@@ -327,7 +335,29 @@ __global__ __launch_bounds__(T::kThreads, T::kThreads / 256) void PrefillKernel(
         for (int j = 0; j < FN; ++j)
           w_operand[now][j] = weights_of(ws[d], j, kk / 2, kk % 2);
         const int ready = T::kAhead ? 1 - now : 0;
-        multiply(x_operand[ready], w_operand[ready]);
+        if constexpr (EXACT) {
+          // A block's float32 sum from zero, then scaled into the row's.
+          static_assert(!EXACT || (!T::kAhead && FN == 1), "exact tiles");
+#pragma unroll
+          for (int i = 0; i < kFm; ++i) {
+            if (kk % 2 == 0) {
+#pragma unroll
+              for (int v = 0; v < 16; ++v)
+                block_sum[i][v] = 0.0F;
+            }
+            block_sum[i] = bf16x3::Mfma32(AsBf16x8(x_operand[0][i]), w_operand[0][0],
+                                          block_sum[i]);
+            if (kk % 2 == 1) {
+              const float scale = HalfValue(static_cast<std::uint16_t>(
+                  kk == 1 ? ws[d].scales[0] & 0xFFFFU : ws[d].scales[0] >> 16));
+#pragma unroll
+              for (int v = 0; v < 16; ++v)
+                acc[i][0][v] = __builtin_fmaf(scale, block_sum[i][v], acc[i][0][v]);
+            }
+          }
+        } else {
+          multiply(x_operand[ready], w_operand[ready]);
+        }
 #pragma unroll
         for (int i = kk * kPieces / 4; i < (kk + 1) * kPieces / 4; ++i) {
           store_x(next, i, xs[next][i]);
@@ -587,28 +617,33 @@ void Launch(const Product& p, Args a, hipStream_t stream) {
   const auto launch = [&](auto kernel) { kernel<<<a.tiles, T::kThreads, 0, stream>>>(a); };
   if (p.bf16) {
     switch (p.kind) {
-      case Out::kStore: launch(PrefillKernel<T, true, 0>); break;
-      case Out::kAccumulate: launch(PrefillKernel<T, true, 1>); break;
-      case Out::kBf16: launch(PrefillKernel<T, true, 2>); break;
-      case Out::kSwiGlu: launch(PrefillKernel<T, true, 3>); break;
+      case Out::kStore: launch(PrefillKernel<T, kPanels16, 0>); break;
+      case Out::kAccumulate: launch(PrefillKernel<T, kPanels16, 1>); break;
+      case Out::kBf16: launch(PrefillKernel<T, kPanels16, 2>); break;
+      case Out::kSwiGlu: launch(PrefillKernel<T, kPanels16, 3>); break;
       case Out::kQkvCache:
         if constexpr (kTakesQkv<T>)
-          launch(PrefillKernel<T, true, 4>);
+          launch(PrefillKernel<T, kPanels16, 4>);
         break;
     }
   } else {
     switch (p.kind) {
-      case Out::kStore: launch(PrefillKernel<T, false, 0>); break;
-      case Out::kAccumulate: launch(PrefillKernel<T, false, 1>); break;
-      case Out::kBf16: launch(PrefillKernel<T, false, 2>); break;
-      case Out::kSwiGlu: launch(PrefillKernel<T, false, 3>); break;
+      case Out::kStore: launch(PrefillKernel<T, kExpanded, 0>); break;
+      case Out::kAccumulate: launch(PrefillKernel<T, kExpanded, 1>); break;
+      case Out::kBf16: launch(PrefillKernel<T, kExpanded, 2>); break;
+      case Out::kSwiGlu: launch(PrefillKernel<T, kExpanded, 3>); break;
       case Out::kQkvCache:
         if constexpr (kTakesQkv<T>)
-          launch(PrefillKernel<T, false, 4>);
+          launch(PrefillKernel<T, kExpanded, 4>);
         break;
     }
   }
 }
+
+/// The exact kernels' one tile: 32 x 32, sixteen groups of k. Each 32-column
+/// block's products sum from zero on the matrix cores and are then scaled
+/// into the group's sums (kernels/wmma_products.hip:192-215).
+using ExactTile = Tile<32, 1, 1, 16, 2>;
 
 }  // namespace
 
@@ -686,7 +721,9 @@ void Scale(const float* h, const Norm& norm, std::size_t m, std::size_t width,
       h, norm, static_cast<int>(m), static_cast<int>(width));
 }
 
-int Run(const Product& p, hipStream_t stream, int shape) {
+namespace {
+
+Args ArgsOf(const Product& p) {
   Args a{};
   a.x = p.x;
   a.w = static_cast<const std::uint8_t*>(p.w);
@@ -702,6 +739,43 @@ int Run(const Product& p, hipStream_t stream, int shape) {
                                              : 1;
   a.norm = p.norm;
   a.qkv = p.qkv;
+  return a;
+}
+
+}  // namespace
+
+bool UseExact(std::size_t m, std::size_t k, std::size_t n) {
+  // Past 64 rows the engine needs a second block of rows, and its 16-column
+  // workgroups each read all of x: over more than 4096 columns of k these
+  // tiles are faster while they take one round (77 x 6144 x 2055 19.1 ->
+  // 11.5 us, 100 x 6144 x 1024 12.5 -> 10.7, 128 x 8192 x 2048 18.4 -> 14.5,
+  // 65 x 5120 x 130 10.3 -> 9.6, 77 x 4128 x 2048 10.4 -> 10.2 on MI355X, with
+  // the call). In one block the engine is the faster one (49 x 6144 x 2048
+  // 10.2 there, 10.8 here; 49 x 8192 x 70 8.6 and 12.1). Over shorter k its
+  // sums come out closer to 64 bits (100 x 1024 x 1024 7.0e-8 there, 8.3e-8
+  // here; 77 x 6144 x 2048 1.06e-7 and 1.01e-7).
+  return m > 64 && m <= kExactRows && k > 4096 && Supported(m, k, n) &&
+         ((m + 31) / 32) * ((n + 31) / 32) <= kComputeUnits;
+}
+
+int RunExact(const Product& p, hipStream_t stream) {
+  Args a = ArgsOf(p);
+  a.m_tiles = static_cast<int>((p.m + 31) / 32);
+  a.tiles = a.m_tiles * static_cast<int>((p.n + 31) / 32);
+  const auto launch = [&](auto kernel) {
+    kernel<<<a.tiles, ExactTile::kThreads, 0, stream>>>(a);
+  };
+  if (p.kind == Out::kBf16)
+    launch(PrefillKernel<ExactTile, kExact, 2>);
+  else if (p.kind == Out::kAccumulate)
+    launch(PrefillKernel<ExactTile, kExact, 1>);
+  else
+    launch(PrefillKernel<ExactTile, kExact, 0>);
+  return LaunchStatus("exact product");
+}
+
+int Run(const Product& p, hipStream_t stream, int shape) {
+  const Args a = ArgsOf(p);
   if (shape < 0)
     shape = PickShape(p.m, p.k, p.n);
   if (p.kind == Out::kQkvCache && ShapeOf(shape).bm == 160)

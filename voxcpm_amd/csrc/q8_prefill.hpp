@@ -73,6 +73,12 @@ Shape ShapeOf(int shape);
 int PickShape(std::size_t m, std::size_t k, std::size_t n, double* microseconds = nullptr);
 /// Whether the standalone products of more than 128 rows take these kernels.
 bool Use(std::size_t m, std::size_t k, std::size_t n);
+/// Whether an m x k x n product of Q8_0 panels with the exact per-block
+/// arithmetic (33 to 128 rows) takes RunExact rather than the engine.
+bool UseExact(std::size_t m, std::size_t k, std::size_t n);
+/// The product with each 32-column block's float32 sum scaled into the row's
+/// (kernels/wmma_products.hip:192-215): kStore, kAccumulate or kBf16.
+int RunExact(const Product& p, hipStream_t stream);
 /// The norm's operand of rows h [m][width], width a multiple of 32.
 void Scale(const float* h, const Norm& norm, std::size_t m, std::size_t width,
            hipStream_t stream);

@@ -770,6 +770,13 @@ struct vx_stack {
       product.y = y;
       return vx::prefill::Run(product, stream);
     }
+    if (Kind() == vx::q8::Weights::kQ8 && vx::prefill::UseExact(m, k, n)) {
+      auto product = PromptProduct(
+          x, w, m, k, n,
+          accumulate ? vx::prefill::Out::kAccumulate : vx::prefill::Out::kStore);
+      product.y = y;
+      return vx::prefill::RunExact(product, stream);
+    }
     if (m > vx::kExactRows) {
       VX_TRY(Grow(&product_partials, &product_partial_floats, 2 * m * n,
                   "vx_stack_forward: hipMalloc"));
