@@ -58,17 +58,6 @@ __device__ inline Octet Split(const float4& a, const float4& b) {
                uint4{p0.l, p1.l, p2.l, p3.l}};
 }
 
-/// c += a b over the kept products, the smallest first.
-__device__ inline F32x16 Multiply(const Octet& a, const Octet& b, F32x16 c) {
-  using q8::AsBf16x8;
-  c = Mfma32(AsBf16x8(a.l), AsBf16x8(b.h), c);
-  c = Mfma32(AsBf16x8(a.m), AsBf16x8(b.m), c);
-  c = Mfma32(AsBf16x8(a.h), AsBf16x8(b.l), c);
-  c = Mfma32(AsBf16x8(a.m), AsBf16x8(b.h), c);
-  c = Mfma32(AsBf16x8(a.h), AsBf16x8(b.m), c);
-  return Mfma32(AsBf16x8(a.h), AsBf16x8(b.h), c);
-}
-
 }  // namespace vx::bf16x3
 
 #endif  // VOXCPM_AMD_BF16X3_HPP_

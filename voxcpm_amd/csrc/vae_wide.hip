@@ -177,8 +177,8 @@ __device__ inline int DieOrdered(int b, int blocks) {
   return die * per + min(die, extra) + b / kDies;
 }
 
-/// The six products of two bfloat16 triples (bf16x3::Multiply's) and mm's,
-/// from two planes at a time: pass 0 holds h and m, pass 1 h and l.
+/// The six kept products of two bfloat16 triples (bf16x3.hpp), from two
+/// planes at a time: pass 0 holds h and m, pass 1 h and l.
 template<int PASS>
 __device__ inline F32x16 MultiplyLarge(const Octet& x, const Octet& w, F32x16 sum) {
   using q8::AsBf16x8;
