@@ -408,3 +408,48 @@ def test_tile_attention_past_float16(vx, cuda, stream, heads, kv_heads, head_dim
                           bound[last:][:, :, rest])
     assert np.all(np.abs(attend(q, kc, vc * 2.0**20) * 2.0**-20 - plain) <= bound)
     assert np.all(np.abs(attend(q * 2.0**-20, kc * 2.0**20, vc) - plain) <= bound)
+
+
+@pytest.mark.parametrize("heads,kv_heads,head_dim", [(16, 2, 128), (4, 4, 64)])
+@pytest.mark.parametrize("rows,past", [(150, 40), (129, 700)])
+def test_tile_attention_below_float16(vx, cuda, stream, heads, kv_heads, head_dim, rows, past):
+    """What lies below the range of the matrix-core attention's float16 pairs
+    keeps float32's precision: small values all over, of the first keys only
+    (rows that count no others), and in one dimension; small keys under large
+    queries and the reverse. Each gives what the unscaled call gives times
+    the scale (powers of two: exact, the bound one bf16 ulp of the sum)."""
+    rng = synth.Rng(59, rows + past)
+    keys = past + rows
+    q = f32(1.5 * rng.normal(rows * heads * head_dim).reshape(rows, heads, head_dim))
+    kc = f32(rng.normal(kv_heads * keys * head_dim).reshape(kv_heads, keys, head_dim))
+    vc = f32(rng.normal(kv_heads * keys * head_dim).reshape(kv_heads, keys, head_dim))
+
+    def attend(q, k, v):
+        got = vx.split_attention(dev(f32(q), cuda), dev(f32(k), cuda), dev(f32(v), cuda), rows,
+                                 rows, past, True, heads, kv_heads)
+        torch.cuda.synchronize()
+        return synth.bf16_values(host_bf16(got)).reshape(rows, heads, head_dim)
+
+    def check(got, at, what):
+        worst = float(np.max(np.abs(got - plain[at]) / bound[at]))
+        print(f"{what}: worst {worst:.2f} of the bound", flush=True)
+        assert worst <= 1, what
+
+    plain = attend(q, kc, vc)
+    bound = 2.0**-7 * np.abs(plain) + 2.0**-20 * np.max(np.abs(vc))
+    everything = np.s_[:]
+    for exponent in (-20, -30, -45):
+        scale = 2.0**exponent
+        check(attend(q, kc, vc * scale) / scale, everything, f"values 2^{exponent}")
+        few = vc.copy()
+        few[:, :past + 21] *= scale
+        check(attend(q, kc, few)[:21] / scale, np.s_[:21], f"first keys' values 2^{exponent}")
+        one = vc.copy()
+        one[:, :, 5] *= scale
+        got = attend(q, kc, one)
+        check(got[:, :, 5] / scale, np.s_[:, :, 5], f"one dimension 2^{exponent}")
+        check(got[:, :, 6:], np.s_[:, :, 6:], f"beside a dimension of 2^{exponent}")
+    for exponent in (13, 20):
+        scale = 2.0**exponent
+        check(attend(q * scale, kc / scale, vc), everything, f"queries 2^{exponent}")
+        check(attend(q / scale, kc * scale, vc), everything, f"keys 2^{exponent}")

@@ -6,10 +6,14 @@
 // Against the float32 matrix instructions, a sixteenth of the f16 rate, the
 // operands lose at most two bits, and the sums round once per 16 terms
 // instead of once per 4, which more than makes up for it over long
-// reductions. Below 2^-14 h turns subnormal and l takes over what it drops
-// (absolute error under 2^-35). Past 65504 float16 ends: callers test
-// for it (TooLarge) and take such operands as three bfloat16 terms
-// (bf16x3.hpp).
+// reductions. Below 2^-14 h turns subnormal and l takes over what it drops,
+// in steps of 2^-35: an absolute error of at most 2^-36 per operand, whatever
+// its size, so that operands which are small throughout would lose float32's
+// precision. From 65520 on h is infinite and l is too, of the other sign: a sum
+// with such an operand is NaN, whatever it is multiplied by. Callers start
+// over in a format of float32's range (three bfloat16 terms, bf16x3.hpp, or
+// float32 itself) where a group of operands is neither zeros nor large enough
+// (Least), and where an operand is too large (TooLarge, or by the NaN).
 #ifndef VOXCPM_AMD_F16X2_HPP_
 #define VOXCPM_AMD_F16X2_HPP_
 
@@ -71,6 +75,20 @@ __device__ inline float Largest(float most, const float4& v) {
   return fmaxf(fmaxf(most, fabsf(v.z)), fabsf(v.w));
 }
 __device__ inline bool TooLarge(float most) { return most > kLargest; }
+
+/// The smallest nonzero one of the groups' largest magnitudes: the error of
+/// a small operand, at most 2^-36, is at most 2^-36 / least of its group's
+/// largest.
+struct Least {
+  std::uint32_t bits = ~0U;  // the magnitude's bits less one: zero comes last
+  __device__ void Add(float group) {
+    const std::uint32_t own = __builtin_bit_cast(std::uint32_t, group) - 1U;
+    bits = own < bits ? own : bits;
+  }
+  __device__ bool Below(float limit) const {
+    return bits < __builtin_bit_cast(std::uint32_t, limit) - 1U;
+  }
+};
 
 }  // namespace vx::f16x2
 

@@ -20,9 +20,10 @@
 // unnormalised values, and a second launch merges a row's chunks in chunk
 // order.
 //
-// A workgroup that met a value past float16's range, or whose sums came out
-// NaN or infinite (a masked key's value weighs 0, which a NaN survives),
-// starts over key by key in float32.
+// A workgroup that met values too small for float16 pairs (kLeast), or whose
+// sums came out NaN or infinite, starts over key by key in float32: a value
+// past float16's range makes them NaN, and so does a masked key's NaN or
+// infinity, whose weight is 0.
 //
 // Measured on MI355X: 300 rows of 16 heads over 1800 keys 390 us on the
 // float32 split kernel, 55 us from three bfloat16 terms (twice the products,
@@ -62,6 +63,13 @@ constexpr std::size_t kTargetWorkgroups = 512;
 // A transposed value row in LDS: 32 f16 keys and 16 bytes of padding, so
 // that the 16-byte reads of eight consecutive rows fall on distinct banks.
 constexpr int kValueRow = 80;
+// Eight neighbouring dimensions of a query or a key, four of a value, and one
+// dimension of four neighbouring values (of a run's whole quads of keys: the
+// fifth key of a five-row patch alone would often fail) are each to hold a
+// magnitude of at least this, or zeros alone: the pairs' absolute error of 2^-36 is then 2^-20
+// of it, an eight-hundredth of the bfloat16 output's rounding. (Four values
+// of spread 0.01 are all smaller once in 5 10^11, of spread 0.001 once in 5 10^7.)
+constexpr float kLeast = 0x1p-16F;
 
 struct TileArgs {
   const float* q;
@@ -207,14 +215,14 @@ __global__ __launch_bounds__(kThreads, 2) void TileAttentionKernel(TileArgs a) {
                                                                   4 * dim_quad));
     }
   };
-  float most = 0.0F;  // the largest magnitude this thread has split
-  const auto store = [&]() {
+  f16x2::Least least;  // of what this thread has split
+  const auto store = [&](int key0) {
 #pragma unroll
     for (int i = 0; i < kKeyLoads; ++i) {
       const int piece = tid + kThreads * i;
       const int key = piece / kChunks;
       const Octet o = f16x2::Split(key_next[i][0], key_next[i][1]);
-      most = f16x2::Largest(f16x2::Largest(most, key_next[i][0]), key_next[i][1]);
+      least.Add(f16x2::Largest(f16x2::Largest(0.0F, key_next[i][0]), key_next[i][1]));
       const int at = key * kKeyRow + piece % kChunks;
       key_planes[0][at] = o.h;
       key_planes[1][at] = o.l;
@@ -227,12 +235,16 @@ __global__ __launch_bounds__(kThreads, 2) void TileAttentionKernel(TileArgs a) {
                                 {v[0].w, v[1].w, v[2].w, v[3].w}};
       // S^T leaves keys 16 c + 8 j + 4 half + 0..3 in one lane's registers:
       // the row holds, per 16 keys, half 0's two quads and then half 1's.
+      const bool whole = key0 + 4 * value_quad + 4 <= key_end;
       const int slot = (value_quad / 4) * 32 + (value_quad % 2) * 16 + ((value_quad / 2) % 2) * 8;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const f16x2::Pair p0 = f16x2::Split(rows[e][0], rows[e][1]);
         const f16x2::Pair p1 = f16x2::Split(rows[e][2], rows[e][3]);
-        most = f16x2::Largest(most, v[e]);
+        least.Add(f16x2::Largest(0.0F, v[e]));
+        least.Add(whole ? f16x2::Largest(0.0F, make_float4(rows[e][0], rows[e][1], rows[e][2],
+                                                           rows[e][3]))
+                        : 0.0F);
         const int at = (4 * dim_quad + e) * kValueRow + slot;
         *reinterpret_cast<uint2*>(&value_planes[0][at]) = uint2{p0.h, p1.h};
         *reinterpret_cast<uint2*>(&value_planes[1][at]) = uint2{p0.l, p1.l};
@@ -253,7 +265,7 @@ __global__ __launch_bounds__(kThreads, 2) void TileAttentionKernel(TileArgs a) {
       x = make_float4(x.x * a.scale, x.y * a.scale, x.z * a.scale, x.w * a.scale);
       y = make_float4(y.x * a.scale, y.y * a.scale, y.z * a.scale, y.w * a.scale);
       qs[s] = f16x2::Split(x, y);
-      most = f16x2::Largest(f16x2::Largest(most, x), y);
+      least.Add(f16x2::Largest(f16x2::Largest(0.0F, x), y));
     }
   }
 
@@ -268,7 +280,7 @@ __global__ __launch_bounds__(kThreads, 2) void TileAttentionKernel(TileArgs a) {
 
   for (int key0 = key_begin; key0 < key_end; key0 += kKeys) {
     __syncthreads();  // the step before has been read
-    store();
+    store(key0);
     __syncthreads();
     // Steps past the run's end load zeros.
     load(key0 + kKeys);
@@ -363,7 +375,7 @@ __global__ __launch_bounds__(kThreads, 2) void TileAttentionKernel(TileArgs a) {
 #pragma unroll
     for (int v = 0; v < 16; ++v)
       check[v % 4] = __builtin_fmaf(out[i][v], 0.0F, check[v % 4]);
-  if (f16x2::TooLarge(most) || check[0] + check[1] + (check[2] + check[3]) != 0.0F)
+  if (least.Below(kLeast) || check[0] + check[1] + (check[2] + check[3]) != 0.0F)
     restart = 1;
   __syncthreads();
   // Located again rather than held in registers through the steps (a spilled
