@@ -202,3 +202,66 @@ def test_vae_wide_against_short_chunks(vx, cuda):
     error = float(np.max(np.abs(at_once - np.concatenate(pieces))))
     print(f"wide against 8-frame chunks: max |d| {error:.2e}", flush=True)
     assert error <= BOUND
+
+
+def scaled_blocks(weights, scale):
+    """Every decoder block's residual stream times `scale` (a power of two):
+    its transposed convolution and its units' biases scaled, the next block's
+    input (of the last block the output convolution) scaled back."""
+    blocks = weights.tensors["blocks"]
+    for b, block in enumerate(blocks):
+        for name in ("up", "up_bias"):
+            block[name] = block[name] * np.float32(scale)
+        for unit in block["units"]:
+            for name in ("depthwise_bias", "pointwise_bias"):
+                unit[name] = unit[name] * np.float32(scale)
+        if b + 1 < len(blocks):
+            blocks[b + 1]["scale"] = blocks[b + 1]["scale"] * np.float32(1 / scale)
+    weights.tensors["out_conv"] = weights.tensors["out_conv"] * np.float32(1 / scale)
+
+
+@pytest.mark.parametrize("scale", [2.0**-18, 2.0**-30, 2.0**-45])
+def test_vae_wide_below_float16(vx, oracle, cuda, scale):
+    """Weights and activations below the float16 pairs' range, scaled back
+    where a block hands its rows on: the wide path's workgroups start over
+    from bfloat16 triples. The bound: the float32 products' measured 5.1e-6
+    (module docstring), with a factor of four for these weights."""
+    weights = synth.vae_weights(WIDE, 107)
+    scaled_blocks(weights, scale)
+    frames = 25
+    latents = synth.Rng(108, frames).normal(frames * WIDE.latent).astype(np.float32)
+    latents = latents.reshape(frames, WIDE.latent)
+    ref = oracle.OracleVae(weights).decode(latents)
+    got = vx.Vae(weights).decode(torch.from_numpy(latents).to(cuda)).cpu().numpy()
+    error = float(np.max(np.abs(got - ref)))
+    print(f"blocks scaled by {scale:.1e}: max |d| {error:.2e}, signal std {np.std(ref):.3f}",
+          flush=True)
+    assert np.std(ref) > 0.1
+    assert error <= 2e-5
+
+
+@pytest.mark.parametrize("direction", ["past", "below"])
+def test_vae_wide_out_of_range_tiles(vx, cuda, direction):
+    """Operands outside the float16 pairs' range in every product tile shape
+    of the wide path (61 frames at the VoxCPM2 shape: 64 x 64 tiles in four
+    groups of k, 128 x 128 in two and in one), against the same latents in
+    chunks of 8 frames, which take the float32 kernels."""
+    config = CONFIGS["voxcpm2"]
+    weights = synth.vae_weights(config, 109)
+    if direction == "past":
+        weights.tensors["in_pointwise"] = weights.tensors["in_pointwise"] * np.float32(1e6)
+        weights.tensors["out_conv"] = weights.tensors["out_conv"] * np.float32(1e-6)
+    else:
+        scaled_blocks(weights, 2.0**-30)
+    frames = 61
+    latents = torch.from_numpy(synth.Rng(110, frames).normal(frames * config.latent).astype(
+        np.float32).reshape(frames, config.latent)).to(cuda)
+    at_once = vx.Vae(weights).decode(latents).cpu().numpy()
+    chunked = vx.Vae(weights)
+    pieces = [chunked.decode(latents[at:at + 8]).cpu().numpy() for at in range(0, frames, 8)]
+    want = np.concatenate(pieces)
+    error = float(np.max(np.abs(at_once - want)))
+    print(f"{direction} float16's range: max |d| {error:.2e}, signal std {np.std(want):.3f}",
+          flush=True)
+    assert np.std(want) > 0.1
+    assert error <= BOUND

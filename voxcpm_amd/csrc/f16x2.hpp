@@ -90,6 +90,19 @@ struct Least {
   }
 };
 
+/// The groups' Least and the largest magnitude of all.
+struct Range {
+  float most = 0.0F;
+  Least least;
+  __device__ void Add(float group) {
+    most = fmaxf(most, group);
+    least.Add(group);
+  }
+  __device__ bool Holds(float at_least) const {
+    return !TooLarge(most) && !least.Below(at_least);
+  }
+};
+
 }  // namespace vx::f16x2
 
 #endif  // VOXCPM_AMD_F16X2_HPP_

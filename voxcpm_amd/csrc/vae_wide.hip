@@ -21,10 +21,10 @@
 // traffic. In and out are two buffers: a tile's history rows belong to the
 // tile before it.
 //
-// A workgroup that has met an operand past float16's range (65504) starts
-// over from three bfloat16 terms (bf16x3.hpp), which span float32's: nothing
-// is stored before its last product, and the histories it leaves are the
-// same values again.
+// A workgroup that has met operands outside the float16 pairs' range (kLeast,
+// 65504) starts over from three bfloat16 terms (bf16x3.hpp), which span
+// float32's: nothing is stored before its last product, and the histories it
+// leaves are the same values again.
 //
 // Measured on MI355X over 125 frames at VoxCPM2's shape, per launch, against
 // the float32 kernels' (F32TileKernel and a depthwise launch per unit):
@@ -60,6 +60,11 @@ constexpr int kThreads = 256;
 constexpr int kTaps = 7;
 constexpr int kStep = 32;  // reduction columns per step
 constexpr int kDies = 8;
+// Eight neighbouring operands of a row (four, of a unit's activations) are to
+// hold a magnitude of at least this, or zeros alone: the pairs' absolute error
+// of 2^-36 is then at most 2^-21 of their largest. (Weights of spread 0.001
+// and activations of spread 0.05 hold such a group once in 10^13.)
+constexpr float kLeast = 0x1p-15F;
 
 /// 16-byte chunk `chunk` (8 bf16 values) of row `row` of a plane of 64-byte
 /// rows: the equal chunks of 16 consecutive rows (a 16-lane group of a
@@ -207,7 +212,7 @@ struct ProductTile {
   };
   struct Shared {
     Stages stages[KG];
-    int large;
+    int restart;
   };
   static_assert((KG - 1) * sizeof(float) * BM * BN <= KG * sizeof(Stages), "the groups' sums");
 
@@ -299,19 +304,19 @@ struct ProductTile {
           sums[i][j][v] = 0.0F;
   }
 
-  /// The tile from float16 pairs; false (in every thread) when an operand
-  /// passed their range.
+  /// The tile from float16 pairs; false (in every thread) when operands
+  /// lie outside their range.
   template<int SETS>
   __device__ bool Multiply(Sums& acc) {
     float4 values[SETS][kPieces][2];  // steps in flight
     Sums cross;                       // hl + lh, 2048 times their value
     Clear(acc);
     Clear(cross);
-    float most = 0.0F;
+    f16x2::Range range;
     const auto split_piece = [&](int stage, int i, const float4 (&v)[2]) {
       const Octet o = f16x2::Split(v[0], v[1]);
       Store(stage, i, o.h, o.l);
-      most = f16x2::Largest(f16x2::Largest(most, v[0]), v[1]);
+      range.Add(f16x2::Largest(f16x2::Largest(0.0F, v[0]), v[1]));
     };
 #pragma unroll
     for (int set = 0; set < SETS; ++set)
@@ -319,7 +324,7 @@ struct ProductTile {
       for (int i = 0; i < kPieces; ++i)
         Load(first + set, i, values[set][i]);
     if (threadIdx.x == 0)
-      shared.large = 0;
+      shared.restart = 0;
 #pragma unroll
     for (int i = 0; i < kPieces; ++i) {
       split_piece(0, i, values[0][i]);
@@ -362,8 +367,8 @@ struct ProductTile {
         __syncthreads();
       }
     }
-    if (f16x2::TooLarge(most))
-      shared.large = 1;
+    if (!range.Holds(kLeast))
+      shared.restart = 1;
 #pragma unroll
     for (int i = 0; i < kFm; ++i)
 #pragma unroll
@@ -372,7 +377,7 @@ struct ProductTile {
         for (int v = 0; v < 16; ++v)
           acc[i][j][v] = __builtin_fmaf(cross[i][j][v], f16x2::kCross, acc[i][j][v]);
     __syncthreads();
-    return shared.large == 0;
+    return shared.restart == 0;
   }
 
   /// The tile from bfloat16 triples.
@@ -539,7 +544,7 @@ struct UnitTile {
     Planes<kUnitRows> a;
     Planes<C> w;
     float4 window[kWindowRows * 8];  // [rows][8]
-    int large;
+    int restart;
   };
 
   const Unit& u;
@@ -638,10 +643,10 @@ struct UnitTile {
     const int tid = static_cast<int>(threadIdx.x);
     float4 ys[kLoads];
     float4 ws[kPieces][2];
-    float most = 0.0F;
+    f16x2::Range range;
     Clear(acc);
     if (tid == 0)
-      shared.large = 0;
+      shared.restart = 0;
     LoadWindow(0, ys);
 #pragma unroll
     for (int i = 0; i < kPieces; ++i)
@@ -656,7 +661,7 @@ struct UnitTile {
         const Octet o = f16x2::Split(ws[i][0], ws[i][1]);
         if (piece < 4 * C)
           shared.w.Store(piece / 4, piece % 4, o.h, o.l);
-        most = f16x2::Largest(f16x2::Largest(most, ws[i][0]), ws[i][1]);
+        range.Add(f16x2::Largest(f16x2::Largest(0.0F, ws[i][0]), ws[i][1]));
       }
       __syncthreads();
       if (channel + kStep < C) {
@@ -675,7 +680,7 @@ struct UnitTile {
           const f16x2::Pair p0 = f16x2::Split(out[i].x, out[i].y);
           const f16x2::Pair p1 = f16x2::Split(out[i].z, out[i].w);
           StoreItem(i, uint2{p0.h, p1.h}, uint2{p0.l, p1.l});
-          most = f16x2::Largest(most, out[i]);
+          range.Add(f16x2::Largest(0.0F, out[i]));
         }
       }
       __syncthreads();
@@ -703,10 +708,10 @@ struct UnitTile {
           __builtin_amdgcn_sched_barrier(0);
       }
     }
-    if (f16x2::TooLarge(most))
-      shared.large = 1;
+    if (!range.Holds(kLeast))
+      shared.restart = 1;
     __syncthreads();
-    return shared.large == 0;
+    return shared.restart == 0;
   }
 
   /// The unit's product from bfloat16 triples.
