@@ -155,10 +155,11 @@ int vx_stack_set_path(vx_stack* stack, int path);
 int vx_stack_path(const vx_stack* stack, size_t rows);
 
 /* The stack's attention on one layer's cache (the arguments of
- * vx_attention, kernels/generator_kernels.hpp): the keys of each (row, KV
- * head) in chunks of 64 scored by separate workgroups, a second launch
- * merging the chunks' statistics in chunk order when there are several;
- * output bf16 [rows][heads][head_dim]. `partials` holds
+ * vx_attention, kernels/generator_kernels.hpp), on the faster of two kernels:
+ * the keys of each (row, KV head) in chunks of 64 scored by separate
+ * workgroups, a second launch merging the chunks' statistics in chunk order
+ * when there are several; or many rows at a time on the matrix cores. Output
+ * bf16 [rows][heads][head_dim]. `partials` holds
  * vx_split_attention_floats(...) floats (NULL when that is 0). */
 int vx_split_attention(const float* q, const float* k_cache,
                        const float* v_cache, uint16_t* output, size_t rows,
@@ -166,6 +167,15 @@ int vx_split_attention(const float* q, const float* k_cache,
                        size_t past, int causal, size_t heads, size_t kv_heads,
                        size_t head_dim, size_t capacity, float* partials,
                        size_t partial_floats, void* stream);
+/* vx_split_attention on the matrix-core kernel, whichever is the faster:
+ * VX_UNSUPPORTED where it does not take the call (fewer than 32 query heads'
+ * rows per KV head and sequence, pointers not 16-byte aligned). For tests. */
+int vx_tile_attention(const float* q, const float* k_cache,
+                      const float* v_cache, uint16_t* output, size_t rows,
+                      size_t rows_per_sequence, size_t keys_per_sequence,
+                      size_t past, int causal, size_t heads, size_t kv_heads,
+                      size_t head_dim, size_t capacity, float* partials,
+                      size_t partial_floats, void* stream);
 size_t vx_split_attention_floats(size_t rows, size_t heads, size_t head_dim,
                                  size_t past, size_t rows_per_sequence);
 

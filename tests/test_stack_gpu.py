@@ -57,6 +57,22 @@ def test_split_attention_against_oracle(vx, oracle, cuda, stream, heads, kv_head
     assert diff.max() <= 1, f"max {diff.max()} ulp"
 
 
+def tile_attention(q, k_cache, v_cache, rows_per_sequence, keys_per_sequence, past, causal,
+                   heads, kv_heads):
+    """ops.split_attention on the matrix-core kernel, also where the other one
+    is faster."""
+    rows, _, head_dim = q.shape
+    out = torch.empty((rows, heads, head_dim), dtype=torch.bfloat16, device=q.device)
+    floats = _lib.lib().vx_split_attention_floats(rows, heads, head_dim, past, rows_per_sequence)
+    partials = torch.empty(max(floats, 1), dtype=torch.float32, device=q.device)
+    _lib.check(_lib.lib().vx_tile_attention(
+        q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), out.data_ptr(), rows,
+        rows_per_sequence, keys_per_sequence, past, int(causal), heads, kv_heads, head_dim,
+        k_cache.shape[1], partials.data_ptr() if floats else None, floats,
+        torch.cuda.current_stream().cuda_stream))
+    return out
+
+
 @pytest.mark.parametrize("heads,kv_heads,head_dim", [(16, 2, 128), (3, 3, 64), (16, 1, 64)])
 @pytest.mark.parametrize("rows,rps,past,causal,keys", [
     (32, 32, 0, True, None),      # the least rows of one head; a prompt's first rows
@@ -69,8 +85,9 @@ def test_split_attention_against_oracle(vx, oracle, cuda, stream, heads, kv_head
 ])
 def test_tile_attention_against_oracle(vx, oracle, cuda, stream, heads, kv_heads, head_dim,
                                        rows, rps, past, causal, keys):
-    """The matrix-core attention of many rows against the oracle, what lies
-    in the cache past the attended keys (NaN here) unread. The bound: one
+    """The matrix-core attention of many rows, and the kernel that the call
+    takes by itself, against the oracle, what lies in the cache past the
+    attended keys (NaN here) unread. The bound: one
     bf16 ulp (2^-7 of the value), and what float32 sums in another order
     leave of an output near zero: scores up to about 8 round to 2^-21, each
     weight by as much of itself and so the weighted sum by 2^-20 of the
@@ -92,14 +109,15 @@ def test_tile_attention_against_oracle(vx, oracle, cuda, stream, heads, kv_heads
     oracle.lib().vo_attention(oracle.ptr(q), oracle.ptr(kc), oracle.ptr(vc), oracle.ptr(ref),
                               rows, rps, keys, past, int(causal), heads, kv_heads, head_dim,
                               capacity)
-    got = vx.split_attention(dev(q, cuda), dev(kc, cuda), dev(vc, cuda), rps, keys, past,
-                             causal, heads, kv_heads)
-    torch.cuda.synchronize()
-    got, ref = synth.bf16_values(host_bf16(got)), synth.bf16_values(ref)
+    ref = synth.bf16_values(ref)
     bound = 2.0**-7 * np.abs(ref) + 2.0**-20 * np.nanmax(np.abs(vc))
-    worst = float(np.max(np.abs(got - ref) / bound))
-    print(f"worst {worst:.2f} of the bound", flush=True)
-    assert worst <= 1
+    for attend in (tile_attention, vx.split_attention):
+        got = attend(dev(q, cuda), dev(kc, cuda), dev(vc, cuda), rps, keys, past, causal, heads,
+                     kv_heads)
+        torch.cuda.synchronize()
+        worst = float(np.max(np.abs(synth.bf16_values(host_bf16(got)) - ref) / bound))
+        print(f"{attend.__name__}: worst {worst:.2f} of the bound", flush=True)
+        assert worst <= 1
 
 
 def make_stack(vx, oracle, config, seed, bf16_weights=False, positions=2048):
@@ -386,8 +404,8 @@ def test_tile_attention_past_float16(vx, cuda, stream, heads, kv_heads, head_dim
     vc = f32(rng.normal(kv_heads * keys * head_dim).reshape(kv_heads, keys, head_dim))
 
     def attend(q, k, v):
-        got = vx.split_attention(dev(f32(q), cuda), dev(f32(k), cuda), dev(f32(v), cuda), rows,
-                                 rows, past, True, heads, kv_heads)
+        got = tile_attention(dev(f32(q), cuda), dev(f32(k), cuda), dev(f32(v), cuda), rows,
+                             rows, past, True, heads, kv_heads)
         torch.cuda.synchronize()
         return synth.bf16_values(host_bf16(got)).reshape(rows, heads, head_dim)
 
@@ -425,8 +443,8 @@ def test_tile_attention_below_float16(vx, cuda, stream, heads, kv_heads, head_di
     vc = f32(rng.normal(kv_heads * keys * head_dim).reshape(kv_heads, keys, head_dim))
 
     def attend(q, k, v):
-        got = vx.split_attention(dev(f32(q), cuda), dev(f32(k), cuda), dev(f32(v), cuda), rows,
-                                 rows, past, True, heads, kv_heads)
+        got = tile_attention(dev(f32(q), cuda), dev(f32(k), cuda), dev(f32(v), cuda), rows,
+                             rows, past, True, heads, kv_heads)
         torch.cuda.synchronize()
         return synth.bf16_values(host_bf16(got)).reshape(rows, heads, head_dim)
 

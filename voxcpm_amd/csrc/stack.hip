@@ -472,9 +472,11 @@ void Attention(const float* q, const float* k_cache, const float* v_cache, Bf16*
                std::size_t capacity, int splits, const int* past_device, hipStream_t stream) {
   const AttentionShape shape{rows, rows_per_sequence, keys_per_sequence, past, causal,
                              heads, kv_heads, head_dim, capacity};
+  TileAttentionPlan plan;
   if (!fragment && past_device == nullptr &&
-      UseTileAttention(shape, q, k_cache, v_cache, out, partials)) {
-    TileAttention(shape, q, k_cache, v_cache, out, partials, stream);
+      PlanTileAttention(shape, q, k_cache, v_cache, out, partials, &plan) &&
+      UseTileAttention(shape, plan, splits)) {
+    TileAttention(shape, plan, q, k_cache, v_cache, out, partials, stream);
     return;
   }
   AttentionArgs a{};
@@ -1196,11 +1198,18 @@ int vx_stack_path(const vx_stack* stack, size_t rows) {
   return stack == nullptr ? -1 : stack->Resolved(rows);
 }
 
-int vx_split_attention(const float* q, const float* k_cache, const float* v_cache,
-                       uint16_t* output, size_t rows, size_t rows_per_sequence,
-                       size_t keys_per_sequence, size_t past, int causal, size_t heads,
-                       size_t kv_heads, size_t head_dim, size_t capacity, float* partials,
-                       size_t partial_floats, void* stream) {
+}  // extern "C"
+
+namespace {
+
+/// vx_split_attention, or with `tile` the matrix-core kernel whatever its
+/// speed.
+int SplitAttention(const float* q, const float* k_cache, const float* v_cache, Bf16* output,
+                   std::size_t rows, std::size_t rows_per_sequence,
+                   std::size_t keys_per_sequence, std::size_t past, bool causal,
+                   std::size_t heads, std::size_t kv_heads, std::size_t head_dim,
+                   std::size_t capacity, float* partials, std::size_t partial_floats, bool tile,
+                   hipStream_t stream) {
   if (q == nullptr || k_cache == nullptr || v_cache == nullptr || output == nullptr)
     return vx::Fail(VX_BAD_ARG, "vx_split_attention: null pointer");
   if (rows == 0 || rows_per_sequence == 0 || rows % rows_per_sequence != 0)
@@ -1214,10 +1223,43 @@ int vx_split_attention(const float* q, const float* k_cache, const float* v_cach
   if (vx::stack::AttentionPartialFloats(rows, heads, head_dim, splits) > partial_floats ||
       (splits > 1 && partials == nullptr))
     return vx::Fail(VX_BAD_ARG, "vx_split_attention: partials too small");
+  if (tile) {
+    const vx::AttentionShape shape{rows, rows_per_sequence, keys_per_sequence, past, causal,
+                                   heads, kv_heads, head_dim, capacity};
+    vx::TileAttentionPlan plan;
+    if (!vx::PlanTileAttention(shape, q, k_cache, v_cache, output, partials, &plan))
+      return vx::Fail(VX_UNSUPPORTED, "vx_tile_attention: not this shape");
+    vx::TileAttention(shape, plan, q, k_cache, v_cache, output, partials, stream);
+    return vx::LaunchStatus("vx_tile_attention");
+  }
   vx::stack::Attention(q, k_cache, v_cache, output, false, partials, rows, rows_per_sequence,
-                       keys_per_sequence, past, causal != 0, heads, kv_heads, head_dim,
-                       capacity, splits, nullptr, vx::Stream(stream));
+                       keys_per_sequence, past, causal, heads, kv_heads, head_dim, capacity,
+                       splits, nullptr, stream);
   return vx::LaunchStatus("vx_split_attention");
+}
+
+}  // namespace
+
+extern "C" {
+
+int vx_split_attention(const float* q, const float* k_cache, const float* v_cache,
+                       uint16_t* output, size_t rows, size_t rows_per_sequence,
+                       size_t keys_per_sequence, size_t past, int causal, size_t heads,
+                       size_t kv_heads, size_t head_dim, size_t capacity, float* partials,
+                       size_t partial_floats, void* stream) {
+  return SplitAttention(q, k_cache, v_cache, output, rows, rows_per_sequence, keys_per_sequence,
+                        past, causal != 0, heads, kv_heads, head_dim, capacity, partials,
+                        partial_floats, false, vx::Stream(stream));
+}
+
+int vx_tile_attention(const float* q, const float* k_cache, const float* v_cache,
+                      uint16_t* output, size_t rows, size_t rows_per_sequence,
+                      size_t keys_per_sequence, size_t past, int causal, size_t heads,
+                      size_t kv_heads, size_t head_dim, size_t capacity, float* partials,
+                      size_t partial_floats, void* stream) {
+  return SplitAttention(q, k_cache, v_cache, output, rows, rows_per_sequence, keys_per_sequence,
+                        past, causal != 0, heads, kv_heads, head_dim, capacity, partials,
+                        partial_floats, true, vx::Stream(stream));
 }
 
 size_t vx_split_attention_floats(size_t rows, size_t heads, size_t head_dim, size_t past,

@@ -543,49 +543,77 @@ bool Aligned16(const void* p) { return reinterpret_cast<std::uintptr_t>(p) % 16 
 
 }  // namespace
 
-bool UseTileAttention(const AttentionShape& s, const float* q, const float* k_cache,
-                      const float* v_cache, const Bf16* out, const float* partials) {
+bool PlanTileAttention(const AttentionShape& s, const float* q, const float* k_cache,
+                       const float* v_cache, const Bf16* out, const float* partials,
+                       TileAttentionPlan* plan) {
   const std::size_t group = s.heads / s.kv_heads;
   // The kernel's indices are 32-bit; the caches are read in 16-byte pieces.
-  return s.rows_per_sequence * group >= 32 && s.rows * s.heads < (std::size_t{1} << 24) &&
-         s.past + s.rows_per_sequence < (std::size_t{1} << 21) && Aligned16(q) &&
-         Aligned16(k_cache) && Aligned16(v_cache) && Aligned16(out) && Aligned16(partials);
-}
-
-void TileAttention(const AttentionShape& s, const float* q, const float* k_cache,
-                   const float* v_cache, Bf16* out, float* partials, hipStream_t stream) {
-  const std::size_t group = s.heads / s.kv_heads;
-  const std::size_t sequences = s.rows / s.rows_per_sequence;
+  if (s.rows_per_sequence * group < 32 || s.rows * s.heads >= (std::size_t{1} << 24) ||
+      s.past + s.rows_per_sequence >= (std::size_t{1} << 21) || !Aligned16(q) ||
+      !Aligned16(k_cache) || !Aligned16(v_cache) || !Aligned16(out) || !Aligned16(partials))
+    return false;
   const std::size_t queries = s.rows_per_sequence * group;
   const std::size_t blocks = (queries + kQueries - 1) / kQueries;
+  const std::size_t heads = s.rows / s.rows_per_sequence * s.kv_heads;
   const auto keys_of = [&](std::size_t block) {
     const std::size_t last = std::min((block + 1) * kQueries, queries) - 1;
     return s.past + (s.causal ? last / group + 1 : s.rows_per_sequence);
   };
+  const auto runs_of = [&](std::size_t chunk) {
+    std::size_t runs = 0;
+    for (std::size_t b = 0; b < blocks; ++b)
+      runs += (keys_of(b) + chunk - 1) / chunk;
+    return runs * heads;
+  };
   // The least chunk that cuts all query blocks' keys into at most
   // kTargetWorkgroups runs (or leaves them whole).
-  const std::size_t heads = sequences * s.kv_heads;
   std::size_t steps = 0;
   for (std::size_t b = 0; b < blocks; ++b)
     steps += (keys_of(b) + kKeys - 1) / kKeys;
   const std::size_t most = s.past + s.rows_per_sequence;
   std::size_t chunk = std::max<std::size_t>(
       kLeastChunk, (steps * heads + kTargetWorkgroups - 1) / kTargetWorkgroups * kKeys);
-  for (; chunk < most; chunk += kKeys) {
-    std::size_t runs = 0;
-    for (std::size_t b = 0; b < blocks; ++b)
-      runs += (keys_of(b) + chunk - 1) / chunk;
-    if (runs * heads <= kTargetWorkgroups)
-      break;
-  }
-  const std::size_t splits = (most + chunk - 1) / chunk;
+  while (chunk < most && runs_of(chunk) > kTargetWorkgroups)
+    chunk += kKeys;
+  plan->chunk = chunk;
+  plan->splits = (most + chunk - 1) / chunk;
+  plan->workgroups = plan->splits == 1 ? blocks * heads : runs_of(chunk);
+  return true;
+}
+
+bool UseTileAttention(const AttentionShape& s, const TileAttentionPlan& plan, int splits) {
+  // Both kernels' times in microseconds, fitted to MI355X over rows 4..192,
+  // keys 2..4192, groups 1..16 and head_dim 64 and 128 (592 points, replayed
+  // from a graph): a workgroup's steps of 32 keys here, the workgroups' rounds
+  // there, and a merge each. With the rule's choice none of them takes more
+  // than 4 % longer than on the split kernel, and on average 0.3 % longer than
+  // on the faster of the two. 4 rows of 16 heads over 254 keys 7.6 us there,
+  // 16.4 here; 16 over 716 16.2 and 19.5; 64 over 314 22.8 and 19.6; 128 over
+  // 828 81.7 and 23.1; 40 patches of 5 rows 13.2 and 6.9.
+  const bool wide = s.head_dim > 64;
+  const std::size_t keys = std::min(plan.chunk, s.past + s.rows_per_sequence);
+  const double steps = static_cast<double>((keys + kKeys - 1) / kKeys);
+  const double here = 4.6 + steps * (wide ? 2.85 : 1.75) + (plan.splits > 1 ? 4.7 : 0.0);
+  const double group =
+      static_cast<double>(std::max<std::size_t>(2, s.heads / s.kv_heads));  // one costs as two
+  const double there = 3.2 + (splits > 1 ? 3.0 : 0.0) +
+                       static_cast<double>(s.rows * s.kv_heads) * splits * group *
+                           (wide ? 2.4e-3 : 1.0e-3);
+  return here < there;
+}
+
+void TileAttention(const AttentionShape& s, const TileAttentionPlan& plan, const float* q,
+                   const float* k_cache, const float* v_cache, Bf16* out, float* partials,
+                   hipStream_t stream) {
+  const std::size_t group = s.heads / s.kv_heads;
+  const std::size_t queries = s.rows_per_sequence * group;
   TileArgs args{};
   args.q = q;
   args.k = k_cache;
   args.v = v_cache;
   args.out = out;
   args.values = partials;
-  args.stats = partials == nullptr ? nullptr : partials + s.rows * s.heads * splits * s.head_dim;
+  args.stats = partials == nullptr ? nullptr : partials + s.rows * s.heads * plan.splits * s.head_dim;
   args.rows_per_sequence = static_cast<int>(s.rows_per_sequence);
   args.keys_per_sequence = static_cast<int>(s.keys_per_sequence);
   args.past = static_cast<int>(s.past);
@@ -593,19 +621,16 @@ void TileAttention(const AttentionShape& s, const float* q, const float* k_cache
   args.heads = static_cast<int>(s.heads);
   args.kv_heads = static_cast<int>(s.kv_heads);
   args.capacity = static_cast<int>(s.capacity);
-  args.sequences = static_cast<int>(sequences);
-  args.blocks = static_cast<int>(blocks);
-  args.chunk = static_cast<int>(chunk);
-  args.splits = static_cast<int>(splits);
+  args.sequences = static_cast<int>(s.rows / s.rows_per_sequence);
+  args.blocks = static_cast<int>((queries + kQueries - 1) / kQueries);
+  args.chunk = static_cast<int>(plan.chunk);
+  args.splits = static_cast<int>(plan.splits);
   args.scale = 1.0F / std::sqrt(static_cast<float>(s.head_dim));
-  std::size_t workgroups = 0;
-  for (std::size_t b = 0; b < blocks; ++b)
-    workgroups += splits == 1 ? heads : (keys_of(b) + chunk - 1) / chunk * heads;
   const std::size_t items = s.rows * s.heads;
   if (s.head_dim == 64)
-    Launch<64>(args, workgroups, items, stream);
+    Launch<64>(args, plan.workgroups, items, stream);
   else
-    Launch<128>(args, workgroups, items, stream);
+    Launch<128>(args, plan.workgroups, items, stream);
 }
 
 }  // namespace vx

@@ -19,15 +19,28 @@ struct AttentionShape {
   std::size_t heads, kv_heads, head_dim, capacity;
 };
 
+/// How the matrix-core attention cuts a call's keys.
+struct TileAttentionPlan {
+  std::size_t chunk = 0;       // keys per chunk
+  std::size_t splits = 1;      // chunks of the rows that attend to the most keys
+  std::size_t workgroups = 0;  // of the first launch
+};
+
 /// Whether the matrix-core attention takes these pointers and this shape,
-/// and is the faster kernel for it.
-bool UseTileAttention(const AttentionShape& s, const float* q, const float* k_cache,
-                      const float* v_cache, const Bf16* out, const float* partials);
+/// and how.
+bool PlanTileAttention(const AttentionShape& s, const float* q, const float* k_cache,
+                       const float* v_cache, const Bf16* out, const float* partials,
+                       TileAttentionPlan* plan);
+
+/// Whether it is the faster kernel for them: not the split kernel, `splits`
+/// chunks of whose keys a workgroup each takes.
+bool UseTileAttention(const AttentionShape& s, const TileAttentionPlan& plan, int splits);
 
 /// `partials`: rows x heads x ceil(keys / 64) x (head_dim + 2) floats, or
 /// null where a row attends to at most 64 keys.
-void TileAttention(const AttentionShape& s, const float* q, const float* k_cache,
-                   const float* v_cache, Bf16* out, float* partials, hipStream_t stream);
+void TileAttention(const AttentionShape& s, const TileAttentionPlan& plan, const float* q,
+                   const float* k_cache, const float* v_cache, Bf16* out, float* partials,
+                   hipStream_t stream);
 
 }  // namespace vx
 
