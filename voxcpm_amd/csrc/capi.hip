@@ -116,7 +116,7 @@ int Product(const uint16_t* x, const void* packed, float* y, uint16_t* y_bf16,
             vx::q8::Weights kind = vx::q8::Weights::kQ8) {
   const bool exact = kind == vx::q8::Weights::kQ8 && rg == 0 && waves == 0 && splits == 0 &&
                      vx::prefill::UseExact(m, k, n);
-  if (exact || vx::prefill::Use(m, k, n)) {
+  if (exact || vx::prefill::Use(m, k, n, kind == vx::q8::Weights::kQ8)) {
     vx::prefill::Product p;
     p.x = x;
     p.w = packed;
@@ -371,7 +371,7 @@ int vx_q8_prefill_plan(size_t m, size_t k, size_t n, vx_scratch* scratch, int32_
   if (out4 == nullptr || m <= vx::kExactRows || k % 32 != 0 || k == 0 || n == 0)
     return vx::Fail(VX_BAD_ARG, "vx_q8_prefill_plan: bad arguments");
   const std::size_t floats = scratch != nullptr ? scratch->partial_floats : 0;
-  if (vx::prefill::Use(m, k, n)) {
+  if (vx::prefill::Use(m, k, n, true)) {
     const vx::prefill::Shape shape = vx::prefill::ShapeOf(vx::prefill::PickShape(m, k, n));
     out4[0] = 3;
     out4[1] = shape.bm;

@@ -699,19 +699,55 @@ int PickShape(std::size_t m, std::size_t k, std::size_t n, double* microseconds)
   return best;
 }
 
-bool Use(std::size_t m, std::size_t k, std::size_t n) {
-  // Up to 512 rows over 6144 columns of k and more stay on the kernels whose
-  // split over k uses a scratch: that split is part of what the static
-  // scratch entry promises at those sizes (300 x 6144 x 2048 takes 31.6 us
-  // there, 20.7 us here; the stacks, which use no scratch, come here).
-  if (m <= kExactRows || !Supported(m, k, n) || (k >= 6144 && m <= 512))
+bool Use(std::size_t m, std::size_t k, std::size_t n, bool q8) {
+  // Q8_0 products of up to 512 rows over 6144 columns of k and more stay on the
+  // kernels whose split over k uses a scratch: a caller's, or the static one of
+  // the entry that cannot allocate, whose use at 300 and 320 x 6144 x 2048 the
+  // tests hold fast. These kernels would be the faster ones there too (300 x
+  // 6144 x 2048 31.6 us there, 20.7 here; 129 x 18.1 and 14.7; 512 x 6144 x 4096
+  // 59.3 and 35.6). bf16 panels have no such entry, and the stacks, which use no
+  // scratch, come here.
+  if (m <= kExactRows || !Supported(m, k, n) || (q8 && k >= 6144 && m <= 512))
     return false;
-  // Against the 256 x 256 tiles of q8_gemm.hip by the same model (3 us, 1.5
-  // a step).
+  // Else by both sides' times in microseconds, fitted on MI355X (drawn and
+  // gridded sizes, both weight formats, replayed from a graph).
   double here = 0.0;
-  PickShape(m, k, n, &here);
-  return !UseGemm(m, n) ||
-         here <= Rounds(m, n, 256, 256) * (3.0 + 1.5 * static_cast<double>(q8::Pairs(k)));
+  const int shape = PickShape(m, k, n, &here);
+  const double pairs = static_cast<double>(q8::Pairs(k));
+  if (UseRowBlocks(m, k, n, q8)) {
+    // 2940 sizes, m 129..1500, k 64..6144, n 64..16384: on average 0.4 %
+    // slower than the faster kernel, and one in 130 over 4 % slower than in row
+    // blocks. 129 x 256 x 1024 3.7 us there, 6.4 here; 256 x 1024 x 1024 4.8 and
+    // 6.0; 512 x 544 x 2055 12.5 and 8.9; 448 x 1536 x 2560 16.4 and 11.5.
+    const double output = static_cast<double>(m) * static_cast<double>(n) * 1e-6;  // its writing
+    const std::size_t blocks = (m + 63) / 64;
+    const std::size_t groups = q8::Groups(n);
+    const std::size_t wide = groups <= 256 ? 1 : 2;  // row groups per workgroup
+    const std::size_t tiles = (groups + wide - 1) / wide;
+    const double rounds =
+        static_cast<double>((blocks * tiles + kComputeUnits - 1) / kComputeUnits * wide);
+    const double passes = static_cast<double>((q8::Pairs(k) + 15) / 16);  // of 16 waves
+    // A tile's blocks share a die, and its L2, where tiles are whole eights.
+    const double pair = tiles % kDies == 0 ? 0.064 : 0.079;
+    // The workgroups' rounds, or the rows' reading by few tiles.
+    const double there =
+        std::max(2.7 + 0.41 * passes + rounds * (0.21 + pair * pairs) + 2.5 * output,
+                 2.7 + 0.0083 * static_cast<double>(blocks) * pairs);
+    return 2.0 + 0.78 * here + 0.85 * output < there;
+  }
+  if (!UseGemm(m, n))  // the tiled kernel, slower wherever it was measured
+    return true;
+  // 966 sizes, m 384..3000, k 64..6144, n 6144..24576: on average 0.5 % slower
+  // than the faster kernel, and one in 60 over 4 % slower than the 256-row tiles.
+  // A full grid's later rounds take longer than the first (128 x 128 tiles a
+  // fifth, the others a tenth from the third on). bf16 1024 x 2048 x 12288 56 us
+  // there, 64 here; 777 x 2048 x 12288 56 and 41.
+  const Shape tile = ShapeOf(shape);
+  const double mine = Rounds(m, n, tile.bm, tile.bn);
+  here *= tile.bn == 128 ? (mine > 1.0 ? 1.2 : 1.0) : (mine > 2.0 ? 1.1 : 1.0);
+  const GemmPlan plan = PlanGemm(m, k, n, 0);
+  return here <=
+         Rounds(m, n, plan.bm, plan.bn) * (3.0 + (plan.bn == 256 ? 1.5 : 0.95) * pairs);
 }
 
 void Scale(const float* h, const Norm& norm, std::size_t m, std::size_t width,

@@ -71,8 +71,9 @@ constexpr int kShapes = 7;
 Shape ShapeOf(int shape);
 /// The shape an m x k x n product takes, and its modelled time.
 int PickShape(std::size_t m, std::size_t k, std::size_t n, double* microseconds = nullptr);
-/// Whether the standalone products of more than 128 rows take these kernels.
-bool Use(std::size_t m, std::size_t k, std::size_t n);
+/// Whether a standalone product of more than 128 rows takes these kernels
+/// (`q8`: Q8_0 panels, else bf16 panels).
+bool Use(std::size_t m, std::size_t k, std::size_t n, bool q8);
 /// Whether an m x k x n product of Q8_0 panels with the exact per-block
 /// arithmetic (33 to 128 rows) takes RunExact rather than the engine.
 bool UseExact(std::size_t m, std::size_t k, std::size_t n);

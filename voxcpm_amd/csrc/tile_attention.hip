@@ -582,7 +582,7 @@ bool PlanTileAttention(const AttentionShape& s, const float* q, const float* k_c
 }
 
 bool UseTileAttention(const AttentionShape& s, const TileAttentionPlan& plan, int splits) {
-  // Both kernels' times in microseconds, fitted to MI355X over rows 4..192,
+  // Both kernels' times in microseconds, fitted to MI355X over rows 4..6000,
   // keys 2..4192, groups 1..16 and head_dim 64 and 128 (592 points, replayed
   // from a graph): a workgroup's steps of 32 keys here, the workgroups' rounds
   // there, and a merge each. With the rule's choice none of them takes more
