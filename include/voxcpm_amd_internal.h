@@ -56,7 +56,9 @@ int vx_bf16_linear_gemm(const uint16_t* x, const void* packed, float* y,
 
 /* The default plan of an m x k x n product (m <= 128):
  * out7 = {activation tiles, row groups per workgroup, waves per workgroup,
- * workgroup tiles, splits, pairs per split, pairs per wave}. Counterpart of
+ * workgroup tiles, splits, pairs per split, pairs per wave}, of the engine or
+ * of the panel-operand kernels' exact tiles (two activation tiles by two row
+ * groups, sixteen waves along k). Counterpart of
  * PlanWmma (kernels/wmma_products.hpp:82-85). */
 int vx_q8_plan(size_t m, size_t k, size_t n, vx_scratch* scratch,
                int32_t* out7);
@@ -176,6 +178,12 @@ int vx_tile_attention(const float* q, const float* k_cache,
                       size_t past, int causal, size_t heads, size_t kv_heads,
                       size_t head_dim, size_t capacity, float* partials,
                       size_t partial_floats, void* stream);
+/* The kernel of such a call (16-byte aligned pointers): out3 = {1 the
+ * matrix-core kernel, else 0; keys per chunk; chunks of the rows that attend to
+ * the most keys}. */
+int vx_split_attention_plan(size_t rows, size_t rows_per_sequence, size_t past,
+                            int causal, size_t heads, size_t kv_heads,
+                            size_t head_dim, int32_t* out3);
 size_t vx_split_attention_floats(size_t rows, size_t heads, size_t head_dim,
                                  size_t past, size_t rows_per_sequence);
 

@@ -87,6 +87,43 @@ def test_packed_bytes():
     assert L.vx_q8_packed_bytes(17, 96) == 2 * 2 * 1088
 
 
+# Sizes on whose kernel both sides' measured times leave no doubt (a quarter
+# and more between them): 0 the tiled kernel, 1 the 256-row tiles, 2 blocks of 64
+# rows, 3 the panel-operand kernels.
+@pytest.mark.parametrize("m,k,n,kernel", [
+    (129, 256, 1024, 2), (200, 512, 512, 2), (256, 1024, 1024, 2), (129, 4096, 130, 2),
+    (448, 1536, 2560, 3), (512, 544, 2055, 3), (310, 2048, 2560, 3), (777, 2048, 12288, 3)])
+def test_prefill_plan_takes_the_faster_kernel(m, k, n, kernel):
+    plan = (ctypes.c_int32 * 4)()
+    assert lib().vx_q8_prefill_plan(m, k, n, None, plan) == VX_OK
+    assert plan[0] == kernel, list(plan)
+
+
+# The same for the attention: 1 the matrix-core kernel, 0 chunks of 64 keys.
+@pytest.mark.parametrize("rows,per_sequence,past,causal,heads,kv_heads,head_dim,tile", [
+    (4, 4, 250, 1, 16, 2, 128, 0), (16, 16, 700, 1, 16, 2, 128, 0), (5, 5, 0, 0, 16, 2, 128, 0),
+    (64, 64, 60, 1, 16, 2, 128, 0), (32, 32, 0, 1, 16, 16, 64, 0), (24, 24, 250, 1, 8, 1, 128, 0),
+    (300, 300, 1500, 1, 16, 2, 128, 1), (310, 5, 0, 0, 16, 2, 128, 1),
+    (64, 64, 700, 1, 16, 2, 128, 1), (64, 64, 1000, 1, 16, 16, 64, 1)])
+def test_attention_plan_takes_the_faster_kernel(rows, per_sequence, past, causal, heads, kv_heads,
+                                                head_dim, tile):
+    plan = (ctypes.c_int32 * 3)()
+    assert lib().vx_split_attention_plan(rows, per_sequence, past, causal, heads, kv_heads,
+                                         head_dim, plan) == VX_OK
+    assert plan[0] == tile, list(plan)
+    assert plan[1] * plan[2] >= past + per_sequence > plan[1] * (plan[2] - 1)
+
+
+def test_q8_plan_of_exact_tiles():
+    """Sizes that take the panel-operand kernels' exact tiles report those, not
+    the engine's plan: 32 x 32 tiles, sixteen waves along k."""
+    plan = (ctypes.c_int32 * 7)()
+    assert lib().vx_q8_plan(77, 6144, 2055, None, plan) == VX_OK
+    assert list(plan) == [2, 2, 16, 3 * 65, 1, 96, 6]
+    assert lib().vx_q8_plan(100, 4128, 40, None, plan) == VX_OK
+    assert list(plan) == [2, 2, 16, 4 * 2, 1, 65, 5]
+
+
 @pytest.mark.parametrize("steps,sway,skip", [(10, 1.0, True), (10, 0.0, False),
                                              (1, 1.0, True), (25, 0.5, True),
                                              (64, 1.0, False)])

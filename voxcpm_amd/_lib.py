@@ -186,6 +186,7 @@ _SIGNATURES = {
                            + [c_void_p, c_size, c_void_p], c_int),
     "vx_tile_attention": ([c_void_p] * 4 + [c_size] * 4 + [c_int] + [c_size] * 4
                            + [c_void_p, c_size, c_void_p], c_int),
+    "vx_split_attention_plan": ([c_size] * 3 + [c_int] + [c_size] * 3 + [c_void_p], c_int),
     "vx_split_attention_floats": ([c_size] * 5, c_size),
     "vx_gguf_open": ([ctypes.c_char_p, c_int, ctypes.POINTER(c_void_p)], c_int),
     "vx_gguf_close": ([c_void_p], None),

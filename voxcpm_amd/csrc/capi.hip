@@ -354,6 +354,18 @@ int vx_q8_plan(size_t m, size_t k, size_t n, vx_scratch* scratch,
   if (out7 == nullptr || m == 0 || m > vx::kExactRows || k % 32 != 0 ||
       k == 0 || n == 0)
     return vx::Fail(VX_BAD_ARG, "vx_q8_plan: bad arguments");
+  if (vx::prefill::UseExact(m, k, n)) {
+    const vx::prefill::Shape shape = vx::prefill::ExactShape();
+    const int pairs = static_cast<int>(vx::q8::Pairs(k));
+    out7[0] = shape.bm / 16;
+    out7[1] = shape.bn / 16;
+    out7[2] = shape.groups;  // a wave each
+    out7[3] = static_cast<int32_t>((m + shape.bm - 1) / shape.bm * ((n + shape.bn - 1) / shape.bn));
+    out7[4] = 1;
+    out7[5] = pairs;
+    out7[6] = (pairs + shape.groups - 1) / shape.groups;
+    return vx::Succeed();
+  }
   const vx::ProductPlan plan = vx::PlanSkinny(
       m, k, n, scratch != nullptr ? scratch->partial_floats : 0,
       scratch != nullptr ? scratch->counter_count : 0);

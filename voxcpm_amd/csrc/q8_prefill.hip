@@ -673,6 +673,8 @@ double Rounds(std::size_t m, std::size_t n, int bm, int bn) {
 
 Shape ShapeOf(int shape) { return kModels[shape].shape; }
 
+Shape ExactShape() { return Shape{ExactTile::kBm, ExactTile::kColumns, ExactTile::kKg}; }
+
 bool Supported(std::size_t m, std::size_t k, std::size_t n) {
   // The output tile, the activations and a column tile's panels as buffers
   // of 32-bit offsets.

@@ -1262,6 +1262,26 @@ int vx_tile_attention(const float* q, const float* k_cache, const float* v_cache
                         partial_floats, true, vx::Stream(stream));
 }
 
+int vx_split_attention_plan(size_t rows, size_t rows_per_sequence, size_t past, int causal,
+                            size_t heads, size_t kv_heads, size_t head_dim, int32_t* out3) {
+  if (out3 == nullptr || rows == 0 || rows_per_sequence == 0 || rows % rows_per_sequence != 0)
+    return vx::Fail(VX_BAD_ARG, "vx_split_attention_plan: bad arguments");
+  if (!vx::stack::AttentionSupported(heads, kv_heads, head_dim))
+    return vx::Fail(VX_UNSUPPORTED, "vx_split_attention_plan: unsupported heads or head_dim");
+  const vx::AttentionShape shape{rows, rows_per_sequence, past + rows_per_sequence, past,
+                                 causal != 0, heads, kv_heads, head_dim,
+                                 past + rows_per_sequence};
+  const int splits = vx::stack::AttentionSplits(past, rows_per_sequence);
+  vx::TileAttentionPlan plan;
+  const bool tile =
+      vx::PlanTileAttention(shape, nullptr, nullptr, nullptr, nullptr, nullptr, &plan) &&
+      vx::UseTileAttention(shape, plan, splits);
+  out3[0] = tile ? 1 : 0;
+  out3[1] = tile ? static_cast<int32_t>(plan.chunk) : static_cast<int32_t>(vx::stack::kChunk);
+  out3[2] = tile ? static_cast<int32_t>(plan.splits) : splits;
+  return vx::Succeed();
+}
+
 size_t vx_split_attention_floats(size_t rows, size_t heads, size_t head_dim, size_t past,
                                  size_t rows_per_sequence) {
   if (rows_per_sequence == 0)
