@@ -392,12 +392,18 @@ def test_panel_operand_shapes(vx, oracle, cuda, stream, shape, weights, rows, k,
     assert worst <= LIMIT, worst
 
 
-@pytest.mark.parametrize("rows", [65, 77, 128])
-@pytest.mark.parametrize("k,n", [(6144, 2055), (4192, 70)])
+@pytest.mark.parametrize("rows,k,n", [(65, 6144, 2055), (77, 6144, 2055), (128, 6144, 2040),
+                                      (65, 4192, 70), (77, 4192, 70), (128, 4192, 70),
+                                      # up to 64 rows: more than 2048 columns
+                                      (33, 4128, 2055), (64, 6144, 2055),
+                                      # the tiles would take a second round: the engine
+                                      (128, 6144, 2055)])
 def test_exact_long_reductions(vx, oracle, cuda, stream, rows, k, n):
-    """65 to 128 rows over more than 4096 columns of k take the panel-operand
+    """33 to 128 rows over more than 4096 columns of k take the panel-operand
     kernels with the exact per-block arithmetic: rows, columns and an odd
     block count that end inside a tile, accumulation and bf16 results."""
+    plan = vx.q8_plan(rows, k, n)
+    assert (plan["mt"] == 2 and plan["rg"] == 2) == ((rows, n) != (128, 2055)), plan
     rng = synth.Rng(12, rows + n)
     blocks = synth.q8_blocks(rng, n, k)
     packed = vx.q8_pack(to_device(blocks, cuda), n, k)

@@ -783,17 +783,18 @@ Args ArgsOf(const Product& p) {
 }  // namespace
 
 bool UseExact(std::size_t m, std::size_t k, std::size_t n) {
-  // Past 64 rows the engine needs a second block of rows, and its 16-column
-  // workgroups each read all of x: over more than 4096 columns of k these
-  // tiles are faster while they take one round (77 x 6144 x 2055 19.1 ->
-  // 11.5 us, 100 x 6144 x 1024 12.5 -> 10.7, 128 x 8192 x 2048 18.4 -> 14.5,
-  // 65 x 5120 x 130 10.3 -> 9.6, 77 x 4128 x 2048 10.4 -> 10.2 on MI355X, with
-  // the call). In one block the engine is the faster one (49 x 6144 x 2048
-  // 10.2 there, 10.8 here; 49 x 8192 x 70 8.6 and 12.1). Over shorter k its
-  // sums come out closer to 64 bits (100 x 1024 x 1024 7.0e-8 there, 8.3e-8
-  // here; 77 x 6144 x 2048 1.06e-7 and 1.01e-7).
-  return m > 64 && m <= kExactRows && k > 4096 && Supported(m, k, n) &&
-         ((m + 31) / 32) * ((n + 31) / 32) <= kComputeUnits;
+  // Past 64 rows the engine needs a second block of rows, and past 32 rows over
+  // more than 128 row groups a second round of workgroups, each of which reads
+  // all of its block's x: over more than 4096 columns of k these tiles are faster
+  // there while they take one round (77 x 6144 x 2055 19.1 -> 11.5 us, 128 x 8192 x
+  // 2048 18.4 -> 14.5, 65 x 5120 x 130 10.3 -> 9.6, 77 x 4128 x 2048 10.4 -> 10.2, 33 x
+  // 6144 x 2049 12.5 -> 10.7, 64 x 5120 x 4096 15.5 -> 10.9 on MI355X). Below, the
+  // engine is (64 x 6144 x 2048 10.3 there, 11.0 here; 48 x 8192 x 1024 10.8 and
+  // 12.1; 32 x 6144 x 4000 9.6 and 11.8). Over shorter k its sums come out
+  // closer to 64 bits (100 x 1024 x 1024 7.0e-8 there, 8.3e-8 here; 77 x 6144 x 2048
+  // 1.06e-7 and 1.01e-7, 40 x 4128 x 2560 9.4e-8 and 9.2e-8).
+  return (m > 64 || (m > 32 && n > 2048)) && m <= kExactRows && k > 4096 &&
+         Supported(m, k, n) && ((m + 31) / 32) * ((n + 31) / 32) <= kComputeUnits;
 }
 
 int RunExact(const Product& p, hipStream_t stream) {

@@ -75,7 +75,7 @@ int PickShape(std::size_t m, std::size_t k, std::size_t n, double* microseconds 
 /// (`q8`: Q8_0 panels, else bf16 panels).
 bool Use(std::size_t m, std::size_t k, std::size_t n, bool q8);
 /// Whether an m x k x n product of Q8_0 panels with the exact per-block
-/// arithmetic (65 to 128 rows) takes RunExact rather than the engine.
+/// arithmetic (33 to 128 rows) takes RunExact rather than the engine.
 bool UseExact(std::size_t m, std::size_t k, std::size_t n);
 /// The product with each 32-column block's float32 sum scaled into the row's
 /// (kernels/wmma_products.hip:192-215): kStore, kAccumulate or kBf16.
