@@ -841,6 +841,13 @@ void RunProduct(const Product& p, hipStream_t stream) {
     // A die re-reads the operand that its tiles do not share: the smaller.
     return ProductArgs{p, (p.t + m - 1) / m, (p.n + n - 1) / n, p.n >= p.t ? 1 : 0};
   };
+  // 128 x 128 tiles, k in two groups of waves while they are fewer than one and a
+  // half for each compute unit; 64 x 64 with four groups where even two would
+  // leave half of the units idle. Lower lines are faster and less exact (a
+  // group's sums are the shorter the more groups): with 256 and 128 tiles 72
+  // frames decode in 647 us on MI355X instead of 736, 96 in 708 instead of 824, 40
+  // in 493 instead of 574 (16, 64 and 125 the same), with an error against 64 bits
+  // of 1.79e-5 instead of 1.69e-5 at 96.
   const unsigned big = tiles(128, 128);
   if (big >= 384)
     ProductKernel<128, 128, 1><<<big, kThreads, 0, stream>>>(args(128, 128));
