@@ -606,9 +606,10 @@ __global__ void ScaleKernel(const float* h, Norm norm, int m, int width) {
 }
 
 /// The caches' epilogue over 160-row tiles does not unroll (its sums would
-/// lie in memory): Run picks another shape.
+/// lie in memory): PickShape leaves them out.
+constexpr int kNoQkvRows = 160;
 template<class T>
-constexpr bool kTakesQkv = T::kBm != 160;
+constexpr bool kTakesQkv = T::kBm != kNoQkvRows;
 
 template<class T>
 void Launch(const Product& p, Args a, hipStream_t stream) {
@@ -682,11 +683,13 @@ bool Supported(std::size_t m, std::size_t k, std::size_t n) {
          q8::Bf16PackedBytes(n, k) < (std::size_t{1} << 31);
 }
 
-int PickShape(std::size_t m, std::size_t k, std::size_t n, double* microseconds) {
+int PickShape(std::size_t m, std::size_t k, std::size_t n, double* microseconds, Out kind) {
   int best = 0;
   double least = 0.0;
   for (int i = 0; i < kShapes; ++i) {
     const Model& model = kModels[i];
+    if (kind == Out::kQkvCache && model.shape.bm == kNoQkvRows)
+      continue;
     const std::size_t groups = static_cast<std::size_t>(model.shape.groups);
     const double steps = static_cast<double>((q8::Pairs(k) + groups - 1) / groups);
     const double time = Rounds(m, n, model.shape.bm, model.shape.bn) *
@@ -816,9 +819,7 @@ int RunExact(const Product& p, hipStream_t stream) {
 int Run(const Product& p, hipStream_t stream, int shape) {
   const Args a = ArgsOf(p);
   if (shape < 0)
-    shape = PickShape(p.m, p.k, p.n);
-  if (p.kind == Out::kQkvCache && ShapeOf(shape).bm == 160)
-    shape = 0;
+    shape = PickShape(p.m, p.k, p.n, nullptr, p.kind);
   switch (shape) {
     case 0: Launch<Tile<128, 2, 4, 1, 4>>(p, a, stream); break;
     case 1: Launch<Tile<128, 1, 4, 2, 4>>(p, a, stream); break;

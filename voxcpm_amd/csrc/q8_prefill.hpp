@@ -70,7 +70,8 @@ struct Shape {
 constexpr int kShapes = 7;
 Shape ShapeOf(int shape);
 /// The shape an m x k x n product takes, and its modelled time.
-int PickShape(std::size_t m, std::size_t k, std::size_t n, double* microseconds = nullptr);
+int PickShape(std::size_t m, std::size_t k, std::size_t n, double* microseconds = nullptr,
+              Out kind = Out::kStore);
 /// Whether a standalone product of more than 128 rows takes these kernels
 /// (`q8`: Q8_0 panels, else bf16 panels).
 bool Use(std::size_t m, std::size_t k, std::size_t n, bool q8);
@@ -85,7 +86,8 @@ Shape ExactShape();
 void Scale(const float* h, const Norm& norm, std::size_t m, std::size_t width,
            hipStream_t stream);
 /// Launches the product (arguments checked by the caller: CheckProduct; k a
-/// multiple of 32, and n where the norm or SwiGLU take part). A non-negative `shape` forces that one.
+/// multiple of 32, and n where the norm or SwiGLU take part). A non-negative `shape` forces that one
+/// (not the 160-row tiles for kQkvCache).
 int Run(const Product& p, hipStream_t stream, int shape = -1);
 
 }  // namespace vx::prefill
