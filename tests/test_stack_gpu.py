@@ -254,8 +254,12 @@ def test_stack_bf16_weights(vx, oracle, cuda, stream):
     run.step(h, [5], [5], 1, 1, 5, True, "bf16 decode")
 
 
-# The VoxCPM2 layers give gate_up the wide tiles (128 x 256 at 400 rows, 128 x
-# 128 in two groups at 310), the small ones the tiles of four and eight groups.
+# The products' tiles. gate_up: the base LM's 96 x 256 at 400 rows, 128 x 256 at
+# 500, 160 x 256 at 650, the encoder's 128 x 128 in two groups of k. qkv: the
+# encoder's 64 x 64 in eight groups at 310 rows, 128 x 128 in two at 390, the base
+# LM's 64 x 128 in four. o and down: 32 x 64 (encoder) and 64 x 64 (base LM) in
+# eight groups, 64 x 128 in four at 650. The small layers: 128 x 128 in two groups,
+# and 32 x 64 for down.
 PROMPTS = {"gqa-hd64": STACKS["gqa-hd64"], "no-rope-hd128": STACKS["no-rope-hd128"],
            "voxcpm2-encoder": synth.StackConfig(hidden=1024, ffn=4096, layers=1,
                                                 rope_factors=synth.VOXCPM2_SHORT_FACTORS),
@@ -265,7 +269,8 @@ PROMPTS = {"gqa-hd64": STACKS["gqa-hd64"], "no-rope-hd128": STACKS["no-rope-hd12
 @pytest.mark.parametrize("bf16_weights", [False, True])
 @pytest.mark.parametrize("name,rows", [("gqa-hd64", 129), ("gqa-hd64", 170),
                                        ("no-rope-hd128", 150), ("voxcpm2-encoder", 310),
-                                       ("voxcpm2-lm", 400)])
+                                       ("voxcpm2-encoder", 390), ("voxcpm2-lm", 400),
+                                       ("voxcpm2-lm", 500), ("voxcpm2-lm", 650)])
 def test_stack_prompt_rows(vx, oracle, cuda, stream, name, rows, bf16_weights):
     """A prompt past the exact rows: the norms, the rotary embedding and the
     caches, SwiGLU and the residual adds in the products' epilogues, then a
@@ -393,10 +398,11 @@ def test_stack_decode_replays_past_4096(vx, oracle, cuda, stream):
 @pytest.mark.parametrize("rows,past", [(150, 40), (129, 700)])
 def test_tile_attention_past_float16(vx, cuda, stream, heads, kv_heads, head_dim, rows, past):
     """What the matrix-core attention's float16 pairs cannot hold: rows before
-    a key are untouched by whatever it holds (a NaN value, an infinite one, a
-    NaN key: the same bits as without it), the rows that count it get float32's result; and
-    operands past 65504 give what their scaled copies give (powers of two:
-    exact, the bound one bf16 ulp of the sum)."""
+    a key keep their result whatever it holds (a NaN value, an infinite one, a
+    NaN key; a workgroup that holds rows on both sides of it starts over in
+    float32, so to one bf16 ulp of the sum), the rows that count it get float32's
+    result; and operands past 65504 give what their scaled copies give (powers of
+    two: exact, the bound one bf16 ulp of the sum)."""
     rng = synth.Rng(53, rows + past)
     keys = past + rows
     q = f32(1.5 * rng.normal(rows * heads * head_dim).reshape(rows, heads, head_dim))
