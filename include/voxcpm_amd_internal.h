@@ -156,6 +156,17 @@ int vx_stack_set_path(vx_stack* stack, int path);
 /* The path a call of `rows` rows takes now, or -1 for a null handle. */
 int vx_stack_path(const vx_stack* stack, size_t rows);
 
+/* The AudioVAE decoder's paths: the few-row float32 kernels, and the kernels for
+ * chunks of many rows (at least 9 frames, channels in multiples of 32, and 54
+ * rows of every block's output; other chunks take the few-row kernels whatever
+ * is selected). AUTO, the default, takes the faster one. */
+#define VX_VAE_PATH_AUTO 0
+#define VX_VAE_PATH_FEW_ROWS 1
+#define VX_VAE_PATH_WIDE 2
+int vx_vae_set_path(vx_vae* vae, int path);
+/* The path a chunk of `frames` frames takes now, or -1 for a null handle. */
+int vx_vae_path(const vx_vae* vae, size_t frames);
+
 /* The stack's attention on one layer's cache (the arguments of
  * vx_attention, kernels/generator_kernels.hpp), on the faster of two kernels:
  * the keys of each (row, KV head) in chunks of 64 scored by separate

@@ -141,12 +141,32 @@ def test_vae_decode_argument_checks(vx, cuda):
     torch.cuda.synchronize()
 
 
-# Chunks of 9 frames and more take the wide path (float32 products as float16
-# pairs, units of 32 and 64 channels in one launch): "wide" has a product
-# per kind of block (128 channels by depthwise launch and product, 64 and 32
-# fused), row counts that fill no tile at every dilation, and shorter
-# chunks between wide ones, whose histories the two paths share.
+# The wide path (float32 products as float16 pairs, units of 32 and 64 channels
+# in one launch) takes chunks of 9 frames and more where it is the faster one,
+# and here wherever it can: WIDE has a product per kind of block (128 channels
+# by depthwise launch and product, 64 and 32 fused), row counts that fill no tile
+# at every dilation, and shorter chunks between wide ones, whose histories
+# the two paths share.
 WIDE = synth.VaeConfig(latent=16, decoder_dim=256, rates=(8, 3, 2))
+
+
+def wide_vae(vx, weights, frames):
+    vae = vx.Vae(weights)
+    vae.set_path(_lib.VAE_PATH_WIDE)
+    assert vae.path(frames) == _lib.VAE_PATH_WIDE
+    return vae
+
+
+def test_vae_takes_the_faster_path(vx, cuda):
+    """Sizes on which the two paths' measured times leave no doubt."""
+    vae = vx.Vae(synth.vae_weights(WIDE, 100))
+    assert vae.path(20) == _lib.VAE_PATH_FEW_ROWS and vae.path(96) == _lib.VAE_PATH_FEW_ROWS
+    assert vae.path(500) == _lib.VAE_PATH_WIDE
+    vae = vx.Vae(synth.vae_weights(CONFIGS["voxcpm2"], 100))
+    assert vae.path(8) == _lib.VAE_PATH_FEW_ROWS
+    assert all(vae.path(frames) == _lib.VAE_PATH_WIDE for frames in range(9, 127))
+    vae.set_path(_lib.VAE_PATH_FEW_ROWS)
+    assert vae.path(125) == _lib.VAE_PATH_FEW_ROWS
 
 
 @pytest.mark.parametrize("chunks", [(20, 4, 31), (9, 9), (3, 50, 1, 10)])
@@ -156,7 +176,7 @@ def test_vae_wide_chunks_against_oracle(vx, oracle, cuda, stream, chunks):
     latents = synth.Rng(102, frames).normal(frames * WIDE.latent).astype(np.float32)
     latents = latents.reshape(frames, WIDE.latent)
     ref = oracle.OracleVae(weights).decode(latents)
-    vae = vx.Vae(weights)
+    vae = wide_vae(vx, weights, max(chunks))
     device_latents = torch.from_numpy(latents).to(cuda)
     for attempt in range(3):  # the same buffers again: eager, captured, replayed
         pieces, at = [], 0
@@ -180,7 +200,7 @@ def test_vae_wide_past_float16(vx, oracle, cuda):
     latents = synth.Rng(104, frames).normal(frames * WIDE.latent).astype(np.float32)
     latents = latents.reshape(frames, WIDE.latent)
     ref = oracle.OracleVae(weights).decode(latents)
-    got = vx.Vae(weights).decode(torch.from_numpy(latents).to(cuda)).cpu().numpy()
+    got = wide_vae(vx, weights, frames).decode(torch.from_numpy(latents).to(cuda)).cpu().numpy()
     error = float(np.max(np.abs(got - ref)))
     print(f"past float16: max |d| {error:.2e}, signal std {np.std(ref):.3f}", flush=True)
     assert np.std(ref) > 0.1
@@ -232,7 +252,7 @@ def test_vae_wide_below_float16(vx, oracle, cuda, scale):
     latents = synth.Rng(108, frames).normal(frames * WIDE.latent).astype(np.float32)
     latents = latents.reshape(frames, WIDE.latent)
     ref = oracle.OracleVae(weights).decode(latents)
-    got = vx.Vae(weights).decode(torch.from_numpy(latents).to(cuda)).cpu().numpy()
+    got = wide_vae(vx, weights, frames).decode(torch.from_numpy(latents).to(cuda)).cpu().numpy()
     error = float(np.max(np.abs(got - ref)))
     print(f"blocks scaled by {scale:.1e}: max |d| {error:.2e}, signal std {np.std(ref):.3f}",
           flush=True)

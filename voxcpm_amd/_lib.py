@@ -95,6 +95,9 @@ STACK_PATH_AUTO = 0
 STACK_PATH_FUSED = 2
 STACK_PATH_UNFUSED = 3
 STACK_PATH_ROWS = 4
+VAE_PATH_AUTO = 0
+VAE_PATH_FEW_ROWS = 1
+VAE_PATH_WIDE = 2
 
 
 class StackShape(ctypes.Structure):
@@ -182,6 +185,8 @@ _SIGNATURES = {
                           c_void_p], c_int),
     "vx_stack_set_path": ([c_void_p, c_int], c_int),
     "vx_stack_path": ([c_void_p, c_size], c_int),
+    "vx_vae_set_path": ([c_void_p, c_int], c_int),
+    "vx_vae_path": ([c_void_p, c_size], c_int),
     "vx_split_attention": ([c_void_p] * 4 + [c_size] * 4 + [c_int] + [c_size] * 4
                            + [c_void_p, c_size, c_void_p], c_int),
     "vx_tile_attention": ([c_void_p] * 4 + [c_size] * 4 + [c_int] + [c_size] * 4

@@ -20,8 +20,8 @@
 // products (the reference calls hipblasSgemm) take float32 MFMA kernels:
 // 16-column, 32-row tiles that read the weights in place, or, where those
 // tiles would re-read over 32 MiB of activations between them, 32 x 32
-// tiles staged through LDS. From 9 frames a chunk takes the wide path
-// (LaunchBlocksWide, vae_wide.hip). Up to 16 latent frames per chunk the
+// tiles staged through LDS. Chunks of many rows take the wide path
+// (LaunchBlocksWide, vae_wide.hip) where it is the faster one. Up to 16 latent frames per chunk the
 // launches replay as one HIP graph.
 #include <hip/hip_runtime.h>
 
@@ -35,6 +35,7 @@
 #include "snake.hpp"
 #include "vae_wide.hpp"
 #include "voxcpm_amd.h"
+#include "voxcpm_amd_internal.h"
 
 namespace {
 
@@ -46,9 +47,8 @@ constexpr int kThreads = 256;
 constexpr int kTaps = 7;
 constexpr int kDilations[3] = {1, 3, 9};
 constexpr std::size_t kMaxGraphFrames = 16;
-// Fewest frames of the wide path (measured on MI355X at VoxCPM2's shape: a
-// chunk of 8 frames 309 us on the few-row kernels, 335 us on the wide path;
-// 9 frames 354 and 338 us, 16 frames 435 and 357 us).
+// Fewest frames of the wide path (a chunk of 8 frames at VoxCPM2's shape 309 us
+// on the few-row kernels on MI355X, 335 us on the wide path).
 constexpr std::size_t kWideFrames = 9;
 // Output samples per decode call: a product's row blocks of 32 rows are
 // grid rows, at most 65535 of them.
@@ -988,6 +988,7 @@ struct vx_vae {
   float* partials = nullptr;  // [kMaxSplits][t][n] of split products
   std::size_t capacity_frames = 0;
   GraphKey graph_key;
+  int path = VX_VAE_PATH_AUTO;
   hipGraphExec_t graph = nullptr;
   bool seen = false;  // the key has run once eagerly before its capture
 
@@ -1178,11 +1179,11 @@ struct vx_vae {
     return VX_OK;
   }
 
-  /// Whether a chunk takes the wide path (LaunchBlocksWide): kWideFrames
+  /// Whether the wide path (LaunchBlocksWide) can take a chunk: kWideFrames
   /// frames, channels whole reduction steps of 32, every unit's chunk at
   /// least its history (54 rows), and operands within the kernels' 31-bit
   /// offsets.
-  bool Wide(std::size_t frames) const {
+  bool WideTakes(std::size_t frames) const {
     if (frames < kWideFrames || out_channels % 32 != 0)
       return false;
     constexpr std::size_t kMost = std::size_t{1} << 31;
@@ -1196,6 +1197,38 @@ struct vx_vae {
       t = up;
     }
     return true;
+  }
+
+  /// Whether a chunk takes it: both paths' times in microseconds, fitted on
+  /// MI355X to 226 chunks of 19 decoder shapes (one to six blocks of 64 to 2048
+  /// channels, 9 to 500 frames): a part per launch and per column of the
+  /// transposed convolutions' reductions, the multiply-adds and the streams'
+  /// bytes. Within a tenth the wide path is taken, the more exact one (error
+  /// against 64 bits at VoxCPM2's shape 1.7e-5, 4.7e-5 on the few-row kernels):
+  /// VoxCPM2 from 9 frames on (354 us there, 338 here; 16 frames 435 and 357); 256
+  /// channels and rates 8, 3, 2 from 300 frames (48 frames 70 and 109, 300 frames 129
+  /// and 119). The choice is on average 0.5 % slower than the faster path.
+  bool Wide(std::size_t frames) const {
+    if (path == VX_VAE_PATH_FEW_ROWS || !WideTakes(frames))
+      return false;
+    if (path == VX_VAE_PATH_WIDE)
+      return true;
+    double there = 8.8;
+    double here = 4.7;
+    double t = static_cast<double>(frames);
+    for (const Block& b : blocks) {
+      const double in = static_cast<double>(b.in);
+      const double out = static_cast<double>(b.out);
+      const double up = t * static_cast<double>(b.stride) * out * 2.0 * in;
+      t *= static_cast<double>(b.stride);
+      const double units = 3.0 * t * out * out;
+      const double bytes = 32.0 * t * out;
+      const bool fused = vx::vae::UnitSupported(b.out);
+      there += 0.0192 * in + 17.7e-9 * up + 1.17e-6 * bytes +
+               (fused ? 3 * 5.1 : 3 * 5.5 + 10.6e-9 * units);
+      here += 0.0228 * in + 0.37e-6 * bytes + (fused ? 3 * 8.8 : 3 * 12.7 + 15.0e-9 * units);
+    }
+    return 0.9 * here < there;
   }
 
   /// The decoder blocks over many rows (vae_wide.hip), from block 0's input
@@ -1525,6 +1558,23 @@ int vx_vae_reset(vx_vae* vae, void* stream) {
   if (hipGetLastError() != hipSuccess)
     return vx::Fail(VX_HIP_ERROR, "vx_vae_reset: launch");
   return vx::Succeed();
+}
+
+int vx_vae_set_path(vx_vae* vae, int path) {
+  if (vae == nullptr)
+    return vx::Fail(VX_BAD_ARG, "vx_vae_set_path: null handle");
+  if (path != VX_VAE_PATH_AUTO && path != VX_VAE_PATH_FEW_ROWS && path != VX_VAE_PATH_WIDE)
+    return vx::Fail(VX_BAD_ARG, "vx_vae_set_path: unknown path");
+  if (vae->graph != nullptr)
+    (void)hipGraphExecDestroy(vae->graph);
+  vae->graph = nullptr;
+  vae->seen = false;
+  vae->path = path;
+  return VX_OK;
+}
+
+int vx_vae_path(const vx_vae* vae, size_t frames) {
+  return vae == nullptr ? -1 : vae->Wide(frames) ? VX_VAE_PATH_WIDE : VX_VAE_PATH_FEW_ROWS;
 }
 
 size_t vx_vae_hop(const vx_vae* vae) { return vae == nullptr ? 0 : vae->hop; }

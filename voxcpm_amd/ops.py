@@ -589,6 +589,13 @@ class Vae:
     def __del__(self):
         self.close()
 
+    def set_path(self, path: int) -> None:
+        """Selects the path (voxcpm_amd._lib.VAE_PATH_*)."""
+        check(lib().vx_vae_set_path(self.handle, path))
+
+    def path(self, frames: int) -> int:
+        return lib().vx_vae_path(self.handle, frames)
+
     def reset(self, stream=None) -> None:
         check(lib().vx_vae_reset(self.handle, _stream(stream)))
 
