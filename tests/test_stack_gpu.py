@@ -256,10 +256,9 @@ def test_stack_bf16_weights(vx, oracle, cuda, stream):
 
 # The products' tiles. gate_up: the base LM's 96 x 256 at 400 rows, 128 x 256 at
 # 500, 160 x 256 at 650, the encoder's 128 x 128 in two groups of k. qkv: the
-# encoder's 64 x 64 in eight groups at 310 rows, 128 x 128 in two at 390, the base
+# encoder's 64 x 64 in eight groups at 310 rows, 128 x 128 in two at 800, the base
 # LM's 64 x 128 in four. o and down: 32 x 64 (encoder) and 64 x 64 (base LM) in
-# eight groups, 64 x 128 in four at 650. The small layers: 128 x 128 in two groups,
-# and 32 x 64 for down.
+# eight groups, 64 x 128 in four at 650. The small layers: 32 x 64.
 PROMPTS = {"gqa-hd64": STACKS["gqa-hd64"], "no-rope-hd128": STACKS["no-rope-hd128"],
            "voxcpm2-encoder": synth.StackConfig(hidden=1024, ffn=4096, layers=1,
                                                 rope_factors=synth.VOXCPM2_SHORT_FACTORS),
@@ -269,7 +268,7 @@ PROMPTS = {"gqa-hd64": STACKS["gqa-hd64"], "no-rope-hd128": STACKS["no-rope-hd12
 @pytest.mark.parametrize("bf16_weights", [False, True])
 @pytest.mark.parametrize("name,rows", [("gqa-hd64", 129), ("gqa-hd64", 170),
                                        ("no-rope-hd128", 150), ("voxcpm2-encoder", 310),
-                                       ("voxcpm2-encoder", 390), ("voxcpm2-lm", 400),
+                                       ("voxcpm2-encoder", 800), ("voxcpm2-lm", 400),
                                        ("voxcpm2-lm", 500), ("voxcpm2-lm", 650)])
 def test_stack_prompt_rows(vx, oracle, cuda, stream, name, rows, bf16_weights):
     """A prompt past the exact rows: the norms, the rotary embedding and the

@@ -650,24 +650,33 @@ using ExactTile = Tile<32, 1, 1, 16, 2>;
 
 namespace {
 
-/// A shape and its model: a workgroup's time apart from its steps and per
-/// step (64 columns of k) in microseconds, one workgroup per compute unit
-/// (measured on MI355X over m 129..777, k 1024..6144, n 1024..12288; within
-/// a fifth of every time measured there but for grids that fill every
-/// compute unit, which take up to a third longer, all shapes alike).
+/// A shape and its model in microseconds, one workgroup per compute unit: each
+/// round of workgroups takes `fixed` and `step` per step (64 columns of k of a
+/// group), and a full grid's tiles share another `share` per step (memory and
+/// L2). Fitted on MI355X to 14700 times of both weight formats, forced to each
+/// shape (m 129..3000, k 64..6144, n 64..24576): the picked shape took on average
+/// 0.3 % longer than the best one, one time in twenty over 2 % longer, and the
+/// times lie within a sixth of the model's nine times in ten, long outputs of
+/// short reductions apart.
 struct Model {
   Shape shape;
-  double fixed, step;
+  double fixed, step, share;
 };
 constexpr Model kModels[kShapes] = {
-    {{128, 256, 1}, 3.0, 0.85}, {{128, 128, 2}, 3.0, 0.87}, {{64, 128, 4}, 6.0, 1.0},
-    {{64, 64, 8}, 5.5, 1.03},   {{32, 64, 8}, 4.0, 0.85},   {{160, 256, 1}, 3.0, 0.97},
-    {{96, 256, 1}, 3.0, 0.75}};
+    {{128, 256, 1}, 5.9, 0.58, 0.49}, {{128, 128, 2}, 5.2, 0.60, 0.53},
+    {{64, 128, 4}, 5.3, 0.86, 0.37},  {{64, 64, 8}, 5.5, 1.12, 0.26},
+    {{32, 64, 8}, 4.0, 0.84, 0.09},   {{160, 256, 1}, 6.5, 0.66, 0.61},
+    {{96, 256, 1}, 5.1, 0.53, 0.35}};
 constexpr std::size_t kComputeUnits = 256;
 
-double Rounds(std::size_t m, std::size_t n, int bm, int bn) {
-  const std::size_t tiles = ((m + bm - 1) / bm) * ((n + bn - 1) / bn);
-  return static_cast<double>((tiles + kComputeUnits - 1) / kComputeUnits);
+double Time(const Model& model, std::size_t m, std::size_t k, std::size_t n) {
+  const std::size_t groups = static_cast<std::size_t>(model.shape.groups);
+  const std::size_t tiles =
+      ((m + model.shape.bm - 1) / model.shape.bm) * ((n + model.shape.bn - 1) / model.shape.bn);
+  const double rounds = static_cast<double>((tiles + kComputeUnits - 1) / kComputeUnits);
+  const double steps = static_cast<double>((q8::Pairs(k) + groups - 1) / groups);
+  return rounds * (model.fixed + steps * model.step) +
+         static_cast<double>(tiles) / kComputeUnits * steps * model.share;
 }
 
 }  // namespace
@@ -687,13 +696,9 @@ int PickShape(std::size_t m, std::size_t k, std::size_t n, double* microseconds,
   int best = 0;
   double least = 0.0;
   for (int i = 0; i < kShapes; ++i) {
-    const Model& model = kModels[i];
-    if (kind == Out::kQkvCache && model.shape.bm == kNoQkvRows)
+    if (kind == Out::kQkvCache && kModels[i].shape.bm == kNoQkvRows)
       continue;
-    const std::size_t groups = static_cast<std::size_t>(model.shape.groups);
-    const double steps = static_cast<double>((q8::Pairs(k) + groups - 1) / groups);
-    const double time = Rounds(m, n, model.shape.bm, model.shape.bn) *
-                        (model.fixed + steps * model.step);
+    const double time = Time(kModels[i], m, k, n);
     if (i == 0 || time < least) {
       best = i;
       least = time;
@@ -717,11 +722,11 @@ bool Use(std::size_t m, std::size_t k, std::size_t n, bool q8) {
   // Else by both sides' times in microseconds, fitted on MI355X (drawn and
   // gridded sizes, both weight formats, replayed from a graph).
   double here = 0.0;
-  const int shape = PickShape(m, k, n, &here);
+  PickShape(m, k, n, &here);
   const double pairs = static_cast<double>(q8::Pairs(k));
   if (UseRowBlocks(m, k, n, q8)) {
-    // 2940 sizes, m 129..1500, k 64..6144, n 64..16384: on average 0.4 %
-    // slower than the faster kernel, and one in 130 over 4 % slower than in row
+    // 2936 sizes, m 129..1500, k 64..6144, n 64..16384: on average 0.6 %
+    // slower than the faster kernel, one in fifty over 4 % slower than in row
     // blocks. 129 x 256 x 1024 3.7 us there, 6.4 here; 256 x 1024 x 1024 4.8 and
     // 6.0; 512 x 544 x 2055 12.5 and 8.9; 448 x 1536 x 2560 16.4 and 11.5.
     const double output = static_cast<double>(m) * static_cast<double>(n) * 1e-6;  // its writing
@@ -738,21 +743,17 @@ bool Use(std::size_t m, std::size_t k, std::size_t n, bool q8) {
     const double there =
         std::max(2.7 + 0.41 * passes + rounds * (0.21 + pair * pairs) + 2.5 * output,
                  2.7 + 0.0083 * static_cast<double>(blocks) * pairs);
-    return 2.0 + 0.78 * here + 0.85 * output < there;
+    return here + 0.3 * output < there;
   }
   if (!UseGemm(m, n))  // the tiled kernel, slower wherever it was measured
     return true;
-  // 966 sizes, m 384..3000, k 64..6144, n 6144..24576: on average 0.5 % slower
-  // than the faster kernel, and one in 60 over 4 % slower than the 256-row tiles.
-  // A full grid's later rounds take longer than the first (128 x 128 tiles a
-  // fifth, the others a tenth from the third on). bf16 1024 x 2048 x 12288 56 us
-  // there, 64 here; 777 x 2048 x 12288 56 and 41.
-  const Shape tile = ShapeOf(shape);
-  const double mine = Rounds(m, n, tile.bm, tile.bn);
-  here *= tile.bn == 128 ? (mine > 1.0 ? 1.2 : 1.0) : (mine > 2.0 ? 1.1 : 1.0);
+  // 962 sizes, m 384..3000, k 64..6144, n 6144..24576: on average 0.7 % slower
+  // than the faster kernel, one in 35 over 4 % slower than the 256-row tiles. bf16
+  // 1024 x 2048 x 12288 56 us there, 64 here; 777 x 2048 x 12288 56 and 41.
   const GemmPlan plan = PlanGemm(m, k, n, 0);
-  return here <=
-         Rounds(m, n, plan.bm, plan.bn) * (3.0 + (plan.bn == 256 ? 1.5 : 0.95) * pairs);
+  const Model gemm = plan.bn == 256 ? Model{{256, 256, 1}, 10.9, 0.83, 1.08}
+                                    : Model{{256, 128, 1}, 7.1, 0.48, 0.59};
+  return here < Time(gemm, m, k, n);
 }
 
 void Scale(const float* h, const Norm& norm, std::size_t m, std::size_t width,
