@@ -427,6 +427,12 @@ void LaunchAttention(const AttentionArgs& a, int rows, hipStream_t stream) {
 
 }  // namespace
 
+/// Query heads per workgroup of the split attention of a call.
+int HeadsOf(const AttentionShape& s, int splits) {
+  return HeadsPerWorkgroup(static_cast<int>(s.heads / s.kv_heads),
+                           splits * static_cast<int>(s.rows * s.kv_heads));
+}
+
 /// Chunks per (row, KV head) for rows that attend to at most
 /// past + rows_per_sequence keys.
 int AttentionSplits(std::size_t past, std::size_t rows_per_sequence) {
@@ -475,7 +481,7 @@ void Attention(const float* q, const float* k_cache, const float* v_cache, Bf16*
   TileAttentionPlan plan;
   if (!fragment && past_device == nullptr &&
       PlanTileAttention(shape, q, k_cache, v_cache, out, partials, &plan) &&
-      UseTileAttention(shape, plan, splits)) {
+      UseTileAttention(shape, plan, splits, HeadsOf(shape, splits))) {
     TileAttention(shape, plan, q, k_cache, v_cache, out, partials, stream);
     return;
   }
@@ -1275,7 +1281,7 @@ int vx_split_attention_plan(size_t rows, size_t rows_per_sequence, size_t past, 
   vx::TileAttentionPlan plan;
   const bool tile =
       vx::PlanTileAttention(shape, nullptr, nullptr, nullptr, nullptr, nullptr, &plan) &&
-      vx::UseTileAttention(shape, plan, splits);
+      vx::UseTileAttention(shape, plan, splits, vx::stack::HeadsOf(shape, splits));
   out3[0] = tile ? 1 : 0;
   out3[1] = tile ? static_cast<int32_t>(plan.chunk) : static_cast<int32_t>(vx::stack::kChunk);
   out3[2] = tile ? static_cast<int32_t>(plan.splits) : splits;

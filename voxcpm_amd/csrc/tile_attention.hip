@@ -581,24 +581,31 @@ bool PlanTileAttention(const AttentionShape& s, const float* q, const float* k_c
   return true;
 }
 
-bool UseTileAttention(const AttentionShape& s, const TileAttentionPlan& plan, int splits) {
-  // Both kernels' times in microseconds, fitted to MI355X over rows 4..6000,
-  // keys 2..4192, groups 1..16 and head_dim 64 and 128 (592 points, replayed
-  // from a graph): a workgroup's steps of 32 keys here, the workgroups' rounds
-  // there, and a merge each. With the rule's choice none of them takes more
-  // than 4 % longer than on the split kernel, and on average 0.3 % longer than
-  // on the faster of the two. 4 rows of 16 heads over 254 keys 7.6 us there,
-  // 16.4 here; 16 over 716 16.2 and 19.5; 64 over 314 22.8 and 19.6; 128 over
-  // 828 81.7 and 23.1; 40 patches of 5 rows 13.2 and 6.9.
+bool UseTileAttention(const AttentionShape& s, const TileAttentionPlan& plan, int splits,
+                      int heads_per_workgroup) {
+  // Both kernels' times in microseconds, fitted to MI355X over rows 4..3000, keys
+  // 2..3260, groups 1..16 and head_dim 64 and 128 (2924 points, replayed from a
+  // graph): here a workgroup's steps of 32 keys in its round of two workgroups
+  // per compute unit, there the rounds of one per unit, the longer the more
+  // heads each scores, and a merge each. The choice takes on average 0.5 % longer
+  // than the faster kernel, one in eighty over 5 % longer than the split
+  // kernel. 4 rows of 16 heads over 254 keys 7.6 us there, 16.4 here; 64 rows 5.7
+  // and 11.2, 65 rows (a second chunk and round) 16.4 and 11.1; 16 rows over 716
+  // keys 16.2 and 19.5; 64 over 314 22.8 and 19.6; 128 over 828 81.7 and 23.1; 40
+  // patches of 5 rows 13.2 and 6.9.
   const bool wide = s.head_dim > 64;
   const std::size_t keys = std::min(plan.chunk, s.past + s.rows_per_sequence);
   const double steps = static_cast<double>((keys + kKeys - 1) / kKeys);
-  const double here = 4.6 + steps * (wide ? 2.85 : 1.75) + (plan.splits > 1 ? 4.7 : 0.0);
-  const double group =
-      static_cast<double>(std::max<std::size_t>(2, s.heads / s.kv_heads));  // one costs as two
-  const double there = 3.2 + (splits > 1 ? 3.0 : 0.0) +
-                       static_cast<double>(s.rows * s.kv_heads) * splits * group *
-                           (wide ? 2.4e-3 : 1.0e-3);
+  const double here =
+      4.2 + (plan.splits > 1 ? 4.4 : 0.0) +
+      static_cast<double>((plan.workgroups + kTargetWorkgroups - 1) / kTargetWorkgroups) * steps *
+          (wide ? 2.65 : 1.6);
+  const std::size_t workgroups =
+      s.rows * s.heads / heads_per_workgroup * static_cast<std::size_t>(splits);
+  const double there = 2.8 + (splits > 1 ? 3.2 : 0.0) +
+                       static_cast<double>((workgroups + 255) / 256) *
+                           (wide ? 0.68 + 0.49 * heads_per_workgroup
+                                 : 0.28 + 0.16 * heads_per_workgroup);
   return here < there;
 }
 

@@ -32,9 +32,11 @@ bool PlanTileAttention(const AttentionShape& s, const float* q, const float* k_c
                        const float* v_cache, const Bf16* out, const float* partials,
                        TileAttentionPlan* plan);
 
-/// Whether it is the faster kernel for them: not the split kernel, `splits`
-/// chunks of whose keys a workgroup each takes.
-bool UseTileAttention(const AttentionShape& s, const TileAttentionPlan& plan, int splits);
+/// Whether it is the faster kernel for them: not the split kernel, whose
+/// workgroups each take one of `splits` chunks of a row's keys and
+/// `heads_per_workgroup` of its heads.
+bool UseTileAttention(const AttentionShape& s, const TileAttentionPlan& plan, int splits,
+                      int heads_per_workgroup);
 
 /// `partials`: rows x heads x ceil(keys / 64) x (head_dim + 2) floats, or
 /// null where a row attends to at most 64 keys.
