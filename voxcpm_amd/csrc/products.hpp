@@ -58,7 +58,8 @@ int RunSkinny(const Bf16* x, const void* w, float* y, Bf16* y_bf16,
               hipStream_t stream, q8::Weights kind = q8::Weights::kQ8);
 
 /// Whether an m > 128 product runs on the skinny engine in blocks of 64
-/// rows (RunRowBlocks) rather than the tiled or the 32 x 32 MFMA kernel:
+/// rows (RunRowBlocks) rather than the tiled or the 32 x 32 MFMA kernel, where
+/// it does not run on the panel-operand kernels (q8_prefill.hpp):
 /// the smaller prefill products, where those kernels' grids are few tiles
 /// (`q8`: Q8_0 panels, else bf16 panels).
 bool UseRowBlocks(std::size_t m, std::size_t k, std::size_t n, bool q8);

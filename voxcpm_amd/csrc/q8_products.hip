@@ -715,8 +715,9 @@ int RunSkinny(const Bf16* x, const void* w, float* y, Bf16* y_bf16,
 }
 
 bool UseRowBlocks(std::size_t m, std::size_t k, std::size_t n, bool q8) {
-  // Measured on MI355X against the tiled kernel (with its k split) and the
-  // 32 x 32 MFMA kernel, Q8_0 and bf16 panels alike: faster up to about
+  // Where they beat the kernels with both operands in LDS; the panel-operand
+  // kernels are compared with them first (prefill::Use). Measured on MI355X
+  // against the tiled kernel (with its k split) and the 32 x 32 MFMA kernel, Q8_0 and bf16 panels alike: faster up to about
   // 1.2 G multiply-adds (129 x 2048 x 2048 15.6 -> 9.2 us, 256 x 1024 x 4096
   // 14.3 -> 10.9 us), and on 2048 x 2048 weights up to 512 rows (512 rows
   // 21.0 -> 17.3 us); slower beyond (1024 x 2048 x 2048 24.7 -> 32.9 us),

@@ -12,9 +12,9 @@
 // softmax statistics in chunk order. More rows take the reference's launch
 // sequence; past 128 rows the norms, the rotary embedding and the caches,
 // SwiGLU and the residual adds go into the epilogues of q8_prefill.hip's
-// products (LaunchPrompt: 310 rows through the 12-layer encoder 727 -> 655 us
-// on MI355X, 617 through two base-LM layers 291 -> 281 us, against a launch for
-// each norm and the rotary embedding).
+// products (LaunchPrompt: 310 rows through the 12-layer encoder 700-725 us on
+// MI355X, 617 through two base-LM layers 284-310 us on several cards; a launch for
+// each norm and the rotary embedding took 72 and 10 us more).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

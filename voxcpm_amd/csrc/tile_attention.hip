@@ -27,10 +27,11 @@
 //
 // Measured on MI355X: 300 rows of 16 heads over 1800 keys 390 us on the
 // float32 split kernel, 55 us from three bfloat16 terms (twice the products,
-// and 570 workgroups in two rounds), 38 us now, of which the merge 6.8 us. A
+// and 570 workgroups in two rounds), 34.5 us now, of which the merge 7 us. A
 // step of one workgroup alone takes 2.1 us, of which the products are 0.65:
 // one wave per SIMD runs scores, softmax and values one after the other, and
-// registers (256 of 256) leave two workgroups per compute unit.
+// registers (230 of 256) leave two workgroups per compute unit. Over the launch
+// the matrix cores are busy for 22 % of the time, the vector unit for 47 %.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

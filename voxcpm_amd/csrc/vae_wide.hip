@@ -1,7 +1,7 @@
 // The AudioVAE decoder over many rows (vae.cpp:415-502 of the reference):
 // its products on gfx950's f16 matrix cores with float32 operands split into
 // two float16 terms (f16x2.hpp: three products of a sixteenth of the float32
-// instructions' time each), and a residual unit as one launch up to 256
+// instructions' time each), and a residual unit as one launch at 32 and 64
 // channels.
 //
 // ProductKernel computes BM x BN tiles of y = A W^T with four waves, k in
@@ -31,11 +31,12 @@
 // transposed convolutions 112 / 132 / 176 / 110 / 72 / 52 -> 51 / 57 / 62 /
 // 36 / 25 / 30 us; units of 1024 / 512 / 256 / 128 channels 36 / 60 / 106 /
 // 83 -> 26 / 34 / 43 / 40 us, of 64 and 32 (fused) 87 / 82 -> 28 / 23 us; the
-// decode 2090 -> 855 us, its error against 64 bits 4.6e-5 -> 1.7e-5. The
-// 128 x 128 products keep the matrix cores busy for 45 % of their time and
-// the vector unit, which splits the operands, for 40 %; the fused units
-// wait on memory (61 MB in 23 us). Units of 128 channels measured the same
-// fused as in two launches, of 256 slower.
+// decode 2090 -> 820-875 us on several cards, its error against 64 bits 4.6e-5 ->
+// 1.7e-5. The 128 x 128 products keep the matrix cores busy for 14 % (units of
+// 128 channels) to 45 % (block 1's transposed convolution) of their time and the
+// vector unit, which splits the operands, for 33 to 48 %; the fused units wait
+// on memory (61 MB in 23 us; vector unit 45 to 62 %). Units of 128 channels measured
+// the same fused as in two launches, of 256 slower.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -66,7 +67,7 @@ constexpr int kDies = 8;
 // and activations of spread 0.05 hold such a group once in 10^13.)
 constexpr float kLeast = 0x1p-15F;
 
-/// 16-byte chunk `chunk` (8 bf16 values) of row `row` of a plane of 64-byte
+/// 16-byte chunk `chunk` (8 values of 16 bits) of row `row` of a plane of 64-byte
 /// rows: the equal chunks of 16 consecutive rows (a 16-lane group of a
 /// 16-byte read) fall on distinct banks.
 __device__ inline int PlaneIndex(int row, int chunk) {

@@ -1,6 +1,7 @@
 // The AudioVAE decoder's products over many rows (a whole utterance) on the
-// bf16 matrix cores with float32 operands split into three bf16 terms
-// (bf16x3.hpp), and its residual units as one launch each (vae_wide.hip).
+// f16 matrix cores with float32 operands as two float16 terms (f16x2.hpp;
+// operands outside their range as three bfloat16 ones, bf16x3.hpp), and its
+// residual units of 32 and 64 channels as one launch each (vae_wide.hip).
 #ifndef VOXCPM_AMD_VAE_WIDE_HPP_
 #define VOXCPM_AMD_VAE_WIDE_HPP_
 
