@@ -1200,7 +1200,7 @@ struct vx_vae {
   }
 
   /// Whether a chunk takes it: both paths' times in microseconds, fitted on
-  /// MI355X to 226 chunks of 19 decoder shapes (one to six blocks of 64 to 2048
+  /// MI355X to 230 chunks of 19 decoder shapes (one to six blocks of 64 to 2048
   /// channels, 9 to 500 frames): a part per launch and per column of the
   /// transposed convolutions' reductions, the multiply-adds and the streams'
   /// bytes. Within a tenth the wide path is taken, the more exact one (error
