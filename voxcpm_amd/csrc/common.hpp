@@ -145,22 +145,6 @@ __device__ inline void BroadcastRows01(float x, float& row0, float& row1) {
   row1 = __uint_as_float(odd[0]);
 }
 
-/// The chip's compute dies: workgroup b of a launch runs on die b % kDies, and
-/// each die has an L2 of its own.
-constexpr int kDies = 8;
-
-/// Logical tile of workgroup `b` of `blocks`: die d takes a contiguous range of
-/// logical tiles (the first blocks % kDies dies one more), so that its L2 serves
-/// what neighbouring tiles share. A bijection on 0..blocks-1.
-__device__ inline int DieOrdered(int b, int blocks) {
-  const int per = blocks / kDies;
-  const int extra = blocks % kDies;
-  const int die = b % kDies;
-  const int index = b / kDies;
-  return die < extra ? die * (per + 1) + index
-                     : extra * (per + 1) + (die - extra) * per + index;
-}
-
 /// Sum over a block of up to 1024 threads; `scratch` holds one float per
 /// wave. Every thread receives the total, added in wave order.
 __device__ inline float BlockSum(float value, float* scratch) {

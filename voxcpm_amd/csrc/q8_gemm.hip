@@ -37,6 +37,8 @@ using q8::kUnitBytes;
 using q8::kValueBytes;
 using q8::PackBf16x2;
 
+constexpr int kDies = 8;
+
 typedef float F32x16 __attribute__((ext_vector_type(16)));
 
 /// C (32 x 32, float32) += A (32 x 16, bf16) B (16 x 32, bf16): lane L holds
@@ -62,6 +64,18 @@ struct GemmArgs {
   int splits, pairs_per_split;
   float* partials;
 };
+
+/// Logical tile of workgroup `b` of `blocks`: workgroup b runs on die b % 8;
+/// die d takes a contiguous range of logical tiles (the first blocks % 8
+/// dies one more). A bijection on 0..blocks-1.
+__device__ inline int DieOrdered(int b, int blocks) {
+  const int per = blocks / kDies;
+  const int extra = blocks % kDies;
+  const int die = b % kDies;
+  const int index = b / kDies;
+  return die < extra ? die * (per + 1) + index
+                     : extra * (per + 1) + (die - extra) * per + index;
+}
 
 /// LDS index of 16-byte chunk `chunk` (0..7) of row `row` of a 128-byte-row
 /// operand tile: chunk ^ ((row / 2) % 8). Rows alternate between the two

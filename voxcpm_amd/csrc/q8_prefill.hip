@@ -51,6 +51,8 @@ namespace {
 using bf16x3::F32x16;
 using q8::AsBf16x8;
 
+constexpr int kDies = 8;
+
 struct Args {
   const Bf16* x;
   const std::uint8_t* w;
@@ -64,6 +66,15 @@ struct Args {
   Norm norm;
   Qkv qkv;
 };
+
+/// Workgroup b runs on die b % 8: die d takes a contiguous range of tiles (a
+/// weight tile's row tiles first), so that its L2 serves their weights.
+__device__ inline int DieOrdered(int b, int blocks) {
+  const int per = blocks / kDies;
+  const int extra = blocks % kDies;
+  const int die = b % kDies;
+  return die * per + min(die, extra) + b / kDies;
+}
 
 /// LDS index of 16-byte chunk `chunk` (0..7) of 128-byte row `row`: the rows
 /// alternate between the halves of a 256-byte bank line, so the chunk swaps

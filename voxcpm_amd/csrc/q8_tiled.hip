@@ -44,6 +44,7 @@ constexpr int kTileN = 128;
 // LDS rows: 64 bf16 plus 8 of padding (144 bytes, 9 chunks of 16 bytes), so
 // that the fragment reads of 16 consecutive rows fall on distinct banks.
 constexpr int kRowChunks = 9;
+constexpr int kDies = 8;
 
 struct TiledArgs {
   const Bf16* x;
@@ -60,6 +61,18 @@ struct TiledArgs {
   int splits, pairs_per_split;
   float* partials;
 };
+
+/// Logical tile of workgroup `b` of `blocks`: workgroup b runs on die b % 8;
+/// die d takes a contiguous range of logical tiles (the first blocks % 8
+/// dies one more). A bijection on 0..blocks-1.
+__device__ inline int DieOrdered(int b, int blocks) {
+  const int per = blocks / kDies;
+  const int extra = blocks % kDies;
+  const int die = b % kDies;
+  const int index = b / kDies;
+  return die < extra ? die * (per + 1) + index
+                     : extra * (per + 1) + (die - extra) * per + index;
+}
 
 /// A tile shape: BM activation rows, WM waves along them (x 2 along the 128
 /// weight rows, each wave BM / WM x 64), D register sets of prefetched

@@ -60,6 +60,7 @@ using f16x2::Octet;
 constexpr int kThreads = 256;
 constexpr int kTaps = 7;
 constexpr int kStep = 32;  // reduction columns per step
+constexpr int kDies = 8;
 // Eight neighbouring operands of a row (four, of a unit's activations) are to
 // hold a magnitude of at least this, or zeros alone: the pairs' absolute error
 // of 2^-36 is then at most 2^-21 of their largest. (Weights of spread 0.001
@@ -172,6 +173,15 @@ struct ProductArgs {
   int n_tiles;
   int columns_first;  // consecutive tiles of a die share weights (else rows)
 };
+
+/// Workgroup b runs on die b % 8: die d takes a contiguous range of tiles,
+/// so that neighbouring tiles share its L2.
+__device__ inline int DieOrdered(int b, int blocks) {
+  const int per = blocks / kDies;
+  const int extra = blocks % kDies;
+  const int die = b % kDies;
+  return die * per + min(die, extra) + b / kDies;
+}
 
 /// The six kept products of two bfloat16 triples (bf16x3.hpp), from two
 /// planes at a time: pass 0 holds h and m, pass 1 h and l.
